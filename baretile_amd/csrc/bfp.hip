@@ -7,7 +7,7 @@
 //          below it, rounding half up (bfp8) or to nearest with ties up (bfp4), saturating at 127 / 7. A zero keeps no
 //          sign.
 //   decode tensor.py:1093-1104 (_bf16s): normalize the magnitude, exponent (e - shift) mod 256.
-#include "common.h"
+#include "program.h"
 
 namespace bt {
 
@@ -29,8 +29,7 @@ __device__ __forceinline__ void store_run(const uint32_t (&bits)[16], uint32_t t
   }
 }
 
-// One thread a run: 16 values of one row sharing an exponent. Runs are numbered along rows, so neighbouring threads
-// read neighbouring 32-byte pieces of a bf16 row.
+// One thread a run: 16 values of one row sharing an exponent, at any column stride (a transposed view).
 template <int FMT>
 __global__ void __launch_bounds__(256) pack_kernel(const void *src, int src_dtype, int64_t batch, int64_t rows,
                                                    int64_t cols, int64_t sb, int64_t sr, int64_t sc, uint8_t *exps,
@@ -53,6 +52,62 @@ __global__ void __launch_bounds__(256) pack_kernel(const void *src, int src_dtyp
     top = max(top, (v >> 7) & 255u);
   }
   store_run<FMT>(bits, top, exps + t, vals + t * (FMT == BT_BFP8 ? 16 : 8));
+}
+
+// The same for contiguous columns: two neighbouring threads a run, 8 values each, so that every load of a wave is one
+// contiguous stretch (a thread a run reads 32 bytes apart, value by value). The bound is HBM: 2 bytes read and 1 1/16
+// (bfp8) or 9/16 (bfp4) written a value. Loads of A bytes, the widest that every row's start is aligned to; a piece
+// that crosses the row's end goes value by value. 4096 x 14336 bf16 to bfp4 (154 MB): 107 us with a thread a
+// run, 41 us so (3.7 TB/s).
+template <int FMT, int SRC, int A>
+__global__ void __launch_bounds__(256) pack_half_kernel(const void *src, uint32_t halves, FastDiv runs, FastDiv rows,
+                                                        int64_t cols, int64_t sb, int64_t sr, uint8_t *exps,
+                                                        uint8_t *vals) {
+  constexpr int SIZE = SRC == BT_BF16 ? 2 : 4, W = SIZE * 2;  // words of 4 bytes a piece
+  typedef uint32_t words __attribute__((ext_vector_type(W)));
+  const uint32_t t = blockIdx.x * 256u + threadIdx.x, u = min(t, halves - 1u);  // every lane stays, for the exchange
+  const uint32_t run = u >> 1, br = fdiv(run, runs), b = fdiv(br, rows);
+  const int64_t c0 = (int64_t)(run - br * runs.d) * 16 + 8 * (u & 1u);
+  const uint8_t *p = (const uint8_t *)src + ((int64_t)b * sb + (int64_t)(br - b * rows.d) * sr + c0) * SIZE;
+  uint32_t bits[8];
+  if (c0 + 8 <= cols) {
+    words w;
+    if constexpr (A >= 4) {
+      typedef uint32_t piece __attribute__((ext_vector_type(A / 4)));
+#pragma unroll
+      for (int i = 0; i < 4 * W / A; i++) {
+        const piece x = ((const piece *)p)[i];
+#pragma unroll
+        for (int k = 0; k < A / 4; k++) w[i * (A / 4) + k] = x[k];
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < W; i++) w[i] = ((const uint16_t *)p)[2 * i] | (uint32_t)((const uint16_t *)p)[2 * i + 1] << 16;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++)
+      bits[i] = SRC == BT_BF16 ? w[i / 2 % W] >> (16 * (i & 1)) & 0xFFFFu : bf16_rne(__uint_as_float(w[i % W]));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      bits[i] = 0;
+      if (c0 + i < cols) bits[i] = SRC == BT_BF16 ? ((const uint16_t *)p)[i] : bf16_rne(((const float *)p)[i]);
+    }
+  }
+  uint32_t top = 0;
+#pragma unroll
+  for (int i = 0; i < 8; i++) top = max(top, bits[i] >> 7 & 255u);
+  top = max(top, (uint32_t)__builtin_amdgcn_update_dpp((int)top, (int)top, 0xB1, 0xF, 0xF, false));  // the run's other half
+  if (t >= halves) return;
+  uint32_t w[2] = {0, 0};
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    if (FMT == BT_BFP8) w[i / 4] |= ((uint32_t)bfp_signed<8>(bits[i], top) & 255u) << (8 * (i % 4));
+    else w[0] |= ((uint32_t)bfp_signed<4>(bits[i], top) & 15u) << (4 * i);
+  }
+  if (FMT == BT_BFP8) *(uint2 *)(vals + (int64_t)t * 8) = make_uint2(w[0], w[1]);
+  else *(uint32_t *)(vals + (int64_t)t * 4) = w[0];
+  if (!(t & 1u)) exps[t >> 1] = (uint8_t)top;
 }
 
 // One row of x (bf16) put into a plain block-float tensor at each place (Tensor.put into a block-float cache,
@@ -157,34 +212,62 @@ __device__ __forceinline__ int nibble_q(uint32_t w, int j) {  // the inverse: va
   return sgn ? -(int)mag : (int)mag;
 }
 
-// One block a columns tile, one thread a lane. Reads the plain planes, writes the tile.
-template <int FMT>
-__global__ void __launch_bounds__(64) columns_kernel(const uint8_t *exps, const uint8_t *vals, int64_t rows,
-                                                     int64_t cols, int64_t chunks, int64_t nruns, uint8_t *dst) {
-  constexpr int TB = FMT == BT_BFP8 ? 1088 : 576;
-  int64_t tile = blockIdx.x;  // (b * nruns + run) * chunks + chunk
-  int64_t chunk = tile % chunks, run = tile / chunks % nruns, b = tile / chunks / nruns;
-  int l = threadIdx.x;
-  int64_t runs = (cols + 15) / 16, cols16 = runs * 16;
-  uint8_t *out = dst + tile * TB;
-  {  // exponent byte l
-    int64_t k = chunk * 64 + tile_row_of_exp(l);
-    uint32_t e = k < rows ? exps[(b * rows + k) * runs + run] : 0;
-    out[l] = (uint8_t)((e - exp_bias<FMT>()) & 255u);
-  }
-  int64_t n = run * 16 + (l & 15);
-  uint32_t w[4] = {0, 0, 0, 0};
+// A block re-lays 16 neighbouring runs of one 64-row chunk through LDS: it reads the chunk's rows as whole stretches of
+// the planes (a run's 8 or 16 bytes a thread, 128 or 256 bytes a row), and each of its 4 waves then gathers 4 tiles from
+// LDS and writes each as one contiguous stretch. One block a tile, each lane fetching its 16 values a byte at a time from
+// 16 rows, left the loads' lines mostly unused. The bound is HBM: 9/16 (bfp4) or 17/16 (bfp8) bytes a value each way.
+// LDS rows are 8 bytes longer than their runs, so that the 4 lane groups' rows, 8 apart, start 16 banks apart. WIDE: the
+// value plane starts on 8 bytes (it is byte addressed otherwise). 4096 x 14336 in bfp4: 53 us a block a tile, 25 us so (2.9 TB/s).
+constexpr int RUNS_B = 16;  // runs a block
+template <int FMT, bool WIDE>
+__global__ void __launch_bounds__(256) columns_kernel(const uint8_t *exps, const uint8_t *vals, int64_t rows,
+                                                      uint32_t runs, uint32_t chunks, FastDiv groups, FastDiv chunks_d,
+                                                      uint8_t *dst) {
+  constexpr int TB = FMT == BT_BFP8 ? 1088 : 576, RB = FMT == BT_BFP8 ? 16 : 8, S = RUNS_B * RB + 8;
+  __shared__ __attribute__((aligned(16))) uint8_t lv[64 * S];
+  __shared__ __attribute__((aligned(16))) uint8_t le[RUNS_B][64];  // a tile's exponent bytes, as it stores them
+  const uint32_t q = fdiv(blockIdx.x, groups), b = fdiv(q, chunks_d), chunk = q - b * chunks, run0 = (blockIdx.x - q * groups.d) * RUNS_B;
+  const int t = threadIdx.x;
+  const int64_t k0 = (int64_t)chunk * 64;
 #pragma unroll
-  for (int h = 0; h < 2; h++)
+  for (int i = 0; i < 4; i++) {
+    const int row = t / RUNS_B + 16 * i, run = t % RUNS_B;
+    const bool in = k0 + row < rows && run0 + run < runs;
+    const int64_t at = ((int64_t)b * rows + k0 + row) * runs + run0 + run;  // the run's number in the planes
+    uint2 w[RB / 8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-      int64_t k = chunk * 64 + tile_row(l, h, j);
-      int q = (k < rows && n < cols16) ? plain_q<FMT>(vals, FMT == BT_BFP8 ? cols16 : cols16 / 2, b * rows + k, n) : 0;
-      if (FMT == BT_BFP8) w[(h * 8 + j) / 4] |= ((uint32_t)q & 255u) << (8 * (j % 4));
-      else w[h] |= nibble_bits(q, j);
+    for (int k = 0; k < RB / 8; k++) {
+      w[k] = make_uint2(0, 0);
+      if (!in) continue;
+      const uint8_t *p = vals + at * RB + 8 * k;
+      if (WIDE) w[k] = *(const uint2 *)p;
+      else w[k] = make_uint2(p[0] | p[1] << 8 | p[2] << 16 | (uint32_t)p[3] << 24, p[4] | p[5] << 8 | p[6] << 16 | (uint32_t)p[7] << 24);
     }
-  if (FMT == BT_BFP8) *(uint4 *)(out + 64 + 16 * l) = make_uint4(w[0], w[1], w[2], w[3]);
-  else *(uint2 *)(out + 64 + 8 * l) = make_uint2(w[0], w[1]);
+    const uint32_t e = in ? exps[at] : 0u;
+    le[run][16 * (row >> 3 & 3) + 8 * (row >> 5) + (row & 7)] = (uint8_t)(e - exp_bias<FMT>());
+#pragma unroll
+    for (int k = 0; k < RB / 8; k++) *(uint2 *)(lv + row * S + run * RB + 8 * k) = w[k];
+  }
+  __syncthreads();
+  const int l = t & 63, n = l & 15;
+#pragma unroll
+  for (int i = 0; i < RUNS_B / 4; i++) {
+    const uint32_t run = (t >> 6) + 4 * i;
+    if (run0 + run >= runs) break;  // uniform in the wave
+    uint8_t *out = dst + ((int64_t)((int64_t)b * runs + run0 + run) * chunks + chunk) * TB;
+    if (l < 16) ((uint32_t *)out)[l] = ((const uint32_t *)le[run])[l];
+    uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const uint8_t *p = lv + tile_row(l, h, j) * S + run * RB;
+        if (FMT == BT_BFP8) w[(h * 8 + j) / 4] |= (uint32_t)p[n] << (8 * (j % 4));
+        else w[h] |= nibble_bits((int32_t)((uint32_t)p[n / 2] << (28 - 4 * (n & 1))) >> 28, j);
+      }
+    if (FMT == BT_BFP8) *(uint4 *)(out + 64 + 16 * l) = make_uint4(w[0], w[1], w[2], w[3]);
+    else *(uint2 *)(out + 64 + 8 * l) = make_uint2(w[0], w[1]);
+  }
 }
 
 __global__ void __launch_bounds__(64) bf16_columns_kernel(const uint16_t *src, int64_t rows, int64_t cols, int64_t sb,
@@ -212,30 +295,69 @@ __global__ void __launch_bounds__(64) bf16_columns_kernel(const uint16_t *src, i
   out[1] = make_uint4(w[4], w[5], w[6], w[7]);
 }
 
-// One thread a value of the result: finds it in its tile, decodes it exactly.
-template <int FMT>
-__global__ void __launch_bounds__(256) columns_unpack_kernel(const uint8_t *src, int64_t batch, int64_t rows,
-                                                             int64_t cols, int64_t chunks, int64_t nruns,
-                                                             uint16_t *dst) {
-  int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= batch * rows * cols) return;
-  int64_t n = t % cols, k = t / cols % rows, b = t / cols / rows;
-  int64_t run = n / 16, chunk = k / 64;
-  int kk = (int)(k % 64), h = kk / 32, g = (kk % 32) / 8, j = kk % 8, l = g * 16 + (int)(n % 16);
-  int64_t tile = (b * nruns + run) * chunks + chunk;
-  if (FMT == BT_BF16) {
-    dst[t] = ((const uint16_t *)src)[tile * 1024 + 16 * l + 8 * h + j];
-    return;
+// Readback of 16 neighbouring runs of one chunk a block: each of its 4 waves loads 4 tiles as contiguous stretches, every
+// lane decoding its 16 values exactly, and the block stores the 64 rows' 256 columns from LDS as whole 512-byte
+// stretches (WIDE: every row of the result starts on 16 bytes; otherwise a thread a column). A thread a value took its
+// exponent and value a byte at a time from tiles that lie `chunks` apart. The bound is HBM: 2 bytes written a value and
+// 9/16 to 2 read. 4096 x 14336 in bfp4: UN107 us with a thread a
+// run, 41 us so (3.7 TB/s).
+template <int FMT, bool WIDE>
+__global__ void __launch_bounds__(256) columns_unpack_kernel(const uint8_t *src, int64_t rows, int64_t cols,
+                                                             uint32_t runs, uint32_t chunks, FastDiv groups,
+                                                             FastDiv chunks_d, uint16_t *dst) {
+  constexpr int TB = FMT == BT_BF16 ? 2048 : FMT == BT_BFP8 ? 1088 : 576, S = 16 * RUNS_B + 4;  // rows 130 dwords apart
+  __shared__ __attribute__((aligned(16))) uint16_t lds[64 * S];
+  const uint32_t q = fdiv(blockIdx.x, groups), b = fdiv(q, chunks_d), chunk = q - b * chunks, run0 = (blockIdx.x - q * groups.d) * RUNS_B;
+  const int t = threadIdx.x, l = t & 63, g = l >> 4, n = l & 15;
+#pragma unroll
+  for (int i = 0; i < RUNS_B / 4; i++) {
+    const uint32_t run = (t >> 6) + 4 * i;
+    if (run0 + run >= runs) break;  // uniform in the wave
+    const uint8_t *tp = src + ((int64_t)((int64_t)b * runs + run0 + run) * chunks + chunk) * TB;
+    uint32_t v[16];  // value 8h + j: row 32h + 8g + j of the tile, column n
+    if (FMT == BT_BF16) {
+      const uint4 w0 = ((const uint4 *)(tp + 32 * l))[0], w1 = ((const uint4 *)(tp + 32 * l))[1];
+      const uint32_t w[8] = {w0.x, w0.y, w0.z, w0.w, w1.x, w1.y, w1.z, w1.w};
+#pragma unroll
+      for (int k = 0; k < 16; k++) v[k] = w[k / 2] >> (16 * (k & 1));
+    } else {
+      const uint4 ew = *(const uint4 *)(tp + 16 * g);
+      const uint32_t es[4] = {ew.x, ew.y, ew.z, ew.w};
+      uint32_t w[4];
+      if (FMT == BT_BFP8) {
+        const uint4 x = *(const uint4 *)(tp + 64 + 16 * l);
+        w[0] = x.x, w[1] = x.y, w[2] = x.z, w[3] = x.w;
+      } else {
+        const uint2 x = *(const uint2 *)(tp + 64 + 8 * l);
+        w[0] = x.x, w[1] = x.y, w[2] = w[3] = 0;
+      }
+#pragma unroll
+      for (int k = 0; k < 16; k++) {
+        const uint32_t e = ((es[k / 4] >> (8 * (k % 4))) + exp_bias<FMT>()) & 255u;
+        const int mag = FMT == BT_BFP8 ? (int32_t)(w[k / 4] << (24 - 8 * (k % 4))) >> 24 : nibble_q(w[k / 8], k % 8) * 16;
+        // for e in 7..254 the value is a normal float whose top half is the exact bf16; mag * 2^(e - 133) in both formats
+        v[k] = e - 7u <= 247u ? __float_as_uint((float)mag * __uint_as_float((e - 6u) << 23)) >> 16 : unpacked_bits(mag, e);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 16; k++) lds[(32 * (k / 8) + 8 * g + k % 8) * S + 16 * run + n] = (uint16_t)v[k];
   }
-  constexpr int TB = FMT == BT_BFP8 ? 1088 : 576;
-  const uint8_t *tp = src + tile * TB;
-  uint32_t e = (tp[16 * g + 8 * h + j] + exp_bias<FMT>()) & 255u;
-  int q;
-  if (FMT == BT_BFP8) q = (int)(int8_t)tp[64 + 16 * l + 8 * h + j];
-  else {
-    q = nibble_q(*(const uint32_t *)(tp + 64 + 8 * l + 4 * h), j) * 16;
+  __syncthreads();
+  const int64_t k0 = (int64_t)chunk * 64, c0 = (int64_t)run0 * 16;
+  uint16_t *out = dst + ((int64_t)b * rows + k0) * cols + c0;
+  if (WIDE) {  // cols is a multiple of 8
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int row = t / 32 + 8 * i, c = t % 32 * 8;
+      const uint2 x = *(const uint2 *)(lds + row * S + c), y = *(const uint2 *)(lds + row * S + c + 4);
+      if (k0 + row < rows && c0 + c < cols) *(uint4 *)(out + row * cols + c) = make_uint4(x.x, x.y, y.x, y.y);
+    }
+  } else {
+    if (c0 + t >= cols) return;
+#pragma unroll 8
+    for (int row = 0; row < 64; row++)
+      if (k0 + row < rows) out[row * cols + t] = lds[row * S + t];
   }
-  dst[t] = (uint16_t)unpacked_bits(q, e);
 }
 
 static int check_fmt(int fmt) {
@@ -252,6 +374,29 @@ static int check_shape(int64_t batch, int64_t rows, int64_t cols) {
 
 static unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
 
+// pack_half_kernel with the widest loads (16, 8, 4 or 2 bytes) that every row's start is aligned to.
+template <int FMT>
+static void launch_pack_half(uint64_t src, int src_dtype, int64_t batch, int64_t rows, int64_t cols, int64_t sb, int64_t sr,
+                             uint64_t exps, uint64_t vals, hipStream_t s) {
+  const int64_t size = src_dtype == BT_BF16 ? 2 : 4, runs = (cols + 15) / 16;
+  const uint32_t halves = (uint32_t)(2 * batch * rows * runs);
+  uint64_t at = src | 16u;  // the starts' common alignment; strides that no second row or matrix uses don't count
+  if (rows > 1) at |= (uint64_t)(sr * size);
+  if (batch > 1) at |= (uint64_t)(sb * size);
+  const uint64_t align = at & (~at + 1);
+  const FastDiv rd = make_fastdiv((uint32_t)runs), wd = make_fastdiv((uint32_t)rows);
+#define BT_PACK(SRC, A)                                                                                              \
+  pack_half_kernel<FMT, SRC, A><<<blocks_for(halves, 256), 256, 0, s>>>((const void *)src, halves, rd, wd, cols, sb, \
+                                                                        sr, (uint8_t *)exps, (uint8_t *)vals)
+  if (src_dtype == BT_FP32) {
+    if (align >= 16) BT_PACK(BT_FP32, 16);
+    else BT_PACK(BT_FP32, 4);
+  } else if (align >= 16) BT_PACK(BT_BF16, 16);
+  else if (align >= 4) BT_PACK(BT_BF16, 4);
+  else BT_PACK(BT_BF16, 2);
+#undef BT_PACK
+}
+
 }  // namespace bt
 
 using namespace bt;
@@ -266,8 +411,11 @@ int bt_bfp_pack(bt_runtime *rt, int fmt, uint64_t src, int src_dtype, int64_t ba
   if (int s = check_shape(batch, rows, cols)) return s;
   if (src_dtype != BT_BF16 && src_dtype != BT_FP32) return fail(BT_EINVAL, "a block float is cast from bf16 or fp32");
   if (vals % 16) return fail(BT_EINVAL, "the value plane must be 16-byte aligned");
-  int64_t n = batch * rows * ((cols + 15) / 16);
-  if (fmt == BT_BFP8)
+  const int64_t runs = (cols + 15) / 16, n = batch * rows * runs;
+  if (sc == 1 && 2 * n < (1ll << 31)) {
+    if (fmt == BT_BFP8) launch_pack_half<BT_BFP8>(src, src_dtype, batch, rows, cols, sb, sr, exps, vals, r->stream);
+    else launch_pack_half<BT_BFP4>(src, src_dtype, batch, rows, cols, sb, sr, exps, vals, r->stream);
+  } else if (fmt == BT_BFP8)
     pack_kernel<BT_BFP8><<<blocks_for(n, 256), 256, 0, r->stream>>>((const void *)src, src_dtype, batch, rows, cols,
                                                                      sb, sr, sc, (uint8_t *)exps, (uint8_t *)vals);
   else
@@ -303,12 +451,16 @@ int bt_bfp_columns(bt_runtime *rt, int fmt, uint64_t exps, uint64_t vals, int64_
   if (dst % 16) return fail(BT_EINVAL, "columns tiles must be 16-byte aligned");
   int64_t chunks = (rows + 63) / 64, nruns = (cols + 15) / 16, tiles = batch * nruns * chunks;
   if (tiles >= (1ll << 31)) return fail(BT_EINVAL, "too many tiles");
-  if (fmt == BT_BFP8)
-    columns_kernel<BT_BFP8><<<(unsigned)tiles, 64, 0, r->stream>>>((const uint8_t *)exps, (const uint8_t *)vals, rows,
-                                                                    cols, chunks, nruns, (uint8_t *)dst);
-  else
-    columns_kernel<BT_BFP4><<<(unsigned)tiles, 64, 0, r->stream>>>((const uint8_t *)exps, (const uint8_t *)vals, rows,
-                                                                    cols, chunks, nruns, (uint8_t *)dst);
+  const int64_t groups = (nruns + RUNS_B - 1) / RUNS_B;
+  const FastDiv gd = make_fastdiv((uint32_t)groups), cd = make_fastdiv((uint32_t)chunks);
+#define BT_COLUMNS(FMT, WIDE)                                                                                        \
+  columns_kernel<FMT, WIDE><<<(unsigned)(batch * chunks * groups), 256, 0, r->stream>>>(                             \
+    (const uint8_t *)exps, (const uint8_t *)vals, rows, (uint32_t)nruns, (uint32_t)chunks, gd, cd, (uint8_t *)dst)
+  if (fmt == BT_BFP8 && vals % 8 == 0) BT_COLUMNS(BT_BFP8, true);
+  else if (fmt == BT_BFP8) BT_COLUMNS(BT_BFP8, false);
+  else if (vals % 8 == 0) BT_COLUMNS(BT_BFP4, true);
+  else BT_COLUMNS(BT_BFP4, false);
+#undef BT_COLUMNS
   BT_LAUNCHED("bfp_columns");
   return BT_OK;
 }
@@ -353,16 +505,20 @@ int bt_columns_unpack(bt_runtime *rt, int fmt, uint64_t src, int64_t batch, int6
   if (int s = enter(rt, &r)) return s;
   if (fmt != BT_BF16 && fmt != BT_BFP8 && fmt != BT_BFP4) return fail(BT_EINVAL, "columns format %d", fmt);
   if (int s = check_shape(batch, rows, cols)) return s;
-  int64_t chunks = (rows + 63) / 64, nruns = (cols + 15) / 16, n = batch * rows * cols;
-  if (fmt == BT_BF16)
-    columns_unpack_kernel<BT_BF16><<<blocks_for(n, 256), 256, 0, r->stream>>>((const uint8_t *)src, batch, rows, cols,
-                                                                               chunks, nruns, (uint16_t *)dst);
-  else if (fmt == BT_BFP8)
-    columns_unpack_kernel<BT_BFP8><<<blocks_for(n, 256), 256, 0, r->stream>>>((const uint8_t *)src, batch, rows, cols,
-                                                                               chunks, nruns, (uint16_t *)dst);
-  else
-    columns_unpack_kernel<BT_BFP4><<<blocks_for(n, 256), 256, 0, r->stream>>>((const uint8_t *)src, batch, rows, cols,
-                                                                               chunks, nruns, (uint16_t *)dst);
+  const int64_t chunks = (rows + 63) / 64, nruns = (cols + 15) / 16, groups = (nruns + RUNS_B - 1) / RUNS_B;
+  if (batch * nruns * chunks >= (1ll << 31)) return fail(BT_EINVAL, "too many tiles");
+  const FastDiv gd = make_fastdiv((uint32_t)groups), cd = make_fastdiv((uint32_t)chunks);
+  const bool wide = cols % 8 == 0 && dst % 16 == 0;
+#define BT_UNPACK(FMT, WIDE)                                                                                         \
+  columns_unpack_kernel<FMT, WIDE><<<(unsigned)(batch * chunks * groups), 256, 0, r->stream>>>(                      \
+    (const uint8_t *)src, rows, cols, (uint32_t)nruns, (uint32_t)chunks, gd, cd, (uint16_t *)dst)
+  if (fmt == BT_BF16 && wide) BT_UNPACK(BT_BF16, true);
+  else if (fmt == BT_BF16) BT_UNPACK(BT_BF16, false);
+  else if (fmt == BT_BFP8 && wide) BT_UNPACK(BT_BFP8, true);
+  else if (fmt == BT_BFP8) BT_UNPACK(BT_BFP8, false);
+  else if (wide) BT_UNPACK(BT_BFP4, true);
+  else BT_UNPACK(BT_BFP4, false);
+#undef BT_UNPACK
   BT_LAUNCHED("columns_unpack");
   return BT_OK;
 }

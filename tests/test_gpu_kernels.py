@@ -144,6 +144,37 @@ def test_columns_read_back_unchanged(rt, fmt):
   assert np.array_equal(down(rt, back, w.shape, np.uint16), B.bf16_bits(w))
 
 
+# around the widths a block takes (16 runs of 64 rows), odd rows, and row starts on 16, 8, 4 and 2 bytes: `lead` values
+# before the first and `gap` after every row
+@pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
+@pytest.mark.parametrize("src", ["bf16", "fp32"])
+@pytest.mark.parametrize("shape,lead,gap", [((1, 1, 1), 0, 0), ((2, 65, 255), 0, 0), ((1, 63, 264), 8, 8), ((1, 129, 513), 1, 2),
+                                            ((3, 64, 256), 4, 4), ((2, 5, 40), 2, 0), ((1, 200, 9), 3, 8)])
+def test_block_floats_at_the_edges_of_blocks(rt, fmt, src, shape, lead, gap):
+  b, r, c = shape
+  rng = np.random.default_rng(17)
+  x = np.zeros(lead + b * r * (c + gap), np.float32)
+  x[:] = rng.normal(0, 1, x.size) * np.exp2(rng.integers(-30, 30, x.size))
+  d = up(rt, B.bf16_bits(x) if src == "bf16" else x) + lead * (2 if src == "bf16" else 4)
+  ne, nv = plain_sizes(b, r, c, fmt)
+  exps, vals = rt.dram_alloc(ne), rt.dram_alloc(nv)
+  rt.run("pack", "bfp_pack", FMT[fmt], d, _lib.DTYPES[src], b, r, c, r * (c + gap), c + gap, 1, exps, vals)
+  values = x[lead:].reshape(b, r, c + gap)[..., :c]
+  top, q = B.bfp_fields(np.pad(values, ((0, 0), (0, 0), (0, -c % 16))), fmt)
+  assert np.array_equal(down(rt, exps, (ne,), np.uint8), top.reshape(-1))
+  raw = down(rt, vals, (nv,), np.uint8)
+  stored = q.reshape(-1).view(np.uint8) if fmt == "bfp8" else (q.reshape(-1, 2)[:, 0] & 15 | (q.reshape(-1, 2)[:, 1] & 15) << 4).view(np.uint8)
+  assert np.array_equal(raw, stored)
+  want = B.decode_fields(top, q, fmt)[..., :c]
+  out = rt.dram_alloc(b * r * c * 2)
+  rt.run("readback", "columns_unpack", FMT[fmt], columns(rt, exps, vals, fmt, b, r, c), b, r, c, out)
+  assert np.array_equal(down(rt, out, (b, r, c), np.uint16), want)
+  shifted = rt.dram_alloc(nv + 8) + 4  # a value plane that starts between 8-byte words
+  rt.copy(shifted, vals, nv)
+  rt.run("readback", "columns_unpack", FMT[fmt], columns(rt, exps, shifted, fmt, b, r, c), b, r, c, out)
+  assert np.array_equal(down(rt, out, (b, r, c), np.uint16), want)
+
+
 # ---- matmul -----------------------------------------------------------------------------------------------------
 
 def test_matmul_exact(rt):
