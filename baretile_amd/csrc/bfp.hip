@@ -217,7 +217,8 @@ __device__ __forceinline__ int nibble_q(uint32_t w, int j) {  // the inverse: va
 // LDS and writes each as one contiguous stretch. One block a tile, each lane fetching its 16 values a byte at a time from
 // 16 rows, left the loads' lines mostly unused. The bound is HBM: 9/16 (bfp4) or 17/16 (bfp8) bytes a value each way.
 // LDS rows are 8 bytes longer than their runs, so that the 4 lane groups' rows, 8 apart, start 16 banks apart. WIDE: the
-// value plane starts on 8 bytes (it is byte addressed otherwise). 4096 x 14336 in bfp4: 53 us a block a tile, 25 us so (2.9 TB/s).
+// value plane starts on 8 bytes (it is byte addressed otherwise). 4096 x 14336 in bfp4: 53 us a block a tile, 25 us so
+// (2.9 TB/s).
 constexpr int RUNS_B = 16;  // runs a block
 template <int FMT, bool WIDE>
 __global__ void __launch_bounds__(256) columns_kernel(const uint8_t *exps, const uint8_t *vals, int64_t rows,
@@ -299,8 +300,8 @@ __global__ void __launch_bounds__(64) bf16_columns_kernel(const uint16_t *src, i
 // lane decoding its 16 values exactly, and the block stores the 64 rows' 256 columns from LDS as whole 512-byte
 // stretches (WIDE: every row of the result starts on 16 bytes; otherwise a thread a column). A thread a value took its
 // exponent and value a byte at a time from tiles that lie `chunks` apart. The bound is HBM: 2 bytes written a value and
-// 9/16 to 2 read. 4096 x 14336 in bfp4: UN107 us with a thread a
-// run, 41 us so (3.7 TB/s).
+// 9/16 to 2 read. 4096 x 14336 in bfp4: 187 us a thread a value, 37 us
+// so (4.1 TB/s).
 template <int FMT, bool WIDE>
 __global__ void __launch_bounds__(256) columns_unpack_kernel(const uint8_t *src, int64_t rows, int64_t cols,
                                                              uint32_t runs, uint32_t chunks, FastDiv groups,
