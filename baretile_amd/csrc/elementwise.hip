@@ -1,7 +1,8 @@
 // Fused elementwise programs, reductions, and the row gather and put that fill and read caches.
-#include "program.h"
 #include "rows.h"
+#include "segprog.h"
 #include <algorithm>
+#include <type_traits>
 
 namespace bt {
 
@@ -44,6 +45,56 @@ __global__ void __launch_bounds__(256) elementwise_seg_kernel(const bt_program p
   uint32_t io[SEG] = {};
   eval_program<DT, SEG>(prog, pre, io);
   store_segment<DT>(out, bb, r, c0, n, io);
+}
+
+// The same on a program that fits SegProgram's slots, as almost every one does. ROWS: `per` waves share a row, a wave
+// taking every per-th stretch of 64 segments of it, so that the row's own values are worked out once a wave and its
+// addresses are scalar; otherwise (rows of fewer than 64 segments) a thread a segment of the whole result.
+template <int DT, bool FULL, bool ROWS>
+__global__ void __launch_bounds__(256) elementwise_row_kernel(const SegProgram p, uint32_t units, FastDiv segs,
+                                                              FastDiv rows, FastDiv per, int32_t cols,
+                                                              const bt_operand out) {
+  uint32_t q, sg, step;  // the row of the result, the first segment, segments between a thread's
+  if constexpr (ROWS) {
+    const uint32_t w = blockIdx.x * 4u + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (w >= units) return;
+    q = fdiv(w, per), sg = (w - q * per.d) * 64 + (threadIdx.x & 63u), step = 64 * per.d;
+  } else {
+    const uint32_t s = blockIdx.x * 256u + threadIdx.x;
+    if (s >= units) return;
+    q = fdiv(s, segs), sg = s - q * segs.d, step = segs.d;
+  }
+  const uint32_t bb = fdiv(q, rows);
+  const int64_t r = q - bb * rows.d;
+  const seg_t rv = run_row<DT>(p, bb, r);
+  for (; sg < segs.d; sg += step) {
+    const int64_t c0 = (int64_t)sg * SEG;
+    const int n = (int)min((int64_t)SEG, cols - c0);
+    SegInputs x;
+    fetch_seg<DT, FULL>(p, bb, r, c0, n, x);
+    const seg_t y = run_seg<DT, FULL>(p, x, rv);
+    const uint32_t io[SEG] = {y[0], y[1], y[2], y[3], y[4], y[5], y[6], y[7]};
+    store_segment<DT>(out, bb, r, c0, n, io);
+    if (!ROWS) break;
+  }
+}
+template <int DT>
+static void launch_rows(const SegProgram &p, int64_t batch, int64_t rows, int64_t cols, const bt_operand &out, hipStream_t s) {
+  const int64_t segs = (cols + SEG - 1) / SEG;
+  const FastDiv fs = make_fastdiv((uint32_t)segs), fr = make_fastdiv((uint32_t)rows);
+  if (segs < 64) {
+    const int64_t units = batch * rows * segs;
+    const unsigned blocks = (unsigned)((units + 255) / 256);
+    if (seg_small(p)) elementwise_row_kernel<DT, false, false><<<blocks, 256, 0, s>>>(p, (uint32_t)units, fs, fr, fr, (int32_t)cols, out);
+    else elementwise_row_kernel<DT, true, false><<<blocks, 256, 0, s>>>(p, (uint32_t)units, fs, fr, fr, (int32_t)cols, out);
+    return;
+  }
+  // as many waves as fill the chip twice over (8192), at most one for each 64 segments of a row
+  const int64_t per = std::max<int64_t>(1, std::min((segs + 63) / 64, 8192 / (batch * rows))), units = batch * rows * per;
+  const FastDiv fp = make_fastdiv((uint32_t)per);
+  const unsigned blocks = (unsigned)((units + 3) / 4);
+  if (seg_small(p)) elementwise_row_kernel<DT, false, true><<<blocks, 256, 0, s>>>(p, (uint32_t)units, fs, fr, fp, (int32_t)cols, out);
+  else elementwise_row_kernel<DT, true, true><<<blocks, 256, 0, s>>>(p, (uint32_t)units, fs, fr, fp, (int32_t)cols, out);
 }
 
 // The same for results of 2^31 elements or more: one element per thread, 64-bit index arithmetic.
@@ -135,12 +186,13 @@ __global__ void __launch_bounds__(WPO > 4 ? 64 * WPO : 256) reduce_kernel(const 
   }
 }
 
-// Reductions along the last axis of large inputs: lanes take segments of SEG neighbouring columns (fetch_segment),
-// otherwise as reduce_kernel.
-template <int DT, int WPO>
-__global__ void __launch_bounds__(WPO > 4 ? 64 * WPO : 256) reduce_seg_kernel(const bt_program prog, int kind,
-                                                                               int64_t batch, int64_t rows,
-                                                                               int64_t cols, const bt_operand out) {
+// Reductions along the last axis of large inputs: lanes take segments of SEG neighbouring columns, otherwise as
+// reduce_kernel. P is a SegProgram, whose row values are worked out once for all of a row's segments, or a bt_program
+// that doesn't fit one (fetch_segment).
+template <int DT, int WPO, class P, bool FULL = true>
+__global__ void __launch_bounds__(WPO > 4 ? 64 * WPO : 256) reduce_seg_kernel(const P prog, int kind, int64_t batch,
+                                                                               int64_t rows, int64_t cols,
+                                                                               const bt_operand out) {
   __shared__ uint32_t part[WPO];
   const int lane = threadIdx.x & 63;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -149,13 +201,23 @@ __global__ void __launch_bounds__(WPO > 4 ? 64 * WPO : 256) reduce_seg_kernel(co
   const int64_t r = w % rows, b = w / rows, nseg = (cols + SEG - 1) / SEG;
   float facc = kind == BT_REDUCE_SUM ? 0.0f : -__builtin_inff();
   int32_t iacc = INT32_MIN;
+  seg_t rv;
+  if constexpr (std::is_same_v<P, SegProgram>) rv = run_row<DT>(prog, b, r);
   for (int64_t sg = (WPO > 1 ? wib * 64 : 0) + lane; sg < nseg; sg += 64 * WPO) {
     const int64_t c0 = sg * SEG;
     const int n = (int)min((int64_t)SEG, cols - c0);
-    prefile pre[SEG];
-    fetch_segment<DT>(prog, b, r, c0, n, pre);
     uint32_t io[SEG] = {};
-    eval_program<DT, SEG>(prog, pre, io);
+    if constexpr (std::is_same_v<P, SegProgram>) {
+      SegInputs x;
+      fetch_seg<DT, FULL>(prog, b, r, c0, n, x);
+      const seg_t y = run_seg<DT, FULL>(prog, x, rv);
+#pragma unroll
+      for (int v = 0; v < SEG; v++) io[v] = y[v];
+    } else {
+      prefile pre[SEG];
+      fetch_segment<DT>(prog, b, r, c0, n, pre);
+      eval_program<DT, SEG>(prog, pre, io);
+    }
 #pragma unroll
     for (int v = 0; v < SEG; v++) {
       if (v >= n) continue;
@@ -313,7 +375,12 @@ int bt_elementwise(bt_runtime *rt, const bt_program *prog, int64_t batch, int64_
     if (total >= (1 << 16) && cols >= SEG && nseg < (1ll << 31)) {
       const FastDiv fs = make_fastdiv((uint32_t)segs);
       const unsigned blocks = (unsigned)((nseg + 255) / 256);
-      if (prog->dtype == BT_BF16)
+      SegProgram sp;
+      if (sp.make(*prog, batch, rows, cols)) {
+        if (prog->dtype == BT_BF16) launch_rows<BT_BF16>(sp, batch, rows, cols, *out, r->stream);
+        else if (prog->dtype == BT_FP32) launch_rows<BT_FP32>(sp, batch, rows, cols, *out, r->stream);
+        else launch_rows<BT_INT32>(sp, batch, rows, cols, *out, r->stream);
+      } else if (prog->dtype == BT_BF16)
         elementwise_seg_kernel<BT_BF16><<<blocks, 256, 0, r->stream>>>(*prog, (uint32_t)nseg, fs, fr, (int32_t)cols, *out);
       else if (prog->dtype == BT_FP32)
         elementwise_seg_kernel<BT_FP32><<<blocks, 256, 0, r->stream>>>(*prog, (uint32_t)nseg, fs, fr, (int32_t)cols, *out);
@@ -362,17 +429,29 @@ int bt_reduce(bt_runtime *rt, const bt_program *prog, int kind, int axis, int64_
     else reduce_kernel<BT_INT32, WPO><<<blocks, threads, 0, r->stream>>>(*prog, kind, axis, batch, rows, cols, sweep, step, *out); \
   } while (0)
   if (axis == 2 && cols >= 64 && outs * cols >= (1 << 16)) {  // large: segments of neighbouring columns
-#define BT_RSEG(WPO, blocks)                                                                                      \
+#define BT_RSEG(WPO, P, FULL, p)                                                                                    \
   do {                                                                                                          \
-    const unsigned threads = WPO > 4 ? 64 * WPO : 256;                                                          \
+    const unsigned blocks = (unsigned)(WPO > 1 ? outs : (outs + 3) / 4), threads = WPO > 4 ? 64 * WPO : 256;    \
     if (prog->dtype == BT_BF16)                                                                                 \
-      reduce_seg_kernel<BT_BF16, WPO><<<blocks, threads, 0, r->stream>>>(*prog, kind, batch, rows, cols, *out);   \
+      reduce_seg_kernel<BT_BF16, WPO, P, FULL><<<blocks, threads, 0, r->stream>>>(p, kind, batch, rows, cols, *out); \
     else if (prog->dtype == BT_FP32)                                                                            \
-      reduce_seg_kernel<BT_FP32, WPO><<<blocks, threads, 0, r->stream>>>(*prog, kind, batch, rows, cols, *out);   \
-    else reduce_seg_kernel<BT_INT32, WPO><<<blocks, threads, 0, r->stream>>>(*prog, kind, batch, rows, cols, *out); \
+      reduce_seg_kernel<BT_FP32, WPO, P, FULL><<<blocks, threads, 0, r->stream>>>(p, kind, batch, rows, cols, *out); \
+    else reduce_seg_kernel<BT_INT32, WPO, P, FULL><<<blocks, threads, 0, r->stream>>>(p, kind, batch, rows, cols, *out); \
   } while (0)
-    if (outs < 2048) BT_RSEG(4, (unsigned)outs);  // (16 waves would leave each lane too few registers)
-    else BT_RSEG(1, (unsigned)((outs + 3) / 4));
+    SegProgram sp;
+    if (!sp.make(*prog, batch, rows, cols)) {
+      if (outs < 2048) BT_RSEG(4, bt_program, true, *prog);  // (16 waves would leave each lane too few registers)
+      else BT_RSEG(1, bt_program, true, *prog);
+    } else {
+      // a row's segments are a chain of loads for each lane, so four waves take a row of more than one turn wherever
+      // the rows alone wouldn't fill the chip several times (2048 rows of 4096: 14.4 -> 9.0 us)
+      const int64_t turns = (cols + 64 * SEG - 1) / (64 * SEG);
+      const bool small = seg_small(sp), four = turns > 1 && outs < 16384;
+      if (small && four) BT_RSEG(4, SegProgram, false, sp);
+      else if (small) BT_RSEG(1, SegProgram, false, sp);
+      else if (four) BT_RSEG(4, SegProgram, true, sp);
+      else BT_RSEG(1, SegProgram, true, sp);
+    }
 #undef BT_RSEG
     BT_LAUNCHED("reduce");
     return BT_OK;

@@ -186,8 +186,8 @@ __device__ __attribute__((noinline)) float long_op(int op, float a) { return lon
 
 // One instruction over V values. op is uniform, so the switch is a scalar branch around straight vector code. INL
 // inlines the long operations too: for callers that hold many live registers (a GEMM's accumulators), which a call
-// would have to save to memory.
-template <int DT, int V, bool INL = false>
+// would have to save to memory. Without LONG the caller takes them itself.
+template <int DT, int V, bool INL = false, bool LONG = true>
 __device__ __forceinline__ Vals<V> apply_op(int op, const Vals<V> &a, const Vals<V> &b) {
   Vals<V> o;
   if (DT == BT_INT32) {
@@ -222,7 +222,7 @@ __device__ __forceinline__ Vals<V> apply_op(int op, const Vals<V> &a, const Vals
     BT_OP(BT_OP_FTOB, round_packed(A))
     default:
 #pragma unroll
-      for (int v = 0; v < V; v++) f[v] = INL ? long_op_inline(op, x[v]) : long_op(op, x[v]);
+      for (int v = 0; v < V; v++) f[v] = !LONG ? x[v] : INL ? long_op_inline(op, x[v]) : long_op(op, x[v]);
   }
 #undef BT_OP
 #pragma unroll

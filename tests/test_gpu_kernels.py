@@ -494,6 +494,70 @@ def test_reductions(rt):
 
 # ---- attention --------------------------------------------------------------------------------------------------
 
+def random_program(rt, rng, dtype, shape, where):
+  """A program of random instructions over inputs of random forms (whole, one row or one value a row for all, every
+  second column, each dtype), and a function that gives it for batch entry b alone."""
+  b, r, c = shape
+  inputs = []
+  for _ in range(int(rng.integers(1, 7))):
+    kind = rng.choice(["bf16", "fp32", "int32"]) if dtype != "int32" else "int32"
+    sb, sr, sc = [(r * c, c, 1), (0, 0, 1), (r, 1, 0), (0, 0, 0), (2 * r * c, 2 * c, 2)][int(rng.choice(5, p=[.4, .2, .2, .1, .1]))]
+    values = rng.normal(0, 2, 2 * b * r * c) if kind != "int32" else rng.integers(-9, 10, 2 * b * r * c)
+    dev = up(rt, B.bf16_bits(values) if kind == "bf16" else values.astype(np.float32 if kind == "fp32" else np.int32))
+    inputs.append((dev, kind, sb, sr, sc))
+  names = (["add", "sub", "mul", "max", "min", "cmplt", "cmpeq", "neg", "relu"] +
+           (["div", "exp", "sqrt", "recip", "sigmoid", "silu", "tanh", "gelu", "sin", "ftob", "log2"] if dtype != "int32" else []) +
+           (["where"] if where else []))
+  picks = [(rng.choice(names), rng.random(3)) for _ in range(int(rng.integers(1, 16)))]
+  def build(entry):
+    p = Program(dtype)
+    size = lambda kind: 2 if kind == "bf16" else 4
+    regs = [p.load(p.input(_lib.operand(dev + entry * sb * size(kind), kind, sb, sr, sc))) for dev, kind, sb, sr, sc in inputs]
+    regs.append(p.const(3 if dtype == "int32" else 0.7))
+    for name, at in picks:  # mostly the newest values, so that chains and values kept for later both come up
+      src = [regs[-1 - int(u * u * len(regs))] for u in at]
+      regs.append(p.op(str(name), *src[:3 if name == "where" else 1 if name in Program.UNARY else 2]))
+    return p.build(regs[-1])
+  return build
+
+
+# results of 65,536 values and more run on segments of 8 columns, smaller ones a value a thread: the same program on
+# both, bit for bit, over programs that fit the segment kernels' slots and ones that don't
+@pytest.mark.parametrize("dtype", ["bf16", "fp32", "int32"])
+@pytest.mark.parametrize("shape", [(2, 40, 1000), (2, 9, 3645), (5, 2000, 9)])
+def test_large_programs_equal_small_ones(rt, dtype, shape):
+  b, r, c = shape
+  assert b * r * c >= 1 << 16 > r * c
+  rng = np.random.default_rng(r)
+  kind = np.uint16 if dtype == "bf16" else np.uint32
+  whole, entry = (rt.dram_alloc(n * r * c * kind().itemsize) for n in (b, 1))
+  out = lambda ptr: ctypes.byref(_lib.operand(ptr, dtype, r * c, c, 1))
+  top, some = rt.dram_alloc(b * r * 4), rt.dram_alloc(b * r * 4)
+  nan = lambda x: np.isnan(bits_to_float(x) if dtype == "bf16" else x.view(np.float32)) if dtype != "int32" else x != x
+  for trial in range(30):
+    build = random_program(rt, rng, dtype, shape, where=trial % 2)
+    prog = build(0)
+    rt.run("elementwise", "elementwise", ctypes.byref(prog), b, r, c, out(whole))
+    got = down(rt, whole, shape, kind)
+    for e in range(b):
+      rt.run("elementwise", "elementwise", ctypes.byref(build(e)), 1, r, c, out(entry))
+      want = down(rt, entry, (r, c), kind)
+      assert np.all((got[e] == want) | nan(got[e]) & nan(want)), (trial, e)
+    if dtype == "bf16" or c < 64: continue
+    row = ctypes.byref(_lib.operand(top, dtype, r, 1, 1))
+    rt.run("reduce", "reduce", ctypes.byref(prog), _lib.REDUCE_MAX, 2, b, r, c, 0, 0, row)
+    vals = got.view(np.float32 if dtype == "fp32" else np.int32)
+    best = down(rt, top, (b, r), vals.dtype)
+    assert np.array_equal(best, vals.max(2), equal_nan=dtype == "fp32"), trial  # a NaN anywhere is the row's maximum
+    if dtype == "fp32" and np.isfinite(vals).all():  # fp32 sums of c values: within c 2^-24 of the sum of magnitudes
+      rt.run("reduce", "reduce", ctypes.byref(prog), _lib.REDUCE_SUM, 2, b, r, c, 0, 0, ctypes.byref(_lib.operand(some, dtype, r, 1, 1)))
+      total = vals.astype(np.float64)
+      bound = c * 2.0 ** -24 * np.abs(total).sum(2)
+      sums = down(rt, some, (b, r), np.float32)
+      ok = np.abs(total).sum(2) < 3e38  # past that fp32 partial sums may overflow
+      assert np.all((np.abs(sums - total.sum(2)) <= bound)[ok]), trial
+
+
 def attend(rt, q, k, v, places, window=0, parts=0):
   """q (E, rows, hd), k/v (E/rep, keys, hd), places (1|E, rows) -> bf16 result as float32."""
   E, rows, hd = q.shape
