@@ -17,6 +17,7 @@
 #include "rows.h"
 #include "lds_load.h"
 #include <cstdlib>
+#include <type_traits>
 
 namespace bt {
 
@@ -84,6 +85,20 @@ __device__ __forceinline__ bf16x8 q8_to_bf16(uint2 q, uint2 d) {
     w[p] = pack_hi(f[0], f[1]);
   }
   uint4 v = make_uint4(w[0], w[1], w[2], w[3]);
+  return *(const bf16x8 *)&v;
+}
+
+// bfp8: eight signed bytes times their own fp32 powers of two (t.x .. u.w), as bf16: the values q8_to_bf16<true> gives.
+__device__ __forceinline__ bf16x8 q8_to_bf16_times(uint2 q, const uint4 &t, const uint4 &u) {
+  const uint32_t sc[8] = {t.x, t.y, t.z, t.w, u.x, u.y, u.z, u.w};
+  uint32_t w[4];
+#pragma unroll
+  for (int p = 0; p < 4; p++) {
+    const uint32_t qw = p < 2 ? q.x : q.y;
+    w[p] = pack_hi((float)(int)(int8_t)(qw >> (16 * (p & 1))) * __uint_as_float(sc[2 * p]),
+                   (float)(int)(int8_t)(qw >> (16 * (p & 1) + 8)) * __uint_as_float(sc[2 * p + 1]));
+  }
+  const uint4 v = make_uint4(w[0], w[1], w[2], w[3]);
   return *(const bf16x8 *)&v;
 }
 
@@ -1417,6 +1432,72 @@ __global__ void __launch_bounds__(256) parts_reduce_kernel(const MatmulArgs args
   }
 }
 
+// The sums of gemm3's partial products (GEMM_PART) and what follows them: EPI 0 the product in out's dtype, 1 a residual
+// added (res, fp32 out), 2 SiLU x up, 3 any epilogue program. A thread takes 4 neighbouring columns with 16-byte loads
+// where n is a multiple of 4 (V 4), else one. The partials are added in fp64, so that splitting K costs no precision:
+// the sum that reaches the epilogue is the exact partials' rounded once.
+template <int V> __device__ __forceinline__ void sum_parts(const float *p, int splits, int64_t stride, float (&o)[V]) {
+  typedef float vec __attribute__((ext_vector_type(V)));
+  double t[V] = {};
+#pragma unroll 4
+  for (int s = 0; s < splits; s++) {
+    const vec x = gload((const vec *)(p + s * stride));
+#pragma unroll
+    for (int v = 0; v < V; v++) t[v] += (double)x[v];
+  }
+#pragma unroll
+  for (int v = 0; v < V; v++) o[v] = (float)t[v];
+}
+template <int DT, int EPI, int V>
+__global__ void __launch_bounds__(256) gemm_sum_kernel(const MatmulArgs args, int splits, FastDiv pieces,
+                                                       const float *part, const bt_operand res) {
+  const uint32_t e = blockIdx.x * 256u + threadIdx.x, row = fdiv(e, pieces);
+  if (row >= (uint32_t)args.m) return;
+  const int m = (int)row, n = (int)(e - row * pieces.d) * V;
+  const int64_t stride = (int64_t)args.m * args.n;
+  const float *p = part + (int64_t)m * args.n + n;
+  const bt_operand &out = args.out;
+  float x[V], r[V];
+  uint32_t o[V];
+  if constexpr (EPI == 1) {
+#pragma unroll
+    for (int v = 0; v < V; v++) r[v] = ((const float *)res.ptr)[(int64_t)m * res.sr + (int64_t)(n + v) * res.sc];
+  }
+  sum_parts<V>(p, splits, stride, x);
+  if constexpr (EPI == 2) {
+    float u[V];
+    sum_parts<V>(p + args.n / 2, splits, stride, u);
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      const float gv = bf16_value(bf16_packed(x[v])), uv = bf16_value(bf16_packed(u[v]));
+      o[v] = bf16_packed(gv / (1.0f + expf(-gv)) * uv);
+    }
+  } else if constexpr (EPI == 3) {
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      const uint32_t y = run_program<DT>(args.prog, 0, m, n + v, __float_as_uint(DT == BT_BF16 ? round_packed(x[v]) : x[v]));
+      store_value<DT>(out, (int64_t)m * out.sr + (int64_t)(n + v) * out.sc, y);
+    }
+    return;
+  } else {
+#pragma unroll
+    for (int v = 0; v < V; v++)
+      o[v] = out.dtype == BT_BF16 ? bf16_packed(x[v]) : __float_as_uint(EPI == 1 ? x[v] + r[v] : x[v]);
+  }
+  const int64_t at = (int64_t)m * out.sr + (int64_t)n * out.sc;
+  if (V == 4 && out.sc == 1 && out.dtype == BT_BF16 && (out.ptr + at * 2) % 8 == 0) {
+    *(uint2 *)((uint16_t *)out.ptr + at) = make_uint2(o[0] | o[1] << 16, o[V / 2] | o[V - 1] << 16);
+  } else if (V == 4 && out.sc == 1 && out.dtype != BT_BF16 && (out.ptr + at * 4) % 16 == 0) {
+    *(uint4 *)((uint32_t *)out.ptr + at) = make_uint4(o[0], o[V / 4], o[V / 2], o[V - 1]);
+  } else {
+#pragma unroll
+    for (int v = 0; v < V; v++) {
+      if (out.dtype == BT_BF16) ((uint16_t *)out.ptr)[at + v * out.sc] = (uint16_t)o[v];
+      else ((uint32_t *)out.ptr)[at + v * out.sc] = o[v];
+    }
+  }
+}
+
 // 5 to 32 rows of one A (K a multiple of 256) against B streamed once. Block (group, split) takes W runs of B, a wave
 // each, over its split's stages of 4 chunks (256 rows of K). Every load goes straight into LDS, whole and aligned: a
 // stage of a run's tiles is one contiguous stretch (4 x 576 bytes for bfp4), loaded 1 KB a wave instruction, and each
@@ -1723,9 +1804,13 @@ gemm2_kernel(const MatmulArgs args, int mblocks, int nblocks) {
 // MODE 2 (SWIGLU): B holds gate then up side by side (n = 2 f columns); a block takes 128 columns of each, at the
 // same place in both halves, and writes silu(gate) * up for those 128 columns (out: m x f, bf16): the gate and up
 // values rounded to bf16 as stored, silu(g) = g / (1 + exp(-g)) and the product in fp32, rounded once.
-constexpr int GEMM_PLAIN = 0, GEMM_RES = 1, GEMM_SWIGLU = 2;
+constexpr int GEMM_PLAIN = 0, GEMM_RES = 1, GEMM_SWIGLU = 2, GEMM_PART = 3;
 // BM: the block's rows, 256 or 128 (a wave BM / 2 of them by 64 columns), for products whose 256-row blocks would
 // leave CUs idle.
+// FMT 3 (bfp8 B) as FMT 4 below, the tiles' values 1 KB a load and their exponent bytes turned into fp32 powers of two
+// once a chunk, so that a value's decode is a convert and a multiply (20 instructions for 8 values, bfp4's 7).
+// MODE GEMM_PART: the grid holds mblocks x nblocks blocks for each of several splits of K (nb_off chunks each), and
+// writes fp32 partial sums for gemm_sum_kernel.
 // FMT 4 (bfp4 B) stages a chunk (64 rows of K) at a time, CS = 3 deep (4 for 128-row blocks): A as BM rows of 128
 // bytes (unit u of row r at u ^ (r % 8), so the fragment reads of 8 neighbouring rows meet different banks) and the
 // block's 16 tiles as they are stored, 576 bytes each (36 lanes of a direct load). The wave that loaded a tile places
@@ -1741,14 +1826,13 @@ constexpr int GEMM_PLAIN = 0, GEMM_RES = 1, GEMM_SWIGLU = 2;
 template <int FMT, int DT, int S, int MODE = GEMM_PLAIN, int BM = 256, int BN = 256>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand res, int nb_off = 0) {
-  static_assert(FMT == BT_BF16 || FMT == BT_BFP4, "gemm3 takes bf16 or bfp4 B");
   static_assert(BN == 256 || (BN == 192 && MODE != GEMM_SWIGLU) ||
                     (BN == 384 && FMT == BT_BFP4 && BM == 128 && MODE != GEMM_SWIGLU),
                 "gemm3 blocks are 256 or 192 columns, or 128 x 384 on bfp4 B");
   constexpr bool RES = MODE == GEMM_RES;
   // the 8 waves as 2 x 4 (each BM / 2 rows by BN / 4 columns); bfp4 B, where the columns allow, as 1 x 8 (each all BM
   // rows by BN / 8 columns), so that each tile is decoded by one wave, not two, for as many matrix instructions
-  constexpr int WAVES_M = FMT == BT_BFP4 && BN % 128 == 0 ? 1 : 2, WAVES_N = 8 / WAVES_M;
+  constexpr int WAVES_M = FMT != BT_BF16 && BN % 128 == 0 ? 1 : 2, WAVES_N = 8 / WAVES_M;
   constexpr int A_BYTES = BM * 64, STAGE = A_BYTES + 16384, WM = BM / (16 * WAVES_M), WN = BN / (16 * WAVES_N),
                 WR = BM / WAVES_M, T = BN / 16;
   static_assert(WN * 16 * WAVES_N == BN, "the waves' columns cover the block");
@@ -1756,7 +1840,11 @@ gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand r
   // bfp4: chunk stages of A's rows, the 16 tiles as stored, then the tiles' exponents as placed gaps (128 B a tile)
   // TT: tile slots a stage (16, or 24 for 384 columns), NB of them loaded by each wave
   constexpr int TT = BN / 16 > 16 ? BN / 16 : 16, NB = TT / 8;
-  constexpr int CS = BM == 128 ? 4 : 3, QTB = 576, QA = BM * 128, QG = QA + TT * QTB, QSTAGE = QG + TT * 128, QAL = BM / 64;
+  // bfp8: chunk stages of A's rows, the tiles' values, their exponents as fp32 powers of two (256 B a tile), and the
+  // exponent bytes as loaded
+  constexpr bool Q8 = FMT == BT_BFP8;
+  constexpr int QTB = Q8 ? 1024 : 576, QG_TILE = Q8 ? 256 : 128, QA = BM * 128, QG = QA + TT * QTB, QE = QG + TT * QG_TILE,
+                QSTAGE = QE + (Q8 ? TT * 64 : 0), QAL = BM / 64, CS = 4 * QSTAGE <= 160 * 1024 ? 4 : 3;
   constexpr int RING = FMT == BT_BF16 ? S * STAGE : CS * QSTAGE;
   constexpr int ESZ = DT == BT_FP32 ? 4 : 2, ES = BN * ESZ + 16;
   constexpr int HALF = (DT == BT_FP32 ? 128 : 256) < BM ? (DT == BT_FP32 ? 128 : 256) : BM;
@@ -1765,16 +1853,20 @@ gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand r
   const Head h = early_head(args);
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, col = lane & 15;
   const int wib = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wib / WAVES_N, wn = wib % WAVES_N;
-  const int per = mblocks * nblocks, total = per * h.batch, full = total / 8 * 8;
+  // GEMM_PART: the grid's batch entries are splits of K, nb_off chunks each
+  const int per = mblocks * nblocks, total = MODE == GEMM_PART ? gridDim.x : per * h.batch, full = total / 8 * 8;
   int pid = blockIdx.x;
   if (pid < full) pid = (pid % 8) * (full / 8) + pid / 8;  // neighbouring blocks on one XCD
-  const int b = pid / per;
+  const int split = MODE == GEMM_PART ? pid / per : 0, b = MODE == GEMM_PART ? 0 : pid / per;
   pid %= per;
+  const int chunk0 = MODE == GEMM_PART ? split * nb_off : 0;
+  const int chunk1 = MODE == GEMM_PART ? min(chunk0 + nb_off, h.chunks) : h.k / 64;  // (bf16 B counts steps of 32)
   // blocks of a column of GROUP block rows run together, sharing B's tiles in L2: 8 rows with bf16 B; 2 with bfp4 B,
   // whose tiles are 0.28 of A's bytes, so that each XCD's blocks hold fewer rows of A at once (1-2% faster there)
-  constexpr int GROUP = FMT == BT_BFP4 ? 2 : 8;
+  constexpr int GROUP = FMT != BT_BF16 ? 2 : 8;
   const int width = GROUP * nblocks, first = pid / width * GROUP, gsz = min(mblocks - first, GROUP);
-  const int bm = first + pid % width % gsz, bn = nb_off + pid % width / gsz;  // nb_off: the launch's first block column
+  const int bm = first + pid % width % gsz;
+  const int bn = (MODE == GEMM_PART ? 0 : nb_off) + pid % width / gsz;  // nb_off: the launch's first block column
   const int m0 = bm * BM, n0 = bn * BN;
 
   const uint16_t *abase = (const uint16_t *)h.a.ptr + operand_matrix(h.a, b) * h.a.sb;
@@ -1822,11 +1914,11 @@ gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand r
       lds_load16(br, bsrc[j] == NOWHERE ? NOWHERE : bsrc[j] + bo, st + A_BYTES + li * 1024);
     }
   };
-  const int steps = h.k / 32;
+  const int steps = MODE == GEMM_PART ? 2 * chunk1 : h.k / 32, step0 = 2 * chunk0;
 #pragma unroll
   for (int t = 0; t < S - 1; t++)
-    if (t < steps) issue(t);
-  for (int t = 0; t < steps; t++) {
+    if (step0 + t < steps) issue(step0 + t);
+  for (int t = step0; t < steps; t++) {
     // step t landed once at most the later steps' loads are outstanding (fewer near the end)
     if (t + S - 2 < steps) wait_vm<(AL + 2) * (S - 2)>();
     else wait_vm<0>();
@@ -1847,7 +1939,8 @@ gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand r
       for (int j = 0; j < WN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
   }
   } else {
-    const i32x4 br = buffer_words(bbase, (uint32_t)((int64_t)h.nruns * h.chunks * QTB));
+    constexpr int TB = Tile<FMT>::bytes;
+    const i32x4 br = buffer_words(bbase, (uint32_t)((int64_t)h.nruns * h.chunks * TB));
     // each lane's source for the wave's QAL A loads (8 rows of 128 bytes each; lane l takes row l / 8, unit
     // (l % 8) ^ (row % 8)) and 2 B tiles (tiles wib and wib + 8, lanes 0..35) of chunk 0; a chunk adds 128 bytes to
     // A's, one tile to B's
@@ -1861,48 +1954,78 @@ gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand r
     for (int j = 0; j < NB; j++) {
       bool in;
       const int run = b_run(wib + 8 * j, in);
-      bq[j] = in ? (uint32_t)((int64_t)run * h.chunks * QTB + 16 * lane) : NOWHERE;
+      bq[j] = in ? (uint32_t)((int64_t)run * h.chunks * TB + (Q8 ? 64 : 0) + 16 * lane) : NOWHERE;
+    }
+    uint32_t be = NOWHERE;  // bfp8: the wave's NB tiles' exponents, 4 lanes a tile
+    if constexpr (Q8) {
+      if (lane < 4 * NB) {
+        bool in;
+        const int run = b_run(wib + 8 * (lane >> 2), in);
+        if (in) be = (uint32_t)((int64_t)run * h.chunks * TB + 16 * (lane & 3));
+      }
     }
     auto issue = [&](int c) {  // chunk c's loads into stage c % CS
       uint8_t *st = lds + (c % CS) * QSTAGE;
-      const uint32_t ao = (uint32_t)c * 128, bo = (uint32_t)c * QTB;
+      const uint32_t ao = (uint32_t)c * 128, bo = (uint32_t)c * TB;
 #pragma unroll
       for (int j = 0; j < QAL; j++) lds_load16(ar, aq[j] == NOWHERE ? NOWHERE : aq[j] + ao, st + (wib + 8 * j) * 1024);
 #pragma unroll
       for (int j = 0; j < NB; j++)
         if (lane < QTB / 16) lds_load16(br, bq[j] == NOWHERE ? NOWHERE : bq[j] + bo, st + QA + (wib + 8 * j) * QTB);
+      if constexpr (Q8)
+        if (lane < 4 * NB) lds_load16(br, be == NOWHERE ? NOWHERE : be + bo, st + QE + wib * 64 * NB);
     };
-    const int chunks = h.k / 64;
+    const int chunks = chunk1;
 #pragma unroll
     for (int c = 0; c < CS - 1; c++)
-      if (c < chunks) issue(c);
-    for (int c = 0; c < chunks; c++) {
-      if (c + CS - 2 < chunks) wait_vm<(QAL + NB) * (CS - 2)>();
+      if (chunk0 + c < chunks) issue(chunk0 + c);
+    for (int c = chunk0; c < chunks; c++) {
+      if (c + CS - 2 < chunks) wait_vm<(QAL + NB + (Q8 ? 1 : 0)) * (CS - 2)>();
       else wait_vm<0>();
       uint8_t *st = lds + (c % CS) * QSTAGE;
       // the exponent bytes of the wave's own two tiles have landed (its loads wrote them): placed as gaps once here,
       // for every wave that reads the tiles, instead of by each of them (lanes 16 s .. 16 s + 15: tile wib + 8 s)
-      if (lane < 16 * NB) {
+      if constexpr (Q8) {  // bfp8: as the powers of two that multiply the values
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+          *(float *)(st + QG + (wib + 8 * j) * QG_TILE + 4 * lane) = ldexpf(1.0f, *(const int8_t *)(st + QE + (wib * NB + j) * 64 + lane));
+      } else if (lane < 16 * NB) {
         const int s = wib + 8 * (lane >> 4), w = lane & 15;
         *(uint2 *)(st + QG + s * 128 + 8 * w) = place_gaps(*(const uint32_t *)(st + QA + s * QTB + 4 * w));
       }
       __syncthreads();
       if (c + CS - 1 < chunks) issue(c + CS - 1);  // into the stage chunk c - 1 used
-      uint2 q[WN];
+      // a tile's values of the lane's two halves, and what scales each half's: gaps (bfp4) or powers of two (bfp8)
+      typedef std::conditional_t<Q8, uint4, uint2> Values;
+      struct Scales {
+        uint4 a, b;
+      };
+      Values q[WN];
 #pragma unroll
-      for (int j = 0; j < WN; j++) q[j] = *(const uint2 *)(st + QA + (wn * WN + j) * QTB + 64 + 8 * lane);
+      for (int j = 0; j < WN; j++)
+        q[j] = *(const Values *)(st + QA + (wn * WN + j) * QTB + (Q8 ? 0 : 64) + sizeof(Values) * lane);
+      auto decode = [&](int j, int hh, const Scales &sc) {
+        if constexpr (Q8) return hh ? q8_to_bf16_times(make_uint2(q[j].z, q[j].w), sc.a, sc.b) : q8_to_bf16_times(make_uint2(q[j].x, q[j].y), sc.a, sc.b);
+        else return q4_to_bf16_placed(hh ? q[j].y : q[j].x, sc.a);
+      };
       // lane group g's 8 values of half hh: A's 16-byte unit g + 4 hh of each row, B's gaps 16 g + 8 hh ..
       auto a_frag = [&](int i, int hh) {
         const int r = wm * WR + 16 * i + col;
         return *(const bf16x8 *)(st + r * 128 + 16 * ((g + 4 * hh) ^ (r & 7)));
       };
-      auto gaps = [&](int j, int hh) { return *(const uint4 *)(st + QG + (wn * WN + j) * 128 + 32 * g + 16 * hh); };
+      auto gaps = [&](int j, int hh) {
+        const uint4 *p = (const uint4 *)(st + QG + (wn * WN + j) * QG_TILE + (Q8 ? 64 * g + 32 * hh : 32 * g + 16 * hh));
+        Scales sc;
+        sc.a = p[0];
+        if constexpr (Q8) sc.b = p[1];
+        return sc;
+      };
       bf16x8 fa[WM], fb[WN], fb1[WN];
-      uint4 gp[WN];
+      Scales gp[WN];
 #pragma unroll
       for (int i = 0; i < WM; i++) fa[i] = a_frag(i, 0);
 #pragma unroll
-      for (int j = 0; j < WN; j++) fb[j] = q4_to_bf16_placed(q[j].x, gaps(j, 0));
+      for (int j = 0; j < WN; j++) fb[j] = decode(j, 0, gaps(j, 0));
       __builtin_amdgcn_sched_barrier(0);
       // the first half's matrix instructions a row of tiles at a time, the second half's reads and decode between
       // them, so that their VALU work issues while the matrix core is busy: after row i, A's fragment i of the second
@@ -1916,7 +2039,7 @@ gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand r
         if (i == 0)
 #pragma unroll
           for (int j = 0; j < WN; j++) gp[j] = gaps(j, 1);
-        if (i >= WM - WN) fb1[i - (WM - WN)] = q4_to_bf16_placed(q[i - (WM - WN)].y, gp[i - (WM - WN)]);
+        if (i >= WM - WN) fb1[i - (WM - WN)] = decode(i - (WM - WN), 1, gp[i - (WM - WN)]);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -1924,6 +2047,19 @@ gemm3_kernel(const MatmulArgs args, int mblocks, int nblocks, const bt_operand r
 #pragma unroll
         for (int j = 0; j < WN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fb1[j], acc[i][j], 0, 0, 0);
     }
+  }
+  if constexpr (MODE == GEMM_PART) {  // fp32 partial sums, matrix `split` of res
+    float *part = (float *)res.ptr + (int64_t)split * res.sb;
+#pragma unroll
+    for (int i = 0; i < WM; i++)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int j = 0; j < WN; j++) {
+          const int m = m0 + wm * WR + 16 * i + 4 * g + r, n = n0 + wn * 16 * WN + 16 * j + col;
+          if (m < h.m && n < h.n) part[(int64_t)m * res.sr + n] = acc[i][j][r];
+        }
+    return;
   }
   if constexpr (RES) {
     // lanes 0..15 of a row group write 16 neighbouring columns: 64 bytes
@@ -2584,6 +2720,72 @@ static bool residual_program(const MatmulArgs &args, bt_operand *res) {
   return true;
 }
 
+// Split-K plan of the tiled GEMM, from the shape alone (so every format of B sums K alike): a prompt's chunk of up to
+// about a thousand rows makes too few 128 x 256 blocks for 256 CUs (48 for 333 rows by 4096 columns), each with all of
+// K to walk. Below the row and size limits the kernels of few rows are faster (64 rows against 4096 x 1024 in bfp8: 12.3
+// us there, 14.1 here; 100 against 2048 x 2048 12.3 and 14.8; 100 against 1024 x 3072 11.2 and 13.8); above them they
+// lose by 1.1-1.6x (64 rows against 4096 x 4096 21.5 and 19.8 us, 100 against 2560 x 2560 24.2 and 17.3). Measured with
+// the splits (bfp8, bf16 out; before, on 128 x 128 blocks or on B unpacked): 333 x 4096 x 4096 70.6 -> 30.6 us,
+// 333 x 14336 x 4096 233 -> 67, 600 x 4096 x 6144 76 -> 53, 1000 x 4096 x 4096 74 -> 55.
+struct GemmSplit {
+  int splits, per, mb, nb;  // per: chunks a split
+};
+static bool gemm_split_plan(const MatmulArgs &args, GemmSplit *p) {
+  const bt_operand &a = args.a;
+  const int64_t size = (int64_t)args.k * args.n;
+  const bool few = args.m <= 32 || (args.m <= 64 ? args.k < 4096 || size < (16 << 20)
+                                                 : args.m <= 128 ? args.k < 1280 || size < 6000000 : args.k < (args.m <= 256 ? 1280 : 1024));
+  if (few || args.batch != 1 || args.k % 64 || a.sc != 1 || a.ptr % 16 || a.sr % 8 || a.rep != 1 || a.cyc != 0 ||
+      ((int64_t)(args.m - 1) * a.sr + args.k) * 2 >= (1ll << 32) || (int64_t)args.chunks * args.nruns * 2048 >= (1ll << 32))
+    return false;
+  p->mb = (args.m + 127) / 128, p->nb = (args.n + 255) / 256;
+  const int64_t blocks = (int64_t)p->mb * p->nb;
+  if (blocks > 128 || (int64_t)args.m * args.n >= (1ll << 31)) return false;
+  // the fewest us by what was measured: a round of blocks 1.2 a chunk and 8 for its fill and store, more than one split
+  // 4 for the summing launch and its partial sums written and read at 4 TB/s
+  double best = 1e30;
+  p->splits = 1;
+  for (int sp = 1; sp <= 16 && args.chunks / sp >= 4; sp++) {
+    const int per = (args.chunks + sp - 1) / sp, real = (args.chunks + per - 1) / per;
+    if (real != sp) continue;
+    const double rounds = (double)((blocks * sp + 255) / 256);
+    const double t = rounds * (per * 1.2 + 8.0) + (sp > 1 ? 4.0 + (double)sp * args.m * args.n * 8 / 4e6 : 0.0);
+    if (t < best) best = t, p->splits = sp, p->per = per;
+  }
+  return p->splits > 1;
+}
+template <int FMT>
+static void launch_gemm_parts(const MatmulArgs &args, const GemmSplit &p, float *part, hipStream_t s) {
+  bt_operand o{};
+  o.ptr = (uint64_t)(uintptr_t)part, o.sb = (int64_t)args.m * args.n, o.sr = args.n, o.sc = 1, o.rep = 1;
+  gemm3_kernel<FMT, BT_BF16, 4, GEMM_PART, 128><<<(unsigned)(p.mb * p.nb * p.splits), 512, 0, s>>>(args, p.mb, p.nb, o, p.per);
+}
+static bool launch_gemm_split(Runtime *r, const MatmulArgs &args, int fmt, bool swi) {
+  GemmSplit p;
+  if (!gemm_split_plan(args, &p)) return false;
+  float *part = (float *)runtime_scratch(r, (size_t)p.splits * args.m * args.n * 4);
+  if (!part) return false;
+  if (fmt == BT_BF16) launch_gemm_parts<BT_BF16>(args, p, part, r->stream);
+  else if (fmt == BT_BFP8) launch_gemm_parts<BT_BFP8>(args, p, part, r->stream);
+  else launch_gemm_parts<BT_BFP4>(args, p, part, r->stream);
+  const int nout = swi ? args.n / 2 : args.n, v = nout % 4 == 0 && args.n % 4 == 0 ? 4 : 1;
+  const FastDiv pieces = make_fastdiv((uint32_t)(nout / v));
+  const unsigned blocks = (unsigned)(((int64_t)args.m * (nout / v) + 255) / 256);
+  bt_operand res{};
+#define BT_SUM(DT, EPI)                                                                                             \
+  do {                                                                                                              \
+    if (v == 4) gemm_sum_kernel<DT, EPI, 4><<<blocks, 256, 0, r->stream>>>(args, p.splits, pieces, part, res);      \
+    else gemm_sum_kernel<DT, EPI, 1><<<blocks, 256, 0, r->stream>>>(args, p.splits, pieces, part, res);             \
+  } while (0)
+  if (swi) BT_SUM(BT_BF16, 2);
+  else if (residual_program(args, &res) && res.ptr) BT_SUM(BT_FP32, 1);
+  else if (args.n_inst == 0 && args.out.dtype != BT_INT32 && (args.out.dtype == BT_FP32) == (args.prog.dtype == BT_FP32)) BT_SUM(BT_FP32, 0);
+  else if (args.prog.dtype == BT_FP32) BT_SUM(BT_FP32, 3);
+  else BT_SUM(BT_BF16, 3);
+#undef BT_SUM
+  return true;
+}
+
 // gemm3's block shape: 256 x 256, 256 x 192 or 128 x 256 (and 128 x 384 on bfp4 B), whichever fills the CUs' rounds
 // best, a full round of the smaller blocks counted at 0.9, 0.85 and 0.95 of the speed of one of 256 x 256.
 struct Gemm3Shape { int bm, bn; };
@@ -2617,10 +2819,11 @@ static void launch_gemm_dt(const MatmulArgs &args, hipStream_t s) {
     const double sc = opts[o].eff * (double)blocks / (double)(rounds * 256);
     if (sc > score + 1e-9) score = sc, best = o;
   }
-  if constexpr (FMT == BT_BF16 || FMT == BT_BFP4) {
+  {
     bt_operand res{};
-    const bool fits = FMT == BT_BF16 ? args.m > 128 && args.k % 32 == 0
-                                     : args.m >= 512 && args.k % 64 == 0 && (int64_t)args.chunks * args.nruns * 576 < (1ll << 32);
+    const bool fits = args.m > 128 && (FMT == BT_BF16 ? args.k % 32 == 0
+                                                      : (args.m >= 512 || (int64_t)((args.m + 127) / 128) * ((args.n + 255) / 256) >= 64) &&
+                                                          args.k % 64 == 0 && (int64_t)args.chunks * args.nruns * Tile<FMT>::bytes < (1ll << 32));
     if (fits && (DT == BT_BF16 || residual_program(args, &res))) {
       const Gemm3Shape sh = gemm3_shape(args, FMT == BT_BFP4);
       const int mb = (args.m + sh.bm - 1) / sh.bm, nb = (args.n + sh.bn - 1) / sh.bn;
@@ -2720,11 +2923,16 @@ extern "C" int bt_matmul(bt_runtime *rt, const bt_operand *a, int b_fmt, uint64_
   }
   args.n_inst = args.prog.n_inst;
   args.out = *out;
-  // A prefill-sized product with bfp8 B (or bfp4 with K not in whole chunks) and bf16 out: B unpacked once into bf16
-  // tiles in the runtime's scratch (the same values bit for bit), then the bf16 GEMM. bfp4 B in whole chunks goes to
-  // the same GEMM reading it as it is stored, decoded in registers.
+  if (launch_gemm_split(r, args, b_fmt, false)) {
+    BT_LAUNCHED("matmul");
+    return BT_OK;
+  }
+  // A prefill-sized product whose block-float B the GEMM doesn't read as stored (K not in whole chunks), or reads more
+  // slowly than bf16 (bfp8 over many 128-row blocks, each decoding B again: 2048 x 4096 x 4096 88 us, 85 unpacked first,
+  // while 256-row blocks gain, 481 us against 534 at 28672 columns): B unpacked once into bf16 tiles in the runtime's
+  // scratch (the same values bit for bit), then the bf16 GEMM.
   const bool bf16_out = out->dtype == BT_BF16 && (!epilogue || epilogue->dtype != BT_FP32);
-  if (b_fmt != BT_BF16 && !(b_fmt == BT_BFP4 && k % 64 == 0) &&
+  if (b_fmt != BT_BF16 && (k % 64 != 0 || (b_fmt == BT_BFP8 && m >= 1024 && gemm3_shape(args, false).bm == 128)) &&
       (bf16_out || residual_program(args, nullptr)) &&
       m >= 512 && k % 32 == 0 && a->sc == 1 && (int64_t)args.chunks * args.nruns * 2048 < (1ll << 32)) {
     const int64_t tiles = (int64_t)args.chunks * args.nruns * (b_batch > 1 ? b_batch : 1);
@@ -2882,6 +3090,10 @@ extern "C" int bt_matmul_swiglu(bt_runtime *rt, const bt_operand *a, int b_fmt, 
   if ((int64_t)args.chunks * args.nruns * 2048 >= (1ll << 32)) return fail(BT_EINVAL, "matmul_swiglu's B is too large");
   const int mb = (int)((m + 255) / 256), nb = (int)((n / 2 + 127) / 128);
   const int64_t gemm_blocks = ((m + 127) / 128) * ((n + 127) / 128);
+  if (launch_gemm_split(r, args, b_fmt, true)) {
+    BT_LAUNCHED("matmul_swiglu");
+    return BT_OK;
+  }
   if ((m <= 64 || (m <= 256 && gemm_blocks < 128)) && a->sr % 8 == 0 && a->ptr % 16 == 0 && ((31 * a->sr + 2 * k + 1024) * 2 < (1ll << 32))) {
     if (launch_stream(r, args, b_fmt, true) || launch_parts(r, args, b_fmt, true)) {
       BT_LAUNCHED("matmul_swiglu");
@@ -2902,10 +3114,9 @@ extern "C" int bt_matmul_swiglu(bt_runtime *rt, const bt_operand *a, int b_fmt, 
     BT_LAUNCHED("matmul_swiglu");
     return BT_OK;
   }
-  // bfp4 B with K in whole chunks: read as it is stored by the GEMM itself; other block floats unpacked once into bf16
+  // block-float B with K in whole chunks: read as it is stored by the GEMM itself; otherwise unpacked once into bf16
   // tiles in the runtime's scratch
-  const bool q4 = b_fmt == BT_BFP4 && k % 64 == 0;
-  if (b_fmt != BT_BF16 && !q4) {
+  if (b_fmt != BT_BF16 && k % 64 != 0) {
     const int64_t tiles = (int64_t)args.chunks * args.nruns;
     void *bt16 = runtime_scratch(r, (size_t)tiles * 2048);
     if (!bt16) return fail(BT_ESTATE, "matmul_swiglu: no scratch for B's bf16 tiles (inside a capture, or out of memory)");
@@ -2914,30 +3125,29 @@ extern "C" int bt_matmul_swiglu(bt_runtime *rt, const bt_operand *a, int b_fmt, 
     else tiles_bf16_kernel<BT_BFP4><<<blocks, 256, 0, r->stream>>>(args.b, (uint8_t *)bt16, tiles);
     BT_LAUNCHED("matmul_swiglu");
     args.b = (const uint8_t *)bt16;
+    b_fmt = BT_BF16;
   }
   // One block a CU (the stages fill its LDS), so the blocks run in rounds of 256. When the last round would be at most
   // half full, the trailing block columns go to a second launch of 128-row blocks: twice the blocks at half the work
   // each, which fill one round that takes half the time (gate_up of 2048 Llama-3-8B tokens: 896 blocks, 3.5 rounds,
   // become 768 + 256 blocks of 128 rows, 3 rounds and a half-length one).
+  const int mb128 = (int)((m + 127) / 128);
   int tail = 0;
   if (mb * nb > 256 && (mb * nb) % 256 != 0 && (mb * nb) % 256 <= 128) {
-    const int mb128 = (int)((m + 127) / 128);
     for (int t = 1; t < nb && mb128 * t <= 256; t++)
       if ((mb * (nb - t)) % 256 == 0) { tail = t; break; }
   }
-  const unsigned blocks = (unsigned)((int64_t)mb * (nb - tail));
-  if (q4) gemm3_kernel<BT_BFP4, BT_BF16, 4, GEMM_SWIGLU><<<blocks, 512, 0, r->stream>>>(args, mb, nb - tail, bt_operand{}, 0);
-  else gemm3_kernel<BT_BF16, BT_BF16, 4, GEMM_SWIGLU><<<blocks, 512, 0, r->stream>>>(args, mb, nb - tail, bt_operand{}, 0);
+  // 128-row blocks throughout where their rounds (half as long) take less than the 256-row ones'
+  if (!tail && (mb128 * nb + 255) / 256 * 1.06 < 2 * ((mb * nb + 255) / 256)) tail = nb;
+  auto launch = [&](auto fmt) {
+    constexpr int FMT = decltype(fmt)::value;
+    if (tail < nb) gemm3_kernel<FMT, BT_BF16, 4, GEMM_SWIGLU><<<(unsigned)((int64_t)mb * (nb - tail)), 512, 0, r->stream>>>(args, mb, nb - tail, bt_operand{}, 0);
+    if (tail) gemm3_kernel<FMT, BT_BF16, 4, GEMM_SWIGLU, 128><<<(unsigned)((int64_t)mb128 * tail), 512, 0, r->stream>>>(args, mb128, tail, bt_operand{}, nb - tail);
+  };
+  if (b_fmt == BT_BF16) launch(std::integral_constant<int, BT_BF16>{});
+  else if (b_fmt == BT_BFP8) launch(std::integral_constant<int, BT_BFP8>{});
+  else launch(std::integral_constant<int, BT_BFP4>{});
   BT_LAUNCHED("matmul_swiglu");
-  if (tail) {
-    const int mb128 = (int)((m + 127) / 128);
-    const unsigned tb = (unsigned)((int64_t)mb128 * tail);
-    if (q4)
-      gemm3_kernel<BT_BFP4, BT_BF16, 4, GEMM_SWIGLU, 128><<<tb, 512, 0, r->stream>>>(args, mb128, tail, bt_operand{}, nb - tail);
-    else
-      gemm3_kernel<BT_BF16, BT_BF16, 4, GEMM_SWIGLU, 128><<<tb, 512, 0, r->stream>>>(args, mb128, tail, bt_operand{}, nb - tail);
-    BT_LAUNCHED("matmul_swiglu");
-  }
   return BT_OK;
 }
 

@@ -333,6 +333,44 @@ def test_split_k_rows(rt, fmt, m, k, n, out):
 # rows; 1000 and 520 leave partial blocks, chunks of K and runs of N. bfp4 B with K in whole chunks (256, 192, 640)
 # is read by the GEMM as it is stored from 512 rows up. 2048 x 6144 takes blocks of 256 x 192 (256 of them, one round
 # of the CUs, where 256 x 256 would leave a quarter idle).
+# a prompt's chunk against a long K: the tiled GEMM's blocks split K between them. Rows either side of the plan's limits
+# and of a block's 128, columns off its 256, K of as few chunks a split as it takes; the formats still sum K alike, so a
+# block float is bit for bit the bf16 product of its values
+@pytest.mark.parametrize("m,k,n", [(33, 4096, 4096), (65, 4096, 1536), (127, 2048, 3000), (129, 1280, 576), (257, 1024, 1001),
+                                   (300, 1088, 500), (520, 4160, 260), (1000, 1024, 130)])
+def test_split_gemm_rows(rt, m, k, n):
+  rng = np.random.default_rng(m)
+  x, w = B.bf16(rng.normal(0, 1, (m, k))), rng.normal(0, 0.05, (k, n)).astype(np.float32)
+  res = rng.normal(0, 1, (m, n)).astype(np.float32)
+  dres = up(rt, res)
+  for fmt in ("bf16", "bfp8", "bfp4"):
+    if fmt == "bf16": cols, wq = bf16_columns(rt, w), B.bf16(w)
+    else:
+      exps, vals = pack(rt, w, fmt)
+      cols, wq = columns(rt, exps, vals, fmt, 1, k, n), bfp_values(w, fmt)
+    want, size = ops.matmul(x, wq), np.abs(x.astype(np.float64)) @ np.abs(wq.astype(np.float64))
+    plain = matmul(rt, x, cols, fmt, 1, n)[0]
+    assert np.all(np.abs(plain - want) <= 2.0 ** -8 * size)
+    same = bf16_columns(rt, wq)
+    assert np.array_equal(plain, matmul(rt, x, same, "bf16", 1, n)[0]), fmt
+    p = Program("bf16", epilogue=True)
+    relu2 = matmul(rt, x, cols, fmt, 1, n, prog=p.build(p.op("mul", p.op("relu", p.value()), p.const(2.0))))[0]
+    assert np.array_equal(relu2, 2 * np.maximum(plain, 0)), fmt
+    p = Program("fp32", epilogue=True)
+    prog = p.build(p.op("add", p.value(), p.load(p.input(_lib.operand(dres, "fp32", m * n, n, 1)))))
+    full = matmul(rt, x, cols, fmt, 1, n, out="fp32")[0]
+    assert np.all(np.abs(full - want) <= k * 2.0 ** -24 * size)  # k fp32 additions at most
+    assert np.array_equal(matmul(rt, x, cols, fmt, 1, n, out="fp32", prog=prog)[0], full + res), fmt
+    if n % 32: continue
+    got = rt.dram_alloc(m * n)
+    rt.run("swiglu", "matmul_swiglu", ctypes.byref(_lib.operand(up(rt, B.bf16_bits(x)), "bf16", m * k, k, 1)), _lib.DTYPES[fmt],
+           cols, m, k, n, ctypes.byref(_lib.operand(got, "bf16", m * n // 2, n // 2, 1)))
+    g, u = plain[:, :n // 2].astype(np.float64), plain[:, n // 2:].astype(np.float64)
+    silu = g / (1 + np.exp(-g)) * u
+    out = bits_to_float(down(rt, got, (m, n // 2), np.uint16))
+    assert np.all(np.abs(out - silu) <= 2.0 ** -7 * np.abs(silu) + 1e-30), fmt  # one bf16 rounding, and fp32's in silu
+
+
 GEMM_CASES = [(300, 1000, 520, "bf16"), (96, 576, 1536, "fp32"), (2048, 256, 8192, "bf16"), (2048, 192, 4096, "fp32"),
               (160, 320, 8192, "bf16"), (1000, 224, 4096, "bf16"), (520, 640, 1296, "fp32"), (2048, 320, 6144, "bf16"),
               (2048, 192, 6144, "fp32"), (2048, 128, 8192, "fp32")]
