@@ -176,27 +176,32 @@ __device__ __forceinline__ float sum_groups(float x) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+// How a key head's query pairs fall into tiles of 16. Packed: pair p = r * rep + h is member p % 16 of tile p / 16. By
+// row (per > 0): each query row has `per` tiles of its own, its heads 16 at a time, for rows that see different regions
+// of one cache (bt_attention's firsts): a packed tile would fold every key from its first row's region to its last's
+// (8 slots of 512 rows: the step of a 30-layer model with 3 heads of 64 a key head 1450 -> 1350 us with the combine below).
+struct Tiles {
+  int n, per;
+  FastDiv rep, dper;  // division by the heads of a key head, and by `per`
+};
+// Member i of tile t as a pair; rep * rows, which is none, past the tile's pairs.
+__device__ __forceinline__ int tile_pair(const bt_attention_args &a, const Tiles &tl, int t, int i) {
+  if (tl.per == 0) return min(16 * t + i, a.rep * a.rows);
+  const int r = (int)fdiv((uint32_t)t, tl.dper), h = 16 * (t - r * tl.per) + i;
+  return h < a.rep ? r * a.rep + h : a.rep * a.rows;
+}
+// How many pairs tile t holds.
+__device__ __forceinline__ int tile_pairs(const bt_attention_args &a, const Tiles &tl, int t) {
+  if (tl.per == 0) return min(16, a.rep * a.rows - 16 * t);
+  return min(16, a.rep - 16 * (t - (int)fdiv((uint32_t)t, tl.dper) * tl.per));
+}
+
 // A lane's pair: which query row it is, which keys it sees, where its q and output rows are.
 struct Pair {
   int lo, hi;  // visible keys lo..hi (empty when lo > hi)
   int64_t q, o;  // element offsets of the pair's q and output rows
   bool valid;
 };
-
-__device__ __forceinline__ Pair pair_of(const bt_attention_args &a, int kvh, int p) {
-  Pair x;
-  const int np = a.rep * a.rows;
-  x.valid = p < np;
-  const int pp = x.valid ? p : 0, h = pp % a.rep, r = pp / a.rep, e = kvh * a.rep + h;
-  const int place = ((const int32_t *)a.places)[(int64_t)e * a.places_sh + r];
-  x.lo = a.window > 0 ? max(0, place - a.window + 1) : 0;
-  if (a.firsts) x.lo = max(x.lo, ((const int32_t *)a.firsts)[(int64_t)e * a.firsts_sh + r]);
-  x.hi = min(place, a.keys - 1);
-  if (!x.valid) x.lo = 1, x.hi = 0;
-  x.q = (int64_t)e * a.q_sh + (int64_t)r * a.q_sr;
-  x.o = (int64_t)e * a.o_sh + (int64_t)r * a.o_sr;
-  return x;
-}
 
 // The running state of one wave's tile: maximum and sum of packed p per pair (every lane holds its pair l%16's), and
 // the unnormalized output O in the matrix-core layout (lane l: pairs 4(l/16)+i, column 16c + l%16).
@@ -277,16 +282,17 @@ __device__ __forceinline__ void fold_scores(State<HD> &st, f32x4 (&s)[4], const 
   }
 }
 
-// pair_of with the Q^T operand fragments of the lane's pair (dims 32kk + 8(l/16) .. +8, zeros for a pair past the
+// Pair p with the Q^T operand fragments of the lane's pair (dims 32kk + 8(l/16) .. +8, zeros for a pair past the
 // last), every load issued before any is used: the place, the first key, the q row, as global loads from addresses
 // that are always valid (a pair past the last reads pair 0's and is then marked empty, a call without firsts reads the
 // place twice). So a kernel's prologue is one trip to memory rather than a chain of three.
 template <int HD>
-__device__ __forceinline__ Pair pair_q(const bt_attention_args &a, int kvh, int p, int lane, bf16x8 (&qf)[HD / 32]) {
+__device__ __forceinline__ Pair pair_q(const bt_attention_args &a, const FastDiv &rep, int kvh, int p, int lane,
+                                       bf16x8 (&qf)[HD / 32]) {
   Pair x;
   const int np = a.rep * a.rows;
   x.valid = p < np;
-  const int pp = x.valid ? p : 0, h = pp % a.rep, r = pp / a.rep, e = kvh * a.rep + h;
+  const int pp = x.valid ? p : 0, r = (int)fdiv((uint32_t)pp, rep), h = pp - r * a.rep, e = kvh * a.rep + h;
   x.q = (int64_t)e * a.q_sh + (int64_t)r * a.q_sr;
   x.o = (int64_t)e * a.o_sh + (int64_t)r * a.o_sr;
   const int32_t *pl = (const int32_t *)a.places + (int64_t)e * a.places_sh + r;
@@ -331,53 +337,62 @@ __device__ __forceinline__ void tile_range(const Pair &pr, int &lo, int &hi) {
 // Floats of one tile's partial result: m[16], l[16], then O[16][HD].
 template <int HD> constexpr int partial_floats() { return 32 + 16 * HD; }
 
+constexpr int NW = 4;  // waves of a decode block
+
+// Where pair p's output row starts.
+__device__ __forceinline__ int64_t pair_out(const bt_attention_args &a, const FastDiv &rep, int kvh, int p) {
+  const int r = (int)fdiv((uint32_t)p, rep), h = p - r * a.rep, e = kvh * a.rep + h;
+  return (int64_t)e * a.o_sh + (int64_t)r * a.o_sr;
+}
+
 // Writes the block's combined result for its tile: the bf16 output of each valid pair (parts == 1), or the partial
-// result into scratch. parts: the wave states in LDS `ws` (4 waves, partial_floats each).
+// result into scratch. ws: the states of the block's NW waves in LDS (partial_floats each).
 template <int HD>
-__device__ __forceinline__ void finish_tile(const bt_attention_args &a, const float *ws, int nwaves, int kvh, int t,
-                                            int part, int parts, int tiles, float *scratch) {
-  constexpr int PF = partial_floats<HD>();
-  const int tid = threadIdx.x;
-  // each thread: one pair and HD / 16 columns
-  const int pr_i = tid / 16, c0 = tid % 16;
-  float M = -__builtin_inff();
-  for (int w = 0; w < nwaves; w++) M = fmaxf(M, ws[w * PF + pr_i]);
-  float wgt[4], L = 0.0f;
-  for (int w = 0; w < nwaves; w++) {
-    wgt[w] = M == -__builtin_inff() ? 0.0f : __expf(ws[w * PF + pr_i] - M);
+__device__ __forceinline__ void finish_tile(const bt_attention_args &a, const float *ws, int kvh, int t, int part,
+                                            int parts, const Tiles &tiles, float *scratch) {
+  constexpr int PF = partial_floats<HD>(), TPP = 4 * NW, C = HD / TPP;  // threads a pair, columns a thread
+  const int pr_i = threadIdx.x / TPP, c0 = threadIdx.x % TPP, p = tile_pair(a, tiles, t, pr_i);
+  if (p >= a.rep * a.rows) return;
+  float wgt[NW], M = -__builtin_inff(), L = 0.0f;
+#pragma unroll
+  for (int w = 0; w < NW; w++) M = fmaxf(M, wgt[w] = ws[w * PF + pr_i]);
+#pragma unroll
+  for (int w = 0; w < NW; w++) {
+    wgt[w] = M == -__builtin_inff() ? 0.0f : __expf(wgt[w] - M);
     L += wgt[w] * ws[w * PF + 16 + pr_i];
   }
-  float o[HD / 16];
+  float o[C];
 #pragma unroll
-  for (int c = 0; c < HD / 16; c++) {
+  for (int c = 0; c < C; c++) {
     float v = 0.0f;
-    for (int w = 0; w < nwaves; w++) v += wgt[w] * ws[w * PF + 32 + pr_i * HD + c0 + 16 * c];
+#pragma unroll
+    for (int w = 0; w < NW; w++) v += wgt[w] * ws[w * PF + 32 + pr_i * HD + c0 + TPP * c];
     o[c] = v;
   }
   if (parts == 1) {
-    const Pair pr = pair_of(a, kvh, 16 * t + pr_i);
-    if (!pr.valid) return;
     const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-    uint16_t *out = (uint16_t *)a.out + pr.o;
+    uint16_t *out = (uint16_t *)a.out + pair_out(a, tiles.rep, kvh, p);
 #pragma unroll
-    for (int c = 0; c < HD / 16; c++) out[c0 + 16 * c] = (uint16_t)bf16_packed(o[c] * inv);
+    for (int c = 0; c < C; c++) out[c0 + TPP * c] = (uint16_t)bf16_packed(o[c] * inv);
   } else {
-    float *dst = scratch + ((int64_t)(kvh * tiles + t) * parts + part) * PF;
+    float *dst = scratch + ((int64_t)(kvh * tiles.n + t) * parts + part) * PF;
     if (c0 == 0) dst[pr_i] = M, dst[16 + pr_i] = L;
 #pragma unroll
-    for (int c = 0; c < HD / 16; c++) dst[32 + pr_i * HD + c0 + 16 * c] = o[c];
+    for (int c = 0; c < C; c++) dst[32 + pr_i * HD + c0 + TPP * c] = o[c];
   }
 }
 
-// Writes a wave's state into its LDS partial: m and l by lanes 0..15, O from the matrix-core layout.
+// Writes a wave's state as a partial: m and l by lanes 0..15, O from the matrix-core layout, the tile's first `pairs`
+// pairs only.
 template <int HD>
-__device__ __forceinline__ void store_state(float *ws, const State<HD> &st, int lane) {
+__device__ __forceinline__ void store_state(float *ws, const State<HD> &st, int lane, int pairs) {
   const int g = lane >> 4, n = lane & 15;
-  if (lane < 16) ws[n] = st.m, ws[16 + n] = st.l;
+  if (lane < min(pairs, 16)) ws[n] = st.m, ws[16 + n] = st.l;
 #pragma unroll
-  for (int c = 0; c < HD / 16; c++)
+  for (int i = 0; i < 4; i++)
+    if (4 * g + i < pairs)
 #pragma unroll
-    for (int i = 0; i < 4; i++) ws[32 + (4 * g + i) * HD + 16 * c + n] = st.o[c][i];
+      for (int c = 0; c < HD / 16; c++) ws[32 + (4 * g + i) * HD + 16 * c + n] = st.o[c][i];
 }
 
 // Decode: block (kvh, t, part). The tile's visible keys, from its smallest first to its largest last, are cut into
@@ -428,22 +443,22 @@ __device__ __forceinline__ void decode_keys(bf16x8 (&kf)[4][HD / 32], const KeyB
 }
 
 template <int HD, int KF, bool WIDE>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-attention_decode_kernel(const bt_attention_args a, int tiles, int parts, float *scratch) {
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+attention_decode_kernel(const bt_attention_args a, const Tiles tiles, int parts, float *scratch) {
   // halfwords of one wave's value block: rows of HD + 16, so that the 8 rows a transposing read's pass of 32 lanes
   // addresses (8 dwords each) start 8 banks apart
   constexpr int VS = HD + 16, VR = KB * VS;
   constexpr int PF = partial_floats<HD>();
-  static_assert(4 * PF * 4 <= 4 * VR * 2, "the wave partials fit in the value blocks' LDS");
-  __shared__ __attribute__((aligned(16))) uint16_t lds[4 * VR];
+  static_assert(PF * 4 <= VR * 2, "the wave partials fit in the value blocks' LDS");
+  __shared__ __attribute__((aligned(16))) uint16_t lds[NW * VR];
   const int lane = threadIdx.x & 63, n = lane & 15;
   const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   int bid = blockIdx.x;
   const int part = bid % parts;
   bid /= parts;
-  const int t = bid % tiles, kvh = bid / tiles;
+  const int t = bid % tiles.n, kvh = bid / tiles.n;
   bf16x8 qf[HD / 32];
-  const Pair pr = pair_q<HD>(a, kvh, 16 * t + n, lane, qf);
+  const Pair pr = pair_q<HD>(a, tiles.rep, kvh, tile_pair(a, tiles, t, n), lane, qf);
   int lo, hi;
   tile_range(pr, lo, hi);
   const int start = lo & ~(KB - 1), nblk = hi >= lo ? (hi - start) / KB + 1 : 0, per = (nblk + parts - 1) / parts;
@@ -482,7 +497,7 @@ attention_decode_kernel(const bt_attention_args a, int tiles, int parts, float *
     wave_lds_sync();  // the previous block's reads of vl are done
 #pragma unroll
     for (int i = 0; i < VI; i++) *(uint4 *)(vl + (vrow + RPI * i) * VS + vcol) = kv_value8<KF>(vq[i], vx[i]);
-    if constexpr (MORE) fetch_values(kb + 4 * KB);
+    if constexpr (MORE) fetch_values(kb + NW * KB);
     wave_lds_sync();
     f32x4 s[4];
     {
@@ -490,34 +505,34 @@ attention_decode_kernel(const bt_attention_args a, int tiles, int parts, float *
       decode_keys<HD, KF, WIDE>(kf, kbytes, lane);
       block_scores<HD>(s, kf, qf);
     }
-    if constexpr (MORE) fetch_keys<HD, KF, WIDE>(kbytes, kr, kb + 4 * KB, a.k_sr, lane);
+    if constexpr (MORE) fetch_keys<HD, KF, WIDE>(kbytes, kr, kb + NW * KB, a.k_sr, lane);
     fold_scores<HD, VS>(st, s, vl, kb, pr, lane, fresh);
     fresh = false;
   };
-  for (; kb + 4 * KB <= last; kb += 4 * KB) step(kb, std::true_type{});
+  for (; kb + NW * KB <= last; kb += NW * KB) step(kb, std::true_type{});
   if (kb <= last) step(kb, std::false_type{});
   __syncthreads();
   float *ws = (float *)lds;
-  store_state<HD>(ws + wib * PF, st, lane);
+  store_state<HD>(ws + wib * PF, st, lane, tile_pairs(a, tiles, t));
   __syncthreads();
-  finish_tile<HD>(a, ws, 4, kvh, t, part, parts, tiles, scratch);
+  finish_tile<HD>(a, ws, kvh, t, part, parts, tiles, scratch);
 }
 
 // Decode in parts of one 64-key block each, a block of one wave: the wave folds its block and writes its state as the
 // part's partial result, from its registers, with no join through LDS (which a 4-wave block of one or two blocks of
 // keys spends most of its time on). The combine kernel joins the parts.
 template <int HD, int KF, bool WIDE>
-__global__ void __launch_bounds__(64) attention_decode1_kernel(const bt_attention_args a, int tiles, int parts,
+__global__ void __launch_bounds__(64) attention_decode1_kernel(const bt_attention_args a, const Tiles tiles, int parts,
                                                                float *scratch) {
   constexpr int VS = HD + 16, VR = KB * VS, PF = partial_floats<HD>();
   __shared__ __attribute__((aligned(16))) uint16_t vl[VR];
-  const int lane = threadIdx.x, g = lane >> 4, n = lane & 15;
+  const int lane = threadIdx.x, n = lane & 15;
   int bid = blockIdx.x;
   const int part = bid % parts;
   bid /= parts;
-  const int t = bid % tiles, kvh = bid / tiles;
+  const int t = bid % tiles.n, kvh = bid / tiles.n;
   bf16x8 qf[HD / 32];
-  const Pair pr = pair_q<HD>(a, kvh, 16 * t + n, lane, qf);
+  const Pair pr = pair_q<HD>(a, tiles.rep, kvh, tile_pair(a, tiles, t, n), lane, qf);
   int lo, hi;
   tile_range(pr, lo, hi);
   const int start = lo & ~(KB - 1), nblk = hi >= lo ? (hi - start) / KB + 1 : 0, per = (nblk + parts - 1) / parts;
@@ -555,67 +570,49 @@ __global__ void __launch_bounds__(64) attention_decode1_kernel(const bt_attentio
     fold_scores<HD, VS>(st, sc, vl, kb, pr, lane, fresh);
     fresh = false;
   }
-  float *dst = scratch + ((int64_t)(kvh * tiles + t) * parts + part) * PF;
-  if (lane < 16) dst[n] = st.m, dst[16 + n] = st.l;
-#pragma unroll
-  for (int c = 0; c < HD / 16; c++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) dst[32 + (4 * g + i) * HD + 16 * c + n] = st.o[c][i];
+  store_state<HD>(scratch + ((int64_t)(kvh * tiles.n + t) * parts + part) * PF, st, lane, tile_pairs(a, tiles, t));
 }
 
-// Joins the parts of each tile: M = max m_p, L = sum e^(m_p - M) l_p, out = sum e^(m_p - M) O_p / L. The block
-// first finds every pair's M, weights and L with its 16 groups of 16 threads splitting the parts (weights kept in
-// LDS), then each thread sums its output columns over the parts, loads independent of one another.
+// Joins the parts of each tile: M = max m_p, L = sum e^(m_p - M) l_p, out = sum e^(m_p - M) O_p / L. A thread a column
+// of a valid pair, with 16 parts' maxima, sums and outputs loaded at once, so that the usual plan is one trip to memory
+// and no barrier; more parts go in turns of 16, the running sums rescaled as a turn's maximum passes theirs. (A block a
+// tile that first found every pair's weights through LDS made three trips and four barriers: B=1, 8 x 128, 512 keys
+// 7.15 -> 6.42 us a call, 4096 12.2 -> 10.6, 16384 20.8 -> 18.1.)
 constexpr int MAX_PARTS = 256;
 template <int HD>
-__global__ void __launch_bounds__(256) attention_combine_kernel(const bt_attention_args a, int tiles, int parts,
-                                                                const float *scratch) {
-  constexpr int PF = partial_floats<HD>();
-  __shared__ float wgt[MAX_PARTS * 16];  // [part][pair]
-  __shared__ float red[16][16], mx[16], ls[16];
-  const int t = blockIdx.x % tiles, kvh = blockIdx.x / tiles;
-  const float *src = scratch + (int64_t)(kvh * tiles + t) * parts * PF;
-  const int pr = threadIdx.x & 15, grp = threadIdx.x >> 4;
-  float M = -__builtin_inff();
-  for (int p = grp; p < parts; p += 16) M = fmaxf(M, src[p * PF + pr]);
-  red[grp][pr] = M;
-  __syncthreads();
-  if (grp == 0) {
-    for (int g = 1; g < 16; g++) M = fmaxf(M, red[g][pr]);
-    mx[pr] = M;
-  }
-  __syncthreads();
-  M = mx[pr];
-  float L = 0.0f;
-  for (int p = grp; p < parts; p += 16) {
-    const float w = M == -__builtin_inff() ? 0.0f : __expf(src[p * PF + pr] - M);
-    wgt[p * 16 + pr] = w;
-    L += w * src[p * PF + 16 + pr];
-  }
-  red[grp][pr] = L;
-  __syncthreads();
-  if (grp == 0) {
-    for (int g = 1; g < 16; g++) L += red[g][pr];
-    ls[pr] = L;
-  }
-  __syncthreads();
-  const int pi = threadIdx.x / 16, c0 = threadIdx.x % 16;
-  const Pair pair = pair_of(a, kvh, 16 * t + pi);
-  if (!pair.valid) return;
-  float o[HD / 16];
+__global__ void __launch_bounds__(256) attention_combine_kernel(const bt_attention_args a, const Tiles tiles, int parts,
+                                                                int per_tile, const float *scratch) {
+  constexpr int PF = partial_floats<HD>(), TURN = 16;
+  const int unit = blockIdx.x / per_tile, e = (blockIdx.x % per_tile) * 256 + threadIdx.x;
+  const int t = unit % tiles.n, kvh = unit / tiles.n, pi = e / HD, col = e % HD;
+  const int p = pi < 16 ? tile_pair(a, tiles, t, pi) : a.rep * a.rows;
+  if (p >= a.rep * a.rows) return;
+  const float *src = scratch + (int64_t)unit * parts * PF;
+  float M = -__builtin_inff(), L = 0.0f, O = 0.0f;
+  for (int p0 = 0; p0 < parts; p0 += TURN) {
+    float m[TURN], l[TURN], o[TURN];
 #pragma unroll
-  for (int c = 0; c < HD / 16; c++) o[c] = 0.0f;
-  const float *col = src + 32 + pi * HD + c0;
-#pragma unroll 4
-  for (int p = 0; p < parts; p++) {
-    const float w = wgt[p * 16 + pi];
+    for (int j = 0; j < TURN; j++) {
+      const float *q = src + (int64_t)min(p0 + j, parts - 1) * PF;  // a part past the last is read and left out
+      m[j] = gload(q + pi), l[j] = gload(q + 16 + pi), o[j] = gload(q + 32 + pi * HD + col);
+    }
+    float top = M;
 #pragma unroll
-    for (int c = 0; c < HD / 16; c++) o[c] += w * col[p * PF + 16 * c];
+    for (int j = 0; j < TURN; j++) {
+      if (p0 + j >= parts) m[j] = -__builtin_inff();
+      top = fmaxf(top, m[j]);
+    }
+    const float keep = M == top ? 1.0f : __expf(M - top);
+    L *= keep, O *= keep;
+#pragma unroll
+    for (int j = 0; j < TURN; j++) {
+      const float w = m[j] == -__builtin_inff() ? 0.0f : __expf(m[j] - top);
+      L += w * l[j], O += w * o[j];
+    }
+    M = top;
   }
-  const float inv = ls[pi] > 0.0f ? 1.0f / ls[pi] : 0.0f;
-  uint16_t *out = (uint16_t *)a.out + pair.o;
-#pragma unroll
-  for (int c = 0; c < HD / 16; c++) out[c0 + 16 * c] = (uint16_t)bf16_packed(o[c] * inv);
+  const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+  ((uint16_t *)a.out)[pair_out(a, tiles.rep, kvh, p) + col] = (uint16_t)bf16_packed(O * inv);
 }
 
 // Prefill. A block is 4 waves and 128 consecutive pairs of one key head; wave w takes pairs 32w .. 32w + 31 of them as
@@ -802,7 +799,7 @@ __device__ __forceinline__ void fold_pairs(Group<HD> (&gr)[2], const bf16x8 (&qf
 // Blocks go heaviest first (the last rows of the causal triangle see the most keys): block u takes key head u % kvhs
 // and row block rblocks - 1 - u / kvhs.
 template <int HD, int KF>
-__global__ void __launch_bounds__(512, 1) attention_prefill_kernel(const bt_attention_args a, int rblocks, int kvhs) {
+__global__ void __launch_bounds__(512, 1) attention_prefill_kernel(const bt_attention_args a, int rblocks, int kvhs, const FastDiv rep) {
   constexpr int KBUF = KB * HD, STG = 2 * KBUF;  // halfwords of one stage: K, then V, row-major, units swizzled (swz)
   constexpr int KW = KB * HD / 8 / 256;  // 16-byte words of K (and of V) each thread of a half moves per block
   constexpr int XF = 2 * (HD / 4 + 8);   // floats per lane a wave hands over: O, l and the maxima of both groups
@@ -819,7 +816,7 @@ __global__ void __launch_bounds__(512, 1) attention_prefill_kernel(const bt_atte
   int lo[2], hi[2];
 #pragma unroll
   for (int q = 0; q < 2; q++) {
-    pr[q] = pair_q<HD>(a, kvh, base + 16 * q + n, lane, qf[q]);
+    pr[q] = pair_q<HD>(a, rep, kvh, base + 16 * q + n, lane, qf[q]);
     lo[q] = pr[q].lo, hi[q] = pr[q].hi;
   }
   // the wave's range (union over its pairs) and the keys every valid pair sees (intersection)
@@ -967,8 +964,7 @@ __global__ void __launch_bounds__(512, 1) attention_prefill_kernel(const bt_atte
       const float w1 = m1 == M ? 1.0f : __builtin_amdgcn_exp2f(m1 - M);
       const float l = gr[q].l[i] * w0 + x[(HD / 4 + i) * 64] * w1;
       const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-      const int h = p % a.rep, r = p / a.rep, e = kvh * a.rep + h;
-      uint16_t *out = (uint16_t *)a.out + (int64_t)e * a.o_sh + (int64_t)r * a.o_sr;
+      uint16_t *out = (uint16_t *)a.out + pair_out(a, rep, kvh, p);
 #pragma unroll
       for (int c = 0; c < HD / 16; c++)
         out[16 * c + n] = (uint16_t)bf16_packed((gr[q].o[c][i] * w0 + x[(4 * c + i) * 64] * w1) * inv);
@@ -977,23 +973,23 @@ __global__ void __launch_bounds__(512, 1) attention_prefill_kernel(const bt_atte
 }
 
 template <int HD>
-static void launch_decode_hd(const bt_attention_args &a, unsigned blocks, int tiles, int parts, float *scratch,
+static void launch_decode_hd(const bt_attention_args &a, unsigned blocks, const Tiles &tiles, int parts, float *scratch,
                              hipStream_t s) {
   // a key row's exponents in one load when every row's start in the plane is aligned to their HD / 16 bytes
   const bool wide = a.k_sr % HD == 0 && a.k_sh % HD == 0 && a.k_exps % (HD / 16) == 0;
-  if (a.kv_fmt == BT_BFP8 && wide) attention_decode_kernel<HD, BT_BFP8, true><<<blocks, 256, 0, s>>>(a, tiles, parts, scratch);
-  else if (a.kv_fmt == BT_BFP8) attention_decode_kernel<HD, BT_BFP8, false><<<blocks, 256, 0, s>>>(a, tiles, parts, scratch);
-  else if (a.kv_fmt == BT_BFP4 && wide) attention_decode_kernel<HD, BT_BFP4, true><<<blocks, 256, 0, s>>>(a, tiles, parts, scratch);
-  else if (a.kv_fmt == BT_BFP4) attention_decode_kernel<HD, BT_BFP4, false><<<blocks, 256, 0, s>>>(a, tiles, parts, scratch);
-  else attention_decode_kernel<HD, BT_BF16, false><<<blocks, 256, 0, s>>>(a, tiles, parts, scratch);
+  if (a.kv_fmt == BT_BFP8 && wide) attention_decode_kernel<HD, BT_BFP8, true><<<blocks, 64 * NW, 0, s>>>(a, tiles, parts, scratch);
+  else if (a.kv_fmt == BT_BFP8) attention_decode_kernel<HD, BT_BFP8, false><<<blocks, 64 * NW, 0, s>>>(a, tiles, parts, scratch);
+  else if (a.kv_fmt == BT_BFP4 && wide) attention_decode_kernel<HD, BT_BFP4, true><<<blocks, 64 * NW, 0, s>>>(a, tiles, parts, scratch);
+  else if (a.kv_fmt == BT_BFP4) attention_decode_kernel<HD, BT_BFP4, false><<<blocks, 64 * NW, 0, s>>>(a, tiles, parts, scratch);
+  else attention_decode_kernel<HD, BT_BF16, false><<<blocks, 64 * NW, 0, s>>>(a, tiles, parts, scratch);
 }
-static void launch_decode(const bt_attention_args &a, unsigned blocks, int tiles, int parts, float *scratch,
+static void launch_decode(const bt_attention_args &a, unsigned blocks, const Tiles &tiles, int parts, float *scratch,
                           hipStream_t s) {
   if (a.head_dim == 64) launch_decode_hd<64>(a, blocks, tiles, parts, scratch, s);
   else launch_decode_hd<128>(a, blocks, tiles, parts, scratch, s);
 }
 template <int HD>
-static void launch_decode1_hd(const bt_attention_args &a, unsigned blocks, int tiles, int parts, float *scratch,
+static void launch_decode1_hd(const bt_attention_args &a, unsigned blocks, const Tiles &tiles, int parts, float *scratch,
                               hipStream_t s) {
   const bool wide = a.k_sr % HD == 0 && a.k_sh % HD == 0 && a.k_exps % (HD / 16) == 0;
   if (a.kv_fmt == BT_BFP8 && wide) attention_decode1_kernel<HD, BT_BFP8, true><<<blocks, 64, 0, s>>>(a, tiles, parts, scratch);
@@ -1004,9 +1000,9 @@ static void launch_decode1_hd(const bt_attention_args &a, unsigned blocks, int t
 }
 template <int HD>
 static void launch_prefill_hd(const bt_attention_args &a, unsigned blocks, int rblocks, int kvh, hipStream_t s) {
-  if (a.kv_fmt == BT_BFP8) attention_prefill_kernel<HD, BT_BFP8><<<blocks, 512, 0, s>>>(a, rblocks, kvh);
-  else if (a.kv_fmt == BT_BFP4) attention_prefill_kernel<HD, BT_BFP4><<<blocks, 512, 0, s>>>(a, rblocks, kvh);
-  else attention_prefill_kernel<HD, BT_BF16><<<blocks, 512, 0, s>>>(a, rblocks, kvh);
+  if (a.kv_fmt == BT_BFP8) attention_prefill_kernel<HD, BT_BFP8><<<blocks, 512, 0, s>>>(a, rblocks, kvh, make_fastdiv((uint32_t)a.rep));
+  else if (a.kv_fmt == BT_BFP4) attention_prefill_kernel<HD, BT_BFP4><<<blocks, 512, 0, s>>>(a, rblocks, kvh, make_fastdiv((uint32_t)a.rep));
+  else attention_prefill_kernel<HD, BT_BF16><<<blocks, 512, 0, s>>>(a, rblocks, kvh, make_fastdiv((uint32_t)a.rep));
 }
 static void launch_prefill(const bt_attention_args &a, unsigned blocks, int rblocks, int kvh, hipStream_t s) {
   if (a.head_dim == 64) launch_prefill_hd<64>(a, blocks, rblocks, kvh, s);
@@ -1016,7 +1012,8 @@ static void launch_prefill(const bt_attention_args &a, unsigned blocks, int rblo
 struct AttnPlan {
   bool decode;
   bool one;  // decode parts of one block of keys each, a wave a part (attention_decode1_kernel)
-  int tiles, parts, kpp;
+  int parts;
+  Tiles tiles;
   uint64_t scratch_bytes;
 };
 
@@ -1042,29 +1039,37 @@ static int plan_attention(const bt_attention_args *a, AttnPlan *p) {
   if (a->firsts && a->firsts % 4) return fail(BT_EINVAL, "attention's firsts must be int32-aligned");
   if (a->firsts && a->firsts_sh != 0 && a->firsts_sh != a->rows) return fail(BT_EINVAL, "firsts' head stride is 0 or rows");
   const int kvh = a->heads / a->rep, np = a->rep * a->rows;
-  p->tiles = (np + 15) / 16;
-  p->decode = p->tiles <= 4;  // few query rows for each key head: split the keys instead
-  p->parts = 1, p->kpp = 0, p->scratch_bytes = 0, p->one = false;
+  // rows with regions of their own: tiles by row while they are few (a decode step's slots, one token or a few each)
+  const bool by_row = a->firsts && a->rows > 1 && a->rows <= 32;
+  const int per_row = (a->rep + 15) / 16;
+  p->tiles = Tiles{by_row ? a->rows * per_row : (np + 15) / 16, by_row ? per_row : 0, make_fastdiv((uint32_t)a->rep),
+                   make_fastdiv((uint32_t)per_row)};
+  p->decode = by_row || p->tiles.n <= 4;  // few query rows for each key head: split the keys instead
+  p->parts = 1, p->scratch_bytes = 0, p->one = false;
   if (p->decode) {
-    const int nblk = (a->keys + KB - 1) / KB;
+    // by row, the regions share the cache's keys: a row's own, and a block for where it starts
+    const int nblk = by_row ? (a->keys / a->rows + KB - 1) / KB + 1 : (a->keys + KB - 1) / KB;
     int parts = a->parts;
     // bf16: one block a CU (MI355X's 256), each wave's loads a block ahead through all of its share of the keys;
     // block floats: two a CU, so one block's decoding overlaps the other's loads. Measured faster than more,
     // shorter-lived blocks at 1-32 batch entries and 4096-16384 keys. A part's keys are a chain of dependent loads,
     // so up to 32 blocks of 64 keys, parts of two blocks (and the combine's launch) beat longer ones; beyond, four;
     // up to 4 blocks, one part (no combine) is the fastest.
-    // 5 to 16 blocks of keys over at most 512 blocks of the grid: a part a block of keys, a wave a part, joined by the
-    // combine alone (B=1 at 512 keys 7.55 -> 6.79 us, at 1024 7.99 -> 7.70; B=8 at 512 the same, at 1024 slower)
-    const int target = a->kv_fmt == BT_BF16 ? 256 : 512, units = kvh * p->tiles;
+    // 5 to 16 blocks of keys over at most 512 blocks of the grid, or 32 over 256: a part a block of keys, a wave a part,
+    // joined by the combine alone (B=1 at 512 keys 7.55 -> 6.79 us, at 1024 7.99 -> 7.70, at 2048 8.68 -> 8.23; B=8 at
+    // 512 the same, at 1024 slower). Heads of 64, half the bytes a block: up to 6 blocks one part where the tiles are
+    // many (64 tiles at 300 keys 7.18 -> 6.49 us, 3 tiles 6.08 and 6.00).
+    const int target = a->kv_fmt == BT_BF16 ? 256 : 512, units = kvh * p->tiles.n;
     const int per_part = nblk <= 4 ? nblk : nblk <= 32 ? 2 : 4;
     if (parts == 0) {
-      if (nblk > 4 && nblk <= 16 && units * nblk <= 512) parts = nblk;
+      if (a->head_dim == 64 && nblk <= 6 && units * nblk > 256) parts = 1;
+      else if (nblk > 4 && (nblk <= 16 ? units * nblk <= 512 : nblk <= 32 && units * nblk <= 256)) parts = nblk;
       else parts = std::min((target + units / 2) / units, std::max(1, nblk / per_part));
     }
     p->parts = std::max(1, std::min(std::min(parts, nblk), MAX_PARTS));
     p->one = p->parts > 1 && p->parts >= nblk;
     const int pf = 32 + 16 * a->head_dim;
-    if (p->parts > 1) p->scratch_bytes = (uint64_t)kvh * p->tiles * p->parts * pf * 4;
+    if (p->parts > 1) p->scratch_bytes = (uint64_t)kvh * p->tiles.n * p->parts * pf * 4;
   }
   return BT_OK;
 }
@@ -1091,7 +1096,7 @@ void attention_noalloc_init(int device) {
 static int run_attention(Runtime *r, const bt_attention_args *a, const AttnPlan &p, float *scratch) {
   const int kvh = a->heads / a->rep;
   if (p.decode) {
-    const unsigned blocks = (unsigned)(kvh * p.tiles * p.parts);
+    const unsigned blocks = (unsigned)(kvh * p.tiles.n * p.parts);
     if (p.one) {
       if (a->head_dim == 64) launch_decode1_hd<64>(*a, blocks, p.tiles, p.parts, scratch, r->stream);
       else launch_decode1_hd<128>(*a, blocks, p.tiles, p.parts, scratch, r->stream);
@@ -1100,9 +1105,11 @@ static int run_attention(Runtime *r, const bt_attention_args *a, const AttnPlan 
     }
     BT_LAUNCHED("attention");
     if (p.parts > 1) {
-      const unsigned cb = (unsigned)(kvh * p.tiles);
-      if (a->head_dim == 64) attention_combine_kernel<64><<<cb, 256, 0, r->stream>>>(*a, p.tiles, p.parts, scratch);
-      else attention_combine_kernel<128><<<cb, 256, 0, r->stream>>>(*a, p.tiles, p.parts, scratch);
+      const int members = std::min(16, p.tiles.per ? a->rep : a->rep * a->rows);
+      const int per_tile = (members * a->head_dim + 255) / 256;
+      const unsigned cb = (unsigned)(kvh * p.tiles.n * per_tile);
+      if (a->head_dim == 64) attention_combine_kernel<64><<<cb, 256, 0, r->stream>>>(*a, p.tiles, p.parts, per_tile, scratch);
+      else attention_combine_kernel<128><<<cb, 256, 0, r->stream>>>(*a, p.tiles, p.parts, per_tile, scratch);
       BT_LAUNCHED("attention combine");
     }
   } else {

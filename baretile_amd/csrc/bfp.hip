@@ -7,7 +7,7 @@
 //          below it, rounding half up (bfp8) or to nearest with ties up (bfp4), saturating at 127 / 7. A zero keeps no
 //          sign.
 //   decode tensor.py:1093-1104 (_bf16s): normalize the magnitude, exponent (e - shift) mod 256.
-#include "program.h"
+#include "common.h"
 
 namespace bt {
 

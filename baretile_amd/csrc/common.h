@@ -96,6 +96,21 @@ int enter(bt_runtime *rt, Runtime **out);
 
 inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
+// n / d for 32-bit n, with a multiplier and shift the host computed for d (the round-up method of Granlund and
+// Montgomery, "Division by invariant integers using multiplication", 1994): q = (umulhi(n, m) + n) >> s.
+struct FastDiv {
+  uint32_t d, m, s;
+};
+__device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv &f) {
+  return (uint32_t)(((uint64_t)__umulhi(n, f.m) + n) >> f.s);
+}
+inline FastDiv make_fastdiv(uint32_t d) {
+  uint32_t s = 0;
+  while ((1ull << s) < d) s++;
+  const uint64_t m = ((1ull << 32) * ((1ull << s) - d)) / d + 1;
+  return FastDiv{d, (uint32_t)m, s};
+}
+
 // ---- number rules (device) -------------------------------------------------------------------------------------
 
 // fp32 -> bf16 bits, round to nearest even, no NaN special case: the host upload rule and the bfp cast's first step.

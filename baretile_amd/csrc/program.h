@@ -396,21 +396,6 @@ __device__ __forceinline__ void store_segment(const bt_operand &out, int64_t b, 
   }
 }
 
-// n / d for 32-bit n, with a multiplier and shift the host computed for d (the round-up method of Granlund and
-// Montgomery, "Division by invariant integers using multiplication", 1994): q = (umulhi(n, m) + n) >> s.
-struct FastDiv {
-  uint32_t d, m, s;
-};
-__device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv &f) {
-  return (uint32_t)(((uint64_t)__umulhi(n, f.m) + n) >> f.s);
-}
-inline FastDiv make_fastdiv(uint32_t d) {
-  uint32_t s = 0;
-  while ((1ull << s) < d) s++;
-  const uint64_t m = ((1ull << 32) * ((1ull << s) - d)) / d + 1;
-  return FastDiv{d, (uint32_t)m, s};
-}
-
 // Stores a result computed in DT as out's dtype at element offset `at`.
 template <int DT>
 __device__ __forceinline__ void store_value(const bt_operand &out, int64_t at, uint32_t v) {

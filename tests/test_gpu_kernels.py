@@ -757,6 +757,41 @@ def test_attention_firsts_keep_each_slot_in_its_region(rt, slots, rep, part):
     assert np.allclose(got[:, u:u + 1], want, rtol=0.011, atol=0.011), (u, np.abs(got[:, u:u + 1] - want).max())
 
 
+# the combine takes 16 parts a turn: whole turns, one more, one less, parts that see no key (a window), 64 and 128 wide
+@pytest.mark.parametrize("hd,keys,window,parts", [(64, 2560, 0, 15), (128, 2560, 0, 16), (64, 2560, 0, 17), (128, 4000, 0, 33),
+                                                  (64, 2560, 200, 32), (128, 1100, 0, 18), (64, 16384, 0, 256)])
+def test_attention_parts_in_turns(rt, hd, keys, window, parts):
+  rng = np.random.default_rng(parts)
+  q = B.bf16(rng.normal(0, 1, (6, 1, hd)) / np.sqrt(hd))
+  k, v = (B.bf16(rng.normal(0, 1, (2, keys, hd))) for _ in range(2))
+  places = np.full((1, 1), keys - 1)
+  got = attend(rt, q, k, v, places, window, parts)
+  assert np.allclose(got, ops.attention(q, k, v, places[..., None], window, 3), rtol=0.011, atol=0.011)
+
+
+# slots' rows in tiles of their own, up to 32 rows, more than 16 heads a key head in two tiles a row; 33 rows packed
+@pytest.mark.parametrize("slots,rep,part,hd", [(2, 17, 70, 64), (32, 20, 40, 64), (32, 1, 129, 128), (33, 2, 64, 64), (3, 3, 1000, 64)])
+def test_attention_rows_in_tiles_of_their_own(rt, slots, rep, part, hd):
+  rng = np.random.default_rng(slots + rep)
+  E, kvh, keys = 2 * rep, 2, slots * part
+  q = B.bf16(rng.normal(0, 1, (E, slots, hd)) / np.sqrt(hd))
+  k, v = (B.bf16(rng.normal(0, 1, (kvh, keys, hd))) for _ in range(2))
+  firsts = np.broadcast_to(np.arange(slots) * part, (E, slots)).astype(np.int32)
+  places = firsts + rng.integers(0, part, slots, dtype=np.int32)
+  o = rt.dram_alloc(E * slots * hd * 2)
+  args = _lib.AttentionArgs(*(up(rt, B.bf16_bits(t)) for t in (q, k, v)), o, up(rt, places), slots * hd, hd, keys * hd, hd, keys * hd,
+                            hd, slots * hd, hd, slots, E, rep, slots, keys, hd, 0, 0, 0, 0, 0, up(rt, firsts.copy()), slots)
+  need = ctypes.c_uint64()
+  _lib.call("attention_scratch", ctypes.byref(args), ctypes.byref(need))
+  if need.value: args.scratch, args.scratch_bytes = rt.dram_alloc(need.value), need.value
+  rt.run("attention", "attention", ctypes.byref(args))
+  got = bits_to_float(down(rt, o, (E, slots, hd), np.uint16))
+  for r in range(slots):
+    own = slice(r * part, places[0, r] + 1)
+    want = ops.attention(q[:, r:r + 1], k[:, own], v[:, own], np.full((1, 1, 1), keys), 0, rep)
+    assert np.allclose(got[:, r:r + 1], want, rtol=0.011, atol=0.011), r
+
+
 def test_attention_rows_without_keys_are_zero(rt):
   # a place before the first key hides every key: p is zero and so is the output (kernels.py:823-826)
   rng = np.random.default_rng(5)
