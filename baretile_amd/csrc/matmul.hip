@@ -220,6 +220,20 @@ __device__ __forceinline__ void load_b(Chunk &r, const uint8_t *t, int lane) {
 
 constexpr int GROUP_B = 8;  // chunks requested together by the B-side kernel
 
+// Whether a program is one two-operand operation on the product and one input (x + r, the residual add, above all):
+// then op and which operand the product is, so that it runs straight on the tile's values, without the evaluator's
+// register file.
+struct OneInput {
+  int op;      // -1: another kind of program
+  bool a, b;   // whether the operand is the product (else the input)
+};
+__device__ __forceinline__ OneInput one_input(const bt_program &p, int n_inst) {
+  const bt_inst ld = p.inst[0], in = p.inst[1];
+  const bool ok = n_inst == 2 && p.n_inputs == 1 && ld.op == BT_OP_LOAD && ld.dst != 0 && in.op >= BT_OP_ADD &&
+                  in.op <= BT_OP_CMPEQ && p.result == in.dst && (in.a == 0 || in.a == ld.dst) && (in.b == 0 || in.b == ld.dst);
+  return OneInput{ok ? in.op : -1, in.a == 0, in.b == 0};
+}
+
 // The epilogue of both kernels: lane holds rows 4g .. 4g+3 of the 16 x 16 tile at (mt, run), column col.
 // ONE: a batch of one, so the output's matrix is matrix 0. PROG: 1 runs the epilogue program, 0 stores plainly, -1
 // reads which from the arguments.
@@ -257,6 +271,26 @@ __device__ __forceinline__ void store_tile(const MatmulArgs &args, const Head &h
       vb.x[i] = in0.b == 0 ? x : 0u;
     }
     const Vals<4> o = apply_op<DT, 4, INL>(in0.op, va, vb);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int mm = mt * 16 + 4 * g + i;
+      if (mm < m) store_value<DT>(out, obase + (int64_t)mm * out.sr, o.x[i]);
+    }
+    return;
+  }
+  // one operation on the product and an input: the lane's 4 values of the input loaded together (3 rows of 2048 x 2048
+  // bfp8 with a residual 10.8 -> 7.7 us, 40 rows 20.4 -> 13.7)
+  const OneInput one = one_input(args.prog, h.n_inst);
+  if (one.op >= 0) {
+    Vals<4> r, va, vb;
+#pragma unroll
+    for (int i = 0; i < 4; i++) r.x[i] = load_operand<DT>(args.prog.in[0], ONE ? 0 : b, min(mt * 16 + 4 * g + i, m - 1), n);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const uint32_t x = __float_as_uint(DT == BT_BF16 ? round_packed(acc[i]) : acc[i]);
+      va.x[i] = one.a ? x : r.x[i], vb.x[i] = one.b ? x : r.x[i];
+    }
+    const Vals<4> o = apply_op<DT, 4, INL>(one.op, va, vb);
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const int mm = mt * 16 + 4 * g + i;
@@ -611,8 +645,13 @@ __global__ void __launch_bounds__(256) gemv_x_kernel(const XArgs h) {
 // waited for behind the values. The weights are read with the streaming cache policy (read once): 6.18 and 8.61.
 // A's rows in LDS are G chunks long, so mapping a thread's pieces of A to rows divides by a constant (about 75
 // fewer VALU instructions a wave than a division by the product's K): 5.92 and 8.35.
-template <int FMT, int DT, int MT, int NRW, int G, bool PROG>
-__global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args) {
+// MODE: 0 stores plainly, 1 runs the epilogue program, 2 adds an fp32 residual (res, fp32 out) whose values are loaded
+// with A, ahead of the weights (8 rows of 576 x 576 bfp8 8.5 us through the evaluator, 4.9 so, 4.8 plain), 3 is SiLU x
+// up (B gate then up columns, bf16 out): the block's first two waves take gate runs, the others the up runs of the same
+// columns, which reach the gate waves through LDS (8 rows of 576 x 3072 bfp8 7.5 us on skinny2_kernel, 5.1 so).
+template <int FMT, int DT, int MT, int NRW, int G, int MODE>
+__global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args, const bt_operand res) {
+  static_assert(MODE < 2 || (MT == 1 && NRW == 1), "the residual and SiLU x up modes take a tile a wave");
   constexpr int TB = Tile<FMT>::bytes, R = (G + 3) / 4;  // R: rounds of 4 chunks (bfp4)
   extern __shared__ __attribute__((aligned(16))) uint16_t la[];  // A: 16 MT rows, kp halfwords apart
   // bfp4: each chunk's exponents as gaps placed in the bf16 exponent field (place_gaps), 128 bytes a chunk a run
@@ -624,7 +663,8 @@ __global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args) 
   // banks), so that a piece's row and place are a division by a constant
   const int chunks = h.chunks;
   constexpr int kp = G * 64 + 8;
-  const int run0 = ((int)blockIdx.x * 4 + wib) * NRW;
+  const int run0 = MODE == 3 ? (int)blockIdx.x * 2 + (wib & 1) + (wib >> 1) * (h.nruns / 2) : ((int)blockIdx.x * 4 + wib) * NRW;
+  const bool own = MODE != 3 || (int)blockIdx.x * 2 + (wib & 1) < h.nruns / 2;  // (MODE 3: the wave's run is in its half)
   const int row0 = 16 * MT * (int)blockIdx.y;  // the block's rows of A (and of the output): row0 .. row0 + 16 MT - 1
   // 1. A's pieces for this thread (16 bytes each; rows past the last and columns past K are zeros), loaded before
   // the weights so that staging them waits for these alone
@@ -643,13 +683,20 @@ __global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args) 
     const auto v = __builtin_amdgcn_raw_buffer_load_b128(ar, off, 0, 0);
     av[j] = make_uint4(v[0], v[1], v[2], v[3]);
   }
+  float rv[4] = {};
+  if constexpr (MODE == 2) {
+    const int n = min(run0 * 16 + col, h.n - 1);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      rv[i] = gload((const float *)res.ptr + (int64_t)min(row0 + 4 * g + i, h.m - 1) * res.sr + (int64_t)n * res.sc);
+  }
   // 2. the wave's exponents, then its weights: in flight while A is staged, the exponents first so that they are
   // ready to use (placed as gaps, or handed to the lanes that use them) while the values are still on their way
   uint4 bq[NRW][G];
   uint32_t ew[NRW][FMT == BT_BFP4 ? R : G];  // bfp8: dword col of each chunk's exponents; bfp4: of chunk 4 t + g
 #pragma unroll
   for (int r = 0; r < NRW; r++) {
-    const bool in = run0 + r < h.nruns;
+    const bool in = own && run0 + r < h.nruns;
     const __amdgpu_buffer_rsrc_t tr = buffer(h.b + (int64_t)(in ? run0 + r : 0) * chunks * TB, in ? (uint32_t)chunks * TB : 0u);
 #pragma unroll
     for (int i = 0; i < G; i++) {
@@ -660,7 +707,7 @@ __global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args) 
   __builtin_amdgcn_sched_barrier(0);  // (the scheduler would otherwise sink them among the value loads)
 #pragma unroll
   for (int r = 0; r < NRW; r++) {
-    const bool in = run0 + r < h.nruns;
+    const bool in = own && run0 + r < h.nruns;
     const __amdgpu_buffer_rsrc_t tr = buffer(h.b + (int64_t)(in ? run0 + r : 0) * chunks * TB, in ? (uint32_t)chunks * TB : 0u);
 #pragma unroll
     for (int i = 0; i < G; i++) {
@@ -726,8 +773,26 @@ __global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args) 
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8 *)(ar + 32), bv[1], acc[t], 0, 0, 0);
       }
     }
+    if constexpr (MODE == 3) {
+      __shared__ f32x4 ups[2][64];
+      if (wib >= 2) ups[wib & 1][lane] = acc[0];
+      __syncthreads();
+      if (wib >= 2 || !own) return;
+      const f32x4 up = ups[wib][lane];
+      uint16_t *o = (uint16_t *)h.out.ptr + (int64_t)(row0 + 4 * g) * h.out.sr + run0 * 16 + col;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const float gv = bf16_value(bf16_packed(acc[0][i])), uv = bf16_value(bf16_packed(up[i]));
+        if (row0 + 4 * g + i < h.m) o[(int64_t)i * h.out.sr] = (uint16_t)bf16_packed(gv / (1.0f + expf(-gv)) * uv);
+      }
+      return;
+    }
     if (run0 + r >= h.nruns) continue;
-    if constexpr (PROG) {
+    if constexpr (MODE == 2) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[0][i] += rv[i];
+    }
+    if constexpr (MODE == 1) {
 #pragma unroll
       for (int t = 0; t < MT; t++)
         store_tile<DT, false, true, 1>(args, h, acc[t], 0, (int)blockIdx.y * MT + t, run0 + r, g, col);
@@ -1422,8 +1487,17 @@ __global__ void __launch_bounds__(256) parts_reduce_kernel(const MatmulArgs args
     // the epilogue's inputs (a residual) are fetched first, so their loads are in flight with the partials'
     Coords<1> at;
     at.b[0] = 0, at.r[0] = m, at.c[0] = n, at.ok[0] = true;
-    prefile pre[1];
     const bool prog = args.n_inst != 0;
+    const OneInput one = one_input(args.prog, args.n_inst);
+    if (one.op >= 0) {
+      const uint32_t r = load_operand<DT>(args.prog.in[0], 0, m, n);
+      const float v = sum_splits(p, splits, stride);
+      const uint32_t x = __float_as_uint(DT == BT_BF16 ? round_packed(v) : v);
+      const Vals<1> y = apply_op<DT, 1>(one.op, Vals<1>{{one.a ? x : r}}, Vals<1>{{one.b ? x : r}});
+      store_value<DT>(out, (int64_t)m * out.sr + (int64_t)n * out.sc, y.x[0]);
+      return;
+    }
+    prefile pre[1];
     if (prog) fetch_inputs<DT, 1>(args.prog, at, pre);
     const float v = sum_splits(p, splits, stride);
     uint32_t x[1] = {__float_as_uint(DT == BT_BF16 ? round_packed(v) : v)};
@@ -2446,8 +2520,11 @@ template <int FMT, int DT, int MT, int NRW, int G>
 static void launch_lds_g(const MatmulArgs &args, unsigned blocks, hipStream_t s) {
   const size_t lds = (size_t)16 * MT * (G * 64 + 8) * 2;  // A, G chunks a row
   const dim3 grid(blocks, (unsigned)((args.m + 16 * MT - 1) / (16 * MT)));  // y: blocks of 16 MT rows
-  if (args.n_inst) skinny_lds_kernel<FMT, DT, MT, NRW, G, true><<<grid, 256, lds, s>>>(args);
-  else skinny_lds_kernel<FMT, DT, MT, NRW, G, false><<<grid, 256, lds, s>>>(args);
+  bt_operand res{};
+  if (DT == BT_FP32 && plain_out(args) && residual_program(args, &res) && res.ptr && res.rep == 1 && res.cyc == 0)
+    skinny_lds_kernel<FMT, BT_FP32, MT, NRW, G, 2><<<grid, 256, lds, s>>>(args, res);
+  else if (args.n_inst) skinny_lds_kernel<FMT, DT, MT, NRW, G, 1><<<grid, 256, lds, s>>>(args, res);
+  else skinny_lds_kernel<FMT, DT, MT, NRW, G, 0><<<grid, 256, lds, s>>>(args, res);
 }
 template <int FMT, int DT, int MT, int NRW>
 static void launch_lds_n(const MatmulArgs &args, unsigned blocks, hipStream_t s) {
@@ -2458,6 +2535,19 @@ static void launch_lds_n(const MatmulArgs &args, unsigned blocks, hipStream_t s)
 template <int FMT, int DT>
 static void launch_lds(const MatmulArgs &args, unsigned blocks, hipStream_t s) {
   launch_lds_n<FMT, DT, 1, 1>(args, blocks, s);
+}
+
+// SiLU x up on skinny_lds_kernel: up to 256 rows of block-float B with a short K; false when the product doesn't fit.
+template <int FMT, int G>
+static void launch_lds_swiglu_g(const MatmulArgs &args, hipStream_t s) {
+  const dim3 grid((unsigned)((args.nruns / 2 + 1) / 2), (unsigned)((args.m + 15) / 16));
+  skinny_lds_kernel<FMT, BT_BF16, 1, 1, G, 3><<<grid, 256, (size_t)16 * (G * 64 + 8) * 2, s>>>(args, bt_operand{});
+}
+template <int FMT>
+static void launch_lds_swiglu(const MatmulArgs &args, hipStream_t s) {
+  if (args.chunks <= 6) launch_lds_swiglu_g<FMT, 6>(args, s);
+  else if (args.chunks <= 9) launch_lds_swiglu_g<FMT, 9>(args, s);
+  else launch_lds_swiglu_g<FMT, 12>(args, s);
 }
 
 template <int FMT, int DT, int ROWS>
@@ -3096,6 +3186,12 @@ extern "C" int bt_matmul_swiglu(bt_runtime *rt, const bt_operand *a, int b_fmt, 
   }
   if ((m <= 64 || (m <= 256 && gemm_blocks < 128)) && a->sr % 8 == 0 && a->ptr % 16 == 0 && ((31 * a->sr + 2 * k + 1024) * 2 < (1ll << 32))) {
     if (launch_stream(r, args, b_fmt, true) || launch_parts(r, args, b_fmt, true)) {
+      BT_LAUNCHED("matmul_swiglu");
+      return BT_OK;
+    }
+    if (b_fmt != BT_BF16 && args.chunks <= 12 && plain_out(args) && ((m - 1) * a->sr + k) * 2 < (1ll << 31)) {
+      if (b_fmt == BT_BFP8) launch_lds_swiglu<BT_BFP8>(args, r->stream);
+      else launch_lds_swiglu<BT_BFP4>(args, r->stream);
       BT_LAUNCHED("matmul_swiglu");
       return BT_OK;
     }

@@ -276,6 +276,37 @@ def test_one_operation_epilogues_equal_the_evaluator(rt, m, out):
   assert np.array_equal(neg, -plain)
 
 
+# one operation on the product and one input (a residual, a bias, a product of two) runs straight on the tile's values,
+# the input on either side: bit for bit the same program made longer by a product with 1 (the evaluator); and SiLU x up
+# with a short K bit for bit silu(g) * u of the plain product's columns, in rows off the tiles of 16
+@pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bfp4"])
+@pytest.mark.parametrize("m,k,n", [(1, 576, 200), (3, 1536, 96), (5, 576, 608), (17, 768, 64), (40, 320, 288), (256, 128, 96), (9, 1024, 320)])
+def test_one_input_epilogues_equal_the_evaluator(rt, fmt, m, k, n):
+  rng = np.random.default_rng(m + n)
+  x, w = rng.normal(0, 1, (m, k)), rng.normal(0, 0.05, (k, n)).astype(np.float32)
+  if fmt == "bf16": cols = bf16_columns(rt, w)
+  else: cols = columns(rt, *pack(rt, w, fmt), fmt, 1, k, n)
+  other, bias = up(rt, rng.normal(0, 1, (m, n)).astype(np.float32)), up(rt, B.bf16_bits(rng.normal(0, 1, (1, n))))
+  for out in ("bf16", "fp32"):
+    for name, side in (("add", 0), ("add", 1), ("sub", 1), ("mul", 0), ("max", 0), ("cmplt", 1)):
+      for ptr, kind, sr in ((other, "fp32", n), (bias, "bf16", 0)):
+        got = []
+        for longer in (False, True):
+          p = Program(out, epilogue=True)
+          v, r = p.value(), p.load(p.input(_lib.operand(ptr, kind, m * n, sr, 1)))
+          y = p.op(name, r, v) if side else p.op(name, v, r)
+          got.append(matmul(rt, x, cols, fmt, 1, n, out=out, prog=p.build(p.op("mul", y, p.const(1.0)) if longer else y))[0])
+        assert np.array_equal(got[0], got[1]), (out, name, side, kind)
+  if n % 32: return
+  res = rt.dram_alloc(m * n)
+  rt.run("swiglu", "matmul_swiglu", ctypes.byref(_lib.operand(up(rt, B.bf16_bits(x)), "bf16", m * k, k, 1)), _lib.DTYPES[fmt],
+         cols, m, k, n, ctypes.byref(_lib.operand(res, "bf16", m * n // 2, n // 2, 1)))
+  plain = matmul(rt, x, cols, fmt, 1, n)[0].astype(np.float64)
+  g, u = plain[:, :n // 2], plain[:, n // 2:]
+  want = g / (1 + np.exp(-g)) * u
+  assert np.all(np.abs(bits_to_float(down(rt, res, (m, n // 2), np.uint16)) - want) <= 2.0 ** -8 * 1.01 * np.abs(want))  # one rounding
+
+
 @pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
 @pytest.mark.parametrize("m,k,n", [(16, 576, 49152), (20, 576, 40000), (7, 320, 1000), (32, 768, 4096)])
 def test_short_k_rows_with_a_in_lds(rt, fmt, m, k, n):
