@@ -131,9 +131,15 @@ def check(status):
     raise EXCEPTIONS.get(status, RuntimeError)(message)
 
 
+_functions = {}  # name: the library's bt_<name>, looked up once
+
+
 def call(name, *args):
   """Calls bt_<name> and raises on a nonzero status."""
-  check(getattr(load(), "bt_" + name)(*args))
+  f = _functions.get(name)
+  if f is None: f = _functions[name] = getattr(load(), "bt_" + name)
+  status = f(*args)
+  if status: check(status)
 
 
 def device_count():

@@ -5,7 +5,7 @@ Instructions are built on virtual registers, one per value. build() maps them on
 liveness, so an expression of up to 48 instructions fits as long as no more than 16 values are alive at once.
 Register 0 is the matmul value in an epilogue, and is never reused there.
 """
-import struct
+import functools, struct
 from baretile_amd import _lib
 
 
@@ -65,40 +65,48 @@ class Program:
 
   def build(self, result):
     """The bt_program struct, with registers allocated. result is the vreg of the value to store."""
-    n = len(self.insts)
-    if n > _lib.MAX_INST: raise ValueError(f"a program has at most {_lib.MAX_INST} instructions, not {n}")
-    load = _lib.OP["load"]
-    last = {}  # vreg -> index of its last reader
-    for i, (op, dst, a, b, c, imm) in enumerate(self.insts):
-      if op == load: continue
-      for s in self._reads(op, a, b, c): last[s] = i
-    last[result] = n
-    phys, free = {}, [r for r in range(_lib.MAX_REGS - 1, 0 if self.epilogue else -1, -1)]
-    if self.epilogue: phys[0] = 0
-    p = _lib.Program()
-    p.n_inst, p.n_inputs, p.dtype = n, len(self.inputs), _lib.DTYPES[self.dtype]
+    p = _lib.Program.from_buffer_copy(_assemble(self.dtype, self.epilogue, tuple(self.insts), len(self.inputs), result))
     for i, op in enumerate(self.inputs): p.inputs[i] = op
-    const = _lib.OP["const"]
-    for i, (op, dst, a, b, c, imm) in enumerate(self.insts):
-      srcs = [] if op in (load, const) else self._reads(op, a, b, c)
-      regs = [phys[s] for s in srcs]
-      for s in set(srcs):  # a register whose value dies here can take the result
-        if last.get(s) == i and not (self.epilogue and s == 0): free.append(phys.pop(s))
-      if not free: raise ValueError(f"a program needs more than {_lib.MAX_REGS} live values")
-      d = free.pop()
-      if dst in last: phys[dst] = d
-      else: free.append(d)  # never read
-      ra, rb, rc = (a, 0, 0) if op == load else tuple(regs + [0, 0, 0])[:3]
-      p.inst[i] = _lib.Inst(op, d, ra, rb, rc, (0, 0, 0), imm)
-    p.result = phys[result]
     return p
 
   UNARY = {"mov", "neg", "relu", "exp", "exp2", "log", "log2", "sqrt", "recip", "rsqrt", "sin", "cos", "sigmoid", "silu",
            "gelu", "tanh", "ftob"}
 
-  def _reads(self, op, a, b, c):
-    name = _lib.OPS[op]
-    if name == "const": return []
-    if name in self.UNARY: return [a]
-    if name == "where": return [a, b, c]
-    return [a, b]
+
+def _reads(op, a, b, c):
+  name = _lib.OPS[op]
+  if name == "const": return []
+  if name in Program.UNARY: return [a]
+  if name == "where": return [a, b, c]
+  return [a, b]
+
+
+@functools.lru_cache(maxsize=1024)
+def _assemble(dtype, epilogue, insts, n_inputs, result):
+  """The bytes of a bt_program of these instructions, its inputs left empty: a function of the instructions alone, so a
+  program that builds the same expression again finds its registers allocated (half of an expression's host time)."""
+  n = len(insts)
+  if n > _lib.MAX_INST: raise ValueError(f"a program has at most {_lib.MAX_INST} instructions, not {n}")
+  load, const = _lib.OP["load"], _lib.OP["const"]
+  last = {}  # vreg -> index of its last reader
+  for i, (op, dst, a, b, c, imm) in enumerate(insts):
+    if op == load: continue
+    for s in _reads(op, a, b, c): last[s] = i
+  last[result] = n
+  phys, free = {}, [r for r in range(_lib.MAX_REGS - 1, 0 if epilogue else -1, -1)]
+  if epilogue: phys[0] = 0
+  p = _lib.Program()
+  p.n_inst, p.n_inputs, p.dtype = n, n_inputs, _lib.DTYPES[dtype]
+  for i, (op, dst, a, b, c, imm) in enumerate(insts):
+    srcs = [] if op in (load, const) else _reads(op, a, b, c)
+    regs = [phys[s] for s in srcs]
+    for s in set(srcs):  # a register whose value dies here can take the result
+      if last.get(s) == i and not (epilogue and s == 0): free.append(phys.pop(s))
+    if not free: raise ValueError(f"a program needs more than {_lib.MAX_REGS} live values")
+    d = free.pop()
+    if dst in last: phys[dst] = d
+    else: free.append(d)  # never read
+    ra, rb, rc = (a, 0, 0) if op == load else tuple(regs + [0, 0, 0])[:3]
+    p.inst[i] = _lib.Inst(op, d, ra, rb, rc, (0, 0, 0), imm)
+  p.result = phys[result]
+  return bytes(p)

@@ -117,9 +117,14 @@ class Runtime:
   def run(self, name, fn, *args, reads=None):
     """Queue bt_<fn>(handle, *args), counted as launch `name` that reads `reads` bytes (None: not counted)."""
     self.check()
-    done = self.launched(name, reads)
-    _lib.call(fn, self.handle, *args)
-    done()
+    if self.timing:
+      done = self.launched(name, reads)
+      _lib.call(fn, self.handle, *args)
+      done()
+    else:
+      self.launches += 1
+      if self.log is not None: self.log.append(name)
+      _lib.call(fn, self.handle, *args)
 
   def sleep(self, seconds):
     """Queue a launch that keeps the device busy for `seconds` (at most 10) and then ends by itself."""

@@ -27,6 +27,7 @@ UNARY = ("neg", "relu", "exp", "exp2", "log", "log2", "sqrt", "recip", "rsqrt", 
 BINARY = ("add", "sub", "mul", "div", "max", "min", "cmplt", "cmple", "cmpne", "cmpeq")
 INT32_OPS = ("add", "sub", "max", "min", "cmplt", "cmple", "cmpne", "cmpeq", "neg", "relu", "where", "mul")
 ELEMENTWISE = UNARY + BINARY + ("where", "cast")
+_ELEMENTWISE = frozenset(ELEMENTWISE)  # for lookups
 REDUCE = ("sum", "amax")
 
 
@@ -39,6 +40,7 @@ def _shape(shape):
 
 def _broadcast(a, b):
   """numpy broadcasting of two shapes, or None."""
+  if a == b: return tuple(a)
   n = max(len(a), len(b))
   a, b = (1,) * (n - len(a)) + tuple(a), (1,) * (n - len(b)) + tuple(b)
   out = []
@@ -113,10 +115,11 @@ class Tensor:
   formats: bf16, fp32, int32, bfp8, bfp4 (tensor.py:25-35). An unrealized tensor holds an op and its operands; a
   realized one holds storage and the strides it is read through."""
   def __init__(self, rt, rows, cols, op=None, srcs=(), batch=1, dtype="bf16", args=()):
-    batch, rows, cols = _shape((batch, rows, cols))
+    if not (type(batch) is type(rows) is type(cols) is int and batch > 0 and rows > 0 and cols > 0):
+      batch, rows, cols = _shape((batch, rows, cols))
     if dtype not in DTYPES: raise ValueError(f"unknown tensor dtype: {dtype}")
-    if any(isinstance(s, Tensor) and s.rt is not rt for s in srcs):
-      raise ValueError("tensor operands must use the same runtime")
+    for s in srcs:
+      if isinstance(s, Tensor) and s.rt is not rt: raise ValueError("tensor operands must use the same runtime")
     rt.check()
     self.rt, self.rows, self.cols, self.batch, self.dtype = rt, rows, cols, batch, dtype
     self.op, self.srcs, self.args, self.lead = op, tuple(srcs), args, (batch,)
@@ -211,14 +214,14 @@ class Tensor:
     out_lead = self.lead if out_lead is None else tuple(out_lead)
     sr = 0 if (out_rows or self.rows) != self.rows and self.rows == 1 else self.sr
     sc = 0 if (out_cols or self.cols) != self.cols and self.cols == 1 else self.sc
+    if self.batch == 1 and len(self.lead) <= len(out_lead):  # one matrix for every batch entry
+      return _lib.Operand(self.addr, 0, sr, sc, _lib.DTYPES[self.dtype], 1, 0, 0)
     mine = (1,) * (len(out_lead) - len(self.lead)) + self.lead
     if len(mine) > len(out_lead) or any(m not in (1, o) for m, o in zip(mine, out_lead)):
       if self.batch == math.prod(out_lead):  # the same matrices under other leading sizes
         return _lib.Operand(self.addr, self.sb, sr, sc, _lib.DTYPES[self.dtype], self.rep, self.cyc, 0)
       raise ValueError(f"cannot read {self.shape} as {out_lead}")
     big = [k for k, n in enumerate(mine) if n > 1]
-    if not big:  # one matrix for every batch entry
-      return _lib.Operand(self.addr, 0, sr, sc, _lib.DTYPES[self.dtype], 1, 0, 0)
     if mine == out_lead:
       return _lib.Operand(self.addr, self.sb, sr, sc, _lib.DTYPES[self.dtype], self.rep, self.cyc, 0)
     if big != list(range(big[0], big[-1] + 1)) or self.rep != 1 or self.cyc != 0:
@@ -500,7 +503,7 @@ class Tensor:
   # ---- elementwise
   def _new(self, op, srcs, shape, dtype, args=()):
     lead, rows, cols = shape[:-2], shape[-2], shape[-1]
-    t = Tensor(self.rt, rows, cols, op, srcs, math.prod(lead) if lead else 1, dtype, args)
+    t = Tensor(self.rt, rows, cols, op, srcs, (lead[0] if len(lead) == 1 else math.prod(lead)) if lead else 1, dtype, args)
     t.lead = tuple(lead) if lead else (1,)
     return t
 
@@ -1005,7 +1008,7 @@ class Tensor:
     out = into if into is not None else None
     if self.op == "matmul": _realize_matmul(self, None, out)
     elif self.op in REDUCE: _realize_reduce(self, out)
-    elif self.op in ELEMENTWISE: _realize_elementwise(self, out)
+    elif self.op in _ELEMENTWISE: _realize_elementwise(self, out)
     else: raise ValueError(f"cannot realize op {self.op}")
     return self
 
@@ -1123,8 +1126,8 @@ class _Lowering:
       if u is self.root or u.dtype == self.dtype and src.dtype == self.dtype: r = self.emit(src)
       elif u.dtype == self.dtype: r = self.leaf(src)  # loading converts src's dtype exactly as the cast does
       else: r = self.leaf(u)  # another dtype: a kernel of its own
-    elif u.op in ELEMENTWISE and u.dtype == self.dtype and _fits_root(u, self.root):
-      r = self.p.op(u.op, *(self.emit(s) for s in u.srcs))
+    elif u.op in _ELEMENTWISE and u.dtype == self.dtype and _fits_root(u, self.root):
+      r = self.p.op(u.op, *[self.emit(s) for s in u.srcs])
     else: r = self.leaf(u)
     self.memo[id(u)] = r
     return r
@@ -1133,6 +1136,7 @@ class _Lowering:
 def _fits_root(u, root):
   """Whether u can be computed inside root's kernel: its shape broadcasts to root's (a broadcast subtree is evaluated
   again at each element it covers, reading its inputs with strides of 0)."""
+  if u.rows == root.rows and u.cols == root.cols and u.lead == root.lead: return True
   return _broadcast(u.shape, root.shape) == tuple(root.shape) and len(u.shape) <= len(root.shape)
 
 
@@ -1152,7 +1156,7 @@ def _find_anchor(t, dtype):
     if u.op == "matmul":
       if u.shape == t.shape and u.dtype == dtype and u.srcs[1].dtype != "fp32": return u
       continue
-    if u.op in ELEMENTWISE and (u.dtype == dtype or u is t) and u.shape == t.shape:
+    if u.op in _ELEMENTWISE and (u.dtype == dtype or u is t) and u.shape == t.shape:
       stack.extend(s for s in u.srcs if isinstance(s, Tensor))
   return None
 
@@ -1193,7 +1197,7 @@ def _realize_elementwise(t, into):
   low, prog = _build(t, dtype, None)
   out = _dest(t, into)
   t.rt.run(_name(prog), "elementwise", ctypes.byref(prog), out.batch, out.rows, out.cols, ctypes.byref(out._operand()),
-           reads=_bytes(*low.keep))
+           reads=_bytes(*low.keep) if t.rt.timing else None)
 
 
 def _name(prog):
@@ -1205,7 +1209,7 @@ def _realize_reduce(t, into):
   src = t.srcs[0]
   axis = t.args[0]
   n = len(src.shape)
-  dtype = _compute_dtype(src) if src.op in ELEMENTWISE else src.dtype
+  dtype = _compute_dtype(src) if src.op in _ELEMENTWISE else src.dtype
   if dtype in BFP: dtype = "bf16"
   low = None
   # the prologue: src's tree at src's shape
@@ -1222,7 +1226,7 @@ def _realize_reduce(t, into):
   kind = _lib.REDUCE_SUM if t.op == "sum" else _lib.REDUCE_MAX  # before _dest, which clears t's op
   out = _dest(t, into)
   t.rt.run("reduce", "reduce", ctypes.byref(prog), kind, k, src.batch, src.rows, src.cols, sweep, step,
-           ctypes.byref(out._operand()), reads=_bytes(*low.keep))
+           ctypes.byref(out._operand()), reads=_bytes(*low.keep) if t.rt.timing else None)
 
 
 def _stream_fits(a, w):
@@ -1310,7 +1314,7 @@ def _realize_matmul(m, root, into):
   else: aop = _lib.Operand(a.addr, a.sb, a.sr, a.sc, _lib.BF16, 1, 0, 0)
   m.rt.run("matmul", "matmul", ctypes.byref(aop), fmt, tiles, b_batch, batch, a.rows, a.cols, m.cols,
            ctypes.byref(prog) if prog is not None else None, ctypes.byref(out._operand()),
-           reads=_bytes(a, keep_b, *keep))
+           reads=_bytes(a, keep_b, *keep) if m.rt.timing else None)
   if root is not None and m is not root:  # the matmul itself was never stored: a later read recomputes it
     pass
   del keep, keep_b

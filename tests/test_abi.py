@@ -65,3 +65,22 @@ def test_struct_sizes_match_the_header(tmp_path):
     assert int(got[name]) == ctypes.sizeof(cls), name
     for field, *_ in cls._fields_:
       assert int(got[f"{name}.{field}"]) == getattr(cls, field).offset, (name, field)
+
+
+def test_a_program_built_again_keeps_its_own_inputs_and_limits():
+  from baretile_amd.program import Program
+  def build(ptr, const=2.0, dtype="bf16"):
+    p = Program(dtype)
+    x, y = (p.load(p.input(_lib.operand(ptr + i, "bf16", 1, 1, 1))) for i in range(2))
+    return p.build(p.op("add", p.op("mul", x, p.const(const)), y))
+  a, b, c, d = build(16), build(32), build(16, 3.0), build(16, dtype="fp32")
+  assert [a.inputs[i].ptr for i in range(2)] == [16, 17] and [b.inputs[i].ptr for i in range(2)] == [32, 33]
+  code = lambda p: (p.n_inst, p.n_inputs, p.dtype, p.result, [(i.op, i.dst, i.a, i.b, i.c, i.imm) for i in p.inst])
+  assert code(a) == code(b) != code(c) and code(d)[2] != code(a)[2]
+  for _ in range(2):  # a refusal is a refusal again
+    p = Program("bf16")
+    v = p.load(p.input(_lib.operand(16, "bf16")))
+    vs = [p.op("add", v, p.const(float(i))) for i in range(17)]
+    out = vs[0]
+    for u in vs[1:]: out = p.op("mul", u, out)
+    with pytest.raises(ValueError, match="more than|at most"): p.build(out)
