@@ -68,6 +68,7 @@ def test_struct_sizes_match_the_header(tmp_path):
 
 
 def test_a_program_built_again_keeps_its_own_inputs_and_limits():
+  from baretile_amd import _lib
   from baretile_amd.program import Program
   def build(ptr, const=2.0, dtype="bf16"):
     p = Program(dtype)
