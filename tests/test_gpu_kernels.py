@@ -849,6 +849,47 @@ def test_attention_extremes(rt):
   assert np.array_equal(attend(rt, q, k, v, np.array([[63]])), np.full((1, 1, 64), 2.0))
 
 
+# Block-float caches read in place give the bits of the values they hold, whatever their exponent bytes: blocks of 64
+# keys whose exponents are all in 7..254 and blocks where some are not (small ones with normalized magnitudes, in V ones
+# that wrap, zeros under any), rows whose exponents come in one load and rows (hd + 16 apart) where they can't; 4-wave
+# parts with one and more blocks a wave, one-wave parts, and prefill
+@pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
+@pytest.mark.parametrize("hd,rows,keys,parts,pad", [(64, 1, 200, 1, 0), (128, 1, 600, 1, 0), (128, 2, 500, 8, 0), (64, 1, 333, 6, 16),
+                                                    (128, 1, 400, 1, 16), (128, 3, 130, 3, 16), (64, 40, 200, 0, 16), (128, 70, 300, 0, 0)])
+def test_attention_block_floats_of_any_exponent(rt, fmt, hd, rows, keys, parts, pad):
+  rng = np.random.default_rng(hd + keys)
+  top, sr = 127 if fmt == "bfp8" else 7, hd + pad
+  planes, bits = [], []
+  for value in (False, True):
+    e = rng.integers(115, 131, (2, keys, sr // 16))
+    q = rng.integers(-top, top + 1, (2, keys, sr // 16, 16))
+    odd = rng.random(e.shape) < (np.arange(keys) // 64 % 2 * 0.05)[:, None]  # in every other block of keys
+    kind = rng.integers(0, 3 if value else 2, e.shape)
+    e[odd], q[odd & (kind == 0)] = rng.integers(0, 7, odd.sum()), 0
+    q[odd & (kind == 1)] = rng.integers(top // 2 + 1, top + 1, (int((odd & (kind == 1)).sum()), 16))
+    q[odd & (kind == 2)] = 1
+    e[odd & (kind == 0)] = rng.integers(0, 256, int((odd & (kind == 0)).sum()))
+    n = q.reshape(2, keys, sr)
+    byte = np.where(n < 0, 256 + n, n) if fmt == "bfp8" else (n[..., 0::2] & 15) | (n[..., 1::2] & 15) << 4
+    planes.append((up(rt, e.astype(np.uint8)), up(rt, byte.astype(np.uint8))))
+    field = (n < 0) * (128 if fmt == "bfp8" else 8) | np.abs(n)
+    bits.append(up(rt, B.decode_bits(np.repeat(e, 16, -1), field, fmt).astype(np.uint16)))
+  E = 6
+  q = up(rt, B.bf16_bits(np.abs(rng.normal(0, 1, (E, rows, hd))) / np.sqrt(hd)))
+  places = up(rt, np.full((1, rows), keys - 1, np.int32))
+  def run(k, v, fmt_, ke=0, ve=0):
+    o = rt.dram_alloc(E * rows * hd * 2)
+    args = _lib.AttentionArgs(q, k, v, o, places, rows * hd, hd, keys * sr, sr, keys * sr, sr, rows * hd, hd, 0, E, 3, rows, keys, hd,
+                              0, parts, 0, 0, 0, 0, 0, fmt_, 0, ke, ve)
+    need = ctypes.c_uint64()
+    _lib.call("attention_scratch", ctypes.byref(args), ctypes.byref(need))
+    if need.value: args.scratch, args.scratch_bytes = rt.dram_alloc(need.value), need.value
+    rt.run("attention", "attention", ctypes.byref(args))
+    return down(rt, o, (E, rows, hd), np.uint16)
+  (ke, k), (ve, v) = planes
+  assert np.array_equal(run(k, v, FMT[fmt], ke, ve), run(*bits, 0))
+
+
 # ---- gather and put ----------------------------------------------------------------------------------------------
 
 def test_gather_and_put(rt):
