@@ -3417,7 +3417,19 @@ extern "C" int bt_matmul_residual_rms(bt_runtime *rt, const bt_operand *a, int b
     return fail(BT_EINVAL, "matmul_residual_rms: fp32 rows 16-byte aligned, bf16 rows 8-byte aligned");
   StreamPlan p;
   float *part;
-  if (int s = stream_partials(r, a, b_fmt, b, m, k, n, "matmul_residual_rms", &p, &part)) return s;
+  if (int s = stream_partials(r, a, b_fmt, b, m, k, n, "matmul_residual_rms", &p, &part)) {
+    if (s != BT_ESTATE) return s;
+    // no room for the partial sums (a capture that the scratch can't grow in): the product with its residual epilogue,
+    // then the norm, as the unfused calls of a step recorded before it has run
+    bt_program add{};
+    add.n_inst = 2, add.n_inputs = 1, add.dtype = BT_FP32, add.result = 1;
+    add.inst[0].op = BT_OP_LOAD, add.inst[0].dst = 1;
+    add.inst[1].op = BT_OP_ADD, add.inst[1].dst = 1, add.inst[1].a = 1;
+    add.in[0] = bt_operand{residual, m * res_sr, res_sr, 1, BT_FP32, 1, 0, 0};
+    const bt_operand out{x, m * x_sr, x_sr, 1, BT_FP32, 1, 0, 0};
+    if (int e = bt_matmul(rt, a, b_fmt, b, 1, 1, m, k, n, &add, &out)) return e;
+    return bt_rms_rows(rt, x, m, n, x_sr, norm, eps, h, h_sr);
+  }
   residual_rms_kernel<<<(unsigned)m, RMS_THREADS, 0, r->stream>>>(part, p.splits, (int64_t)16 * p.mt * n, (int)n,
                                                           (const float *)(uintptr_t)residual, res_sr,
                                                           (float *)(uintptr_t)x, x_sr, (const uint16_t *)(uintptr_t)norm,

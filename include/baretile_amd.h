@@ -262,8 +262,8 @@ int bt_matmul_row_rope(bt_runtime *rt, const bt_row_args *args, const bt_rope_ar
  * 32 rows of A (bf16, contiguous 16-byte aligned rows) against a long K (a multiple of 256, over 768) is left as
  * split-K partial sums in the runtime's scratch and the kernel that consumes it sums them, in split order as
  * bt_matmul's reduction does, so the product and its reduction are neither stored nor launched on their own. Each is
- * bit for bit the unfused calls. Inside a graph capture the runtime's scratch can't grow: make the call once before
- * capturing. BT_EINVAL for a product outside those shapes.
+ * bit for bit the unfused calls. Inside a graph capture the runtime's scratch can't grow: bt_matmul_rope_put is then to
+ * be called once before capturing (else BT_ESTATE), bt_matmul_residual_rms makes the unfused calls. BT_EINVAL for a product outside those shapes.
  *
  * bt_matmul_rope_put: bt_matmul (bf16 product, no epilogue) then bt_rope_put on its product. rope->qkv and qkv_sr
  * are not used; rope->rows is m, n is (heads + 2 kv) head_dim with head_dim a multiple of 16, and the tables, q and

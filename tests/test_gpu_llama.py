@@ -174,6 +174,21 @@ def test_slots_layer_matches_each_slot_in_numpy(rt):
       assert np.abs(got_r - want_r).max() <= 0.03 * np.abs(want_r).max(), (s, np.abs(got_r - want_r).max())
 
 
+@pytest.mark.parametrize("n", [5, 8, 32])
+def test_forward_of_slots_equals_its_layers(rt, n):
+  # forward() ends each block in the next block's norm (chained_layer) up to 32 tokens: the logits of layer() by layer()
+  c, ref, dc, dw = setup(rt, 2, 256, "bfp8")
+  ids, places = (Tensor.of(rt, [v], "int32") for v in (list(range(3, 3 + n)), [2] * n))
+  caches, other = (llama.kv_cache(rt, dc, 4 * n) for _ in range(2))
+  got = llama.forward(ids, places, dw, dc, caches, slots=n).tobytes()
+  x, first = dw["embed"].gather(ids).float(), llama.starts(dw, n, n, 4)
+  rot = (dw["cos"].gather(places), dw["sin"].gather(places), dw["turn"])
+  rows, column = (places + first).realize(), (first + places).realize().reshape(1, n, 1)
+  for l in range(2): x = llama.layer(x, llama.block(dw, l), dc, rot, column, other[l], rows, first.reshape(1, n, 1))
+  assert got == llama.rms(x, dw["norm"], dc).matmul(dw["embed.T"], "fp32").tobytes()
+  for a, b in zip(caches, other): assert a.tobytes() == b.tobytes()
+
+
 def test_slots_layer_then_fuses_the_next_norm(rt):
   # slots_layer(h=, then=): the block's input norm given, and the down product's partial sums, the residual add and
   # the next norm in one kernel (bt_matmul_residual_rms) -- bit for bit the block's x and rms_rows of it, in two

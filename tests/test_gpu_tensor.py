@@ -4,7 +4,7 @@ import math
 import numpy as np
 import pytest
 
-from baretile_amd.tensor import Tensor, jit
+from baretile_amd.tensor import Recording, Tensor, jit
 from oracle import bfp as B, ops
 
 pytestmark = pytest.mark.gpu
@@ -435,6 +435,31 @@ def test_matmul_residual_rms_equals_unfused(rt, fmt, rows, k, n):
   want = res + a.astype(np.float64) @ wv
   assert np.all(np.abs(got - want) <= 2.0 ** -8 * (np.abs(a) @ np.abs(wv)) + 1e-3 * np.abs(res) + 1e-6)
   assert np.frombuffer(tr.tobytes(), np.float32).reshape(rows, n).tolist() == res.tolist()  # the residual kept
+
+
+def test_matmul_residual_rms_recorded_first(chip):
+  # recorded on a fresh runtime, whose scratch has no room for the partial sums and can't grow: the unfused calls, whose
+  # one-launch product sums K in another order (fp32, K = 2048: within 2048 2^-24 of the sum of magnitudes), replayed
+  # with eager work between
+  from baretile_amd.runtime import Runtime
+  rt = Runtime(chip)
+  try:
+    rng = np.random.default_rng(31)
+    wt, wv = _weights(rt, 2048, 640, "bfp8", 3)
+    a, res = B.bf16(rng.normal(0, 1, (7, 2048)).astype(np.float32)), rng.normal(0, 4, (7, 640)).astype(np.float32)
+    norm = Tensor.of(rt, B.bf16(rng.normal(1, 0.1, (1, 640)).astype(np.float32)))
+    ta, tr = Tensor.of(rt, a), Tensor.of(rt, res[None], "fp32")
+    rt.wait()
+    rec = Recording(rt)
+    with rec: x, h = ta.matmul_residual_rms(wt, tr, norm, 1e-5)
+    for _ in range(3):
+      rec.send()
+      got = np.frombuffer(x.tobytes(), np.float32).reshape(7, 640)
+      want = res + a.astype(np.float64) @ wv
+      assert np.all(np.abs(got - want) <= 2048 * 2.0 ** -24 * (np.abs(a) @ np.abs(wv) + np.abs(res)))
+      assert h.tobytes() == x.rms_rows(norm, 1e-5).tobytes()
+    rec.close()
+  finally: rt.close()
 
 
 @pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
