@@ -18,9 +18,10 @@
 //
 // Decode (at most 4 tiles, 64 pairs, per key head): the block's 4 waves split the keys of one tile, 64 at a time, and
 // combine their running sums in LDS at the end. Long caches are split further into parts, each a run of the tile's
-// visible keys, written as fp32 partial sums to scratch and combined by a second kernel; from 5 to 16 blocks of keys a
-// part is one block, folded by a block of one wave whose state is the part's partial sum. Prefill: the block's waves take 4 consecutive tiles and share each block
-// of 64 keys and values through LDS, double-buffered.
+// visible keys, written as fp32 partial sums to scratch and combined by a second kernel; while the blocks of keys are few
+// a part is one block, folded by a block of one wave whose state is the part's partial sum (plan_attention says
+// where the lines lie). Prefill: the block's waves take 4 consecutive tiles and share each block of 64 keys and values
+// through LDS, double-buffered.
 #include "common.h"
 #include "lds_load.h"
 #include <mutex>
@@ -943,7 +944,8 @@ __global__ void __launch_bounds__(512, 1) attention_prefill_kernel(const bt_atte
   } else {
     // block floats: loaded into registers, held there as stored while the current block is folded, then decoded on
     // their way to LDS, in the same layout (decoded as they arrived, a branch for each 8 values: 32 heads of 128, 4096
-    // rows of bfp8 310 -> 246 us, bfp4 at 2048 rows 101 -> 75). The thread's words at row kr0 + (256 / (HD / 8)) i, logical unit kc / 8.
+    // rows of bfp8 310 -> 246 us, bfp4 at 2048 rows 101 -> 75). The thread's words at row kr0 + (256 / (HD / 8)) i,
+    // logical unit kc / 8.
     const KvSrc kr = kv_src<KF>(a.k, a.k_exps, (int64_t)kvh * a.k_sh, bhi < 0 ? 0 : (int64_t)bhi * a.k_sr + HD);
     const KvSrc vr = kv_src<KF>(a.v, a.v_exps, (int64_t)kvh * a.v_sh, bhi < 0 ? 0 : (int64_t)bhi * a.v_sr + HD);
     const int kr0 = th / (HD / 8), kc = th % (HD / 8) * 8;
@@ -956,9 +958,15 @@ __global__ void __launch_bounds__(512, 1) attention_prefill_kernel(const bt_atte
     auto fetch = [&](int kb) {
       const uint32_t kbo = (uint32_t)((int64_t)kb * a.k_sr), vbo = (uint32_t)((int64_t)kb * a.v_sr);
 #pragma unroll
-      for (int i = 0; i < KW; i++) kreg[i] = kv_fetch8<KF>(kr, koff + (kbo + i * kstep)), exps[i] = kv_exp8<KF>(kr, koff + (kbo + i * kstep));
+      for (int i = 0; i < KW; i++) {
+        const uint32_t e = koff + (kbo + i * kstep);
+        kreg[i] = kv_fetch8<KF>(kr, e), exps[i] = kv_exp8<KF>(kr, e);
+      }
 #pragma unroll
-      for (int i = 0; i < KW; i++) vreg[i] = kv_fetch8<KF>(vr, voff + (vbo + i * vstep)), exps[KW + i] = kv_exp8<KF>(vr, voff + (vbo + i * vstep));
+      for (int i = 0; i < KW; i++) {
+        const uint32_t e = voff + (vbo + i * vstep);
+        vreg[i] = kv_fetch8<KF>(vr, e), exps[KW + i] = kv_exp8<KF>(vr, e);
+      }
     };
     auto stash = [&](uint16_t *stage) {
       by_exponents(exps, [&](auto ord) {
@@ -1095,8 +1103,10 @@ static int plan_attention(const bt_attention_args *a, AttnPlan *p) {
   if (a->firsts && a->firsts % 4) return fail(BT_EINVAL, "attention's firsts must be int32-aligned");
   if (a->firsts && a->firsts_sh != 0 && a->firsts_sh != a->rows) return fail(BT_EINVAL, "firsts' head stride is 0 or rows");
   const int kvh = a->heads / a->rep, np = a->rep * a->rows;
-  // rows with regions of their own: tiles by row while they are few (a decode step's slots, one token or a few each)
-  const bool by_row = a->firsts && a->rows > 1 && a->rows <= 32;
+  // rows with regions of their own: tiles by row while they are few (a decode step's slots, one token or a few each),
+  // where the parts are the library's to choose: its plans take 5.7 MB of scratch at most, while parts that a caller
+  // chose for packed tiles would outgrow bt_attention_noalloc's 8 MiB over 16 times the tiles
+  const bool by_row = a->firsts && a->rows > 1 && a->rows <= 32 && a->parts == 0;
   const int per_row = (a->rep + 15) / 16;
   p->tiles = Tiles{by_row ? a->rows * per_row : (np + 15) / 16, by_row ? per_row : 0, make_fastdiv((uint32_t)a->rep),
                    make_fastdiv((uint32_t)per_row)};

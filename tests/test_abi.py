@@ -85,3 +85,22 @@ def test_a_program_built_again_keeps_its_own_inputs_and_limits():
     out = vs[0]
     for u in vs[1:]: out = p.op("mul", u, out)
     with pytest.raises(ValueError, match="more than|at most"): p.build(out)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_scratch_of_rows_with_regions(hd):
+  # rows with first keys of their own: parts chosen by the caller keep the packed tiles' partial sums (a tile 16 pairs,
+  # 32 + 16 hd floats a part), the library's own plan fits the 8 MiB of bt_attention_noalloc at every size
+  from baretile_amd import _lib
+  def scratch(kvh, rep, rows, keys, parts, fmt):
+    args = _lib.AttentionArgs(4096, 4096, 4096, 4096, 4096, rows * hd, hd, keys * hd, hd, keys * hd, hd, rows * hd, hd, rows,
+                              kvh * rep, rep, rows, keys, hd, 0, parts, 0, 0, 0, 4096, rows, fmt, 0, 4096, 4096)
+    need = ctypes.c_uint64()
+    _lib.call("attention_scratch", ctypes.byref(args), ctypes.byref(need))
+    return need.value
+  assert scratch(8, 2, 32, 32 * 512, 8, _lib.BF16) == 8 * 4 * 8 * (32 + 16 * hd) * 4
+  for kvh in (1, 2, 3, 8, 10, 40, 170, 341, 512, 4000):
+    for rep in (1, 4, 17):
+      for rows in (2, 8, 31, 32):
+        for keys in (100, 512, 1000, 4096):
+          for fmt in (_lib.BF16, _lib.BFP8): assert scratch(kvh, rep, rows, keys * rows, 0, fmt) <= 8 << 20
