@@ -328,10 +328,11 @@ def layer(x, p, c, rot, places, cache, rows, firsts=None):
 
 def chain_fits(x, norm, c, ps):
   """Whether the blocks ps can each end in the next step's norm (chained_layer): an fp32 stream of one matrix, bf16
-  norms, SwiGLU as the product's epilogue."""
-  return (x.dtype == "fp32" and x.batch == 1 and len(x.shape) <= 3 and norm.dtype == "bf16" and c.dim % 32 == 0 and
-          all(p["input_layernorm"].dtype == p["post_attention_layernorm"].dtype == "bf16" and p["down_proj"].rows % 16 == 0
-              for p in ps))
+  norms stored whole, SwiGLU as the product's epilogue."""
+  norms = [norm] + [p[n] for p in ps for n in ("input_layernorm", "post_attention_layernorm")]
+  return (x.dtype == "fp32" and x.batch == 1 and len(x.shape) <= 3 and c.dim % 32 == 0 and
+          all(w.dtype == "bf16" and w.batch * w.rows * w.cols == c.dim and w._contiguous() for w in norms) and
+          all(p["down_proj"].rows % 16 == 0 for p in ps))
 
 
 def chained_layer(x, h, p, c, rot, places, cache, rows, firsts, then):
