@@ -645,13 +645,13 @@ __global__ void __launch_bounds__(256) attention_combine_kernel(const bt_attenti
     float m[TURN], l[TURN], o[TURN];
 #pragma unroll
     for (int j = 0; j < TURN; j++) {
-      const float *q = src + (int64_t)min(p0 + j, parts - 1) * PF;  // a part past the last is read and left out
+      const float *q = src + (int64_t)min(p0 + j, parts - 1) * PF;  // past the last part it is read again and left out
       m[j] = gload(q + pi), l[j] = gload(q + 16 + pi), o[j] = gload(q + 32 + pi * HD + col);
     }
     float top = M;
 #pragma unroll
     for (int j = 0; j < TURN; j++) {
-      if (p0 + j >= parts) m[j] = -__builtin_inff();
+      if (p0 + j >= parts) m[j] = -__builtin_inff(), l[j] = o[j] = 0.0f;  // (0, not only weighed 0: o may be infinite)
       top = fmaxf(top, m[j]);
     }
     const float keep = M == top ? 1.0f : __expf(M - top);

@@ -800,6 +800,19 @@ def test_attention_parts_in_turns(rt, hd, keys, window, parts):
   assert np.allclose(got, ops.attention(q, k, v, places[..., None], window, 3), rtol=0.011, atol=0.011)
 
 
+# an infinite value in the last part: the turn's places past the last part add nothing to it (not 0 * inf)
+@pytest.mark.parametrize("hd,keys,parts", [(64, 300, 3), (128, 1100, 5), (64, 2560, 20)])
+def test_attention_parts_with_an_infinite_value(rt, hd, keys, parts):
+  rng = np.random.default_rng(keys)
+  q = B.bf16(rng.normal(0, 1, (6, 1, hd)) / np.sqrt(hd))
+  k, v = (B.bf16(rng.normal(0, 1, (2, keys, hd))) for _ in range(2))
+  places = np.full((1, 1), keys - 1)
+  want = ops.attention(q, k, v, places[..., None], 0, 3)
+  v[0, keys - 2, 7], v[1, 3, 11] = np.inf, -np.inf
+  want[:3, 0, 7], want[3:, 0, 11] = np.inf, -np.inf
+  assert np.allclose(attend(rt, q, k, v, places, 0, parts), want, rtol=0.011, atol=0.011)
+
+
 # slots' rows in tiles of their own, up to 32 rows, more than 16 heads a key head in two tiles a row; 33 rows packed
 @pytest.mark.parametrize("slots,rep,part,hd", [(2, 17, 70, 64), (32, 20, 40, 64), (32, 1, 129, 128), (33, 2, 64, 64), (3, 3, 1000, 64)])
 def test_attention_rows_in_tiles_of_their_own(rt, slots, rep, part, hd):
