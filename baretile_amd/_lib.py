@@ -45,7 +45,7 @@ class AttentionArgs(ctypes.Structure):
               ("q_sh", c_int64), ("q_sr", c_int64), ("k_sh", c_int64), ("k_sr", c_int64), ("v_sh", c_int64),
               ("v_sr", c_int64), ("o_sh", c_int64), ("o_sr", c_int64), ("places_sh", c_int64),
               ("heads", c_int32), ("rep", c_int32), ("rows", c_int32), ("keys", c_int32), ("head_dim", c_int32),
-              ("window", c_int32), ("parts", c_int32), ("pad_", c_int32), ("scratch", c_uint64),
+              ("window", c_int32), ("parts", c_int32), ("apart", c_int32), ("scratch", c_uint64),
               ("scratch_bytes", c_uint64), ("firsts", c_uint64), ("firsts_sh", c_int64), ("kv_fmt", c_int32),
               ("pad2_", c_int32), ("k_exps", c_uint64), ("v_exps", c_uint64)]
 

@@ -1103,10 +1103,13 @@ static int plan_attention(const bt_attention_args *a, AttnPlan *p) {
   if (a->firsts && a->firsts % 4) return fail(BT_EINVAL, "attention's firsts must be int32-aligned");
   if (a->firsts && a->firsts_sh != 0 && a->firsts_sh != a->rows) return fail(BT_EINVAL, "firsts' head stride is 0 or rows");
   const int kvh = a->heads / a->rep, np = a->rep * a->rows;
-  // rows with regions of their own: tiles by row while they are few (a decode step's slots, one token or a few each),
-  // where the parts are the library's to choose: its plans take 5.7 MB of scratch at most, while parts that a caller
-  // chose for packed tiles would outgrow bt_attention_noalloc's 8 MiB over 16 times the tiles
-  const bool by_row = a->firsts && a->rows > 1 && a->rows <= 32 && a->parts == 0;
+  // rows with regions of their own: tiles by row while they are few (a decode step's slots, one token each), where the
+  // parts are the library's to choose: its plans take 5.7 MB of scratch at most, while parts that a caller chose for
+  // packed tiles would outgrow bt_attention_noalloc's 8 MiB over 16 times the tiles. Only where the caller says that the
+  // regions are apart: rows that share one would each read it again, which packed tiles read once for 16 pairs, on parts
+  // planned for a region's share of the keys (24 rows of one head of 64 over 23136 shared keys 174.9 us by row, 18.5
+  // packed).
+  const bool by_row = a->apart && a->firsts && a->rows > 1 && a->rows <= 32 && a->parts == 0;
   const int per_row = (a->rep + 15) / 16;
   p->tiles = Tiles{by_row ? a->rows * per_row : (np + 15) / 16, by_row ? per_row : 0, make_fastdiv((uint32_t)a->rep),
                    make_fastdiv((uint32_t)per_row)};

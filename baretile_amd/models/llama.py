@@ -278,22 +278,23 @@ def rope(x, cos, sin, turn):
   return x * cos + (x @ turn) * sin
 
 
-def heads_out(h, p, c, rot, places, cache, rows, firsts=None):
+def heads_out(h, p, c, rot, places, cache, rows, firsts=None, apart=False):
   """One block's attention over its cache, up to the o product (llama.py:132-170): qkv, then RoPE with the new keys and
   values put into the cache at rows in one kernel (x cos + (x @ turn) sin, worked out in fp32 from the turn's pairs),
-  then one attention kernel from each token's place (and, with slots, from its slot's first row)."""
+  then one attention kernel from each token's place (and, with slots, from its slot's first row; apart: a token a slot)."""
   rep = c.heads // c.kv
   qkv = h.matmul(p["qkv_proj"])
   n = qkv.rows
   q = rope_into(qkv.reshape(n, qkv.cols), rot[0].reshape(n, rot[0].cols), rot[1].reshape(n, rot[1].cols), cache,
                 rows, c).split(c.heads)
   k, v = cache[:c.kv, :, :], cache[c.kv:, :, :]
-  return q.attend(k.repeat_interleave(rep), v.repeat_interleave(rep), places, firsts=firsts, merged=True)
+  return q.attend(k.repeat_interleave(rep), v.repeat_interleave(rep), places, firsts=firsts, merged=True,
+                  apart=apart)
 
 
-def attention(h, p, c, rot, places, cache, rows, firsts=None):
+def attention(h, p, c, rot, places, cache, rows, firsts=None, apart=False):
   """One block's attention over its cache (llama.py:132-172): heads_out, then the o product."""
-  return heads_out(h, p, c, rot, places, cache, rows, firsts).matmul(p["o_proj"], "fp32")
+  return heads_out(h, p, c, rot, places, cache, rows, firsts, apart).matmul(p["o_proj"], "fp32")
 
 
 def mlp(h, p):
@@ -320,9 +321,9 @@ def blocks(w, layers):
   return out
 
 
-def layer(x, p, c, rot, places, cache, rows, firsts=None):
+def layer(x, p, c, rot, places, cache, rows, firsts=None, apart=False):
   """Attention, then the MLP, each after an RMSNorm and added onto the fp32 stream in its own kernel (llama.py:106-130)."""
-  x = (x + attention(rms(x, p["input_layernorm"], c), p, c, rot, places, cache, rows, firsts)).realize()
+  x = (x + attention(rms(x, p["input_layernorm"], c), p, c, rot, places, cache, rows, firsts, apart)).realize()
   return (x + mlp(rms(x, p["post_attention_layernorm"], c), p)).realize()
 
 
@@ -335,12 +336,12 @@ def chain_fits(x, norm, c, ps):
           all(p["down_proj"].rows % 16 == 0 for p in ps))
 
 
-def chained_layer(x, h, p, c, rot, places, cache, rows, firsts, then):
+def chained_layer(x, h, p, c, rot, places, cache, rows, firsts, then, apart=False):
   """layer() with x's input norm h made already, ending in the norm the next step applies (weights `then`): (x, its h).
   The o and the down product each feed the residual add and the norm (matmul_residual_rms, which for a batched decode
   step's few rows sums a long product's parts in the norm's kernel: a launch less), with layer()'s results: a step of 30
   blocks, dim 576, 8 slots 1066 -> 995 us."""
-  o = heads_out(h, p, c, rot, places, cache, rows, firsts)
+  o = heads_out(h, p, c, rot, places, cache, rows, firsts, apart)
   x, h = o.matmul_residual_rms(p["o_proj"], x, p["post_attention_layernorm"], c.eps)
   return h.matmul_swiglu(p["gate_up_proj"]).matmul_residual_rms(p["down_proj"], x, then, c.eps)
 
@@ -431,7 +432,7 @@ def forward(ids, places, w, c, caches, every=False, slots=None):
     rot = (both[0:1, :], both[1:2, :], w["turn"])
   else:
     rot = (w["cos"].gather(places), w["sin"].gather(places), w["turn"])
-  firsts = None
+  firsts, apart = None, slots == n  # apart: a token a slot, so no two rows of attention share a region
   if not slots:
     rows, column = places, places.reshape(1, n, 1)
   else:
@@ -450,9 +451,9 @@ def forward(ids, places, w, c, caches, every=False, slots=None):
   if n <= 32 and ps and chain_fits(x, w["norm"], c, ps):
     norms = [p["input_layernorm"] for p in ps[1:]] + [w["norm"]]
     h = rms(x, ps[0]["input_layernorm"], c)
-    for l in range(c.layers): x, h = chained_layer(x, h, ps[l], c, rot, column, caches[l], rows, firsts, norms[l])
+    for l in range(c.layers): x, h = chained_layer(x, h, ps[l], c, rot, column, caches[l], rows, firsts, norms[l], apart)
   else:
-    for l in range(c.layers): x = layer(x, ps[l], c, rot, column, caches[l], rows, firsts)
+    for l in range(c.layers): x = layer(x, ps[l], c, rot, column, caches[l], rows, firsts, apart)
     h = rms(x, w["norm"], c)
   if not (every or slots) and n > 1: h = h[:, n - 1:n, :]  # the last token's row
   return h.matmul(w["embed.T"], "fp32")

@@ -851,11 +851,12 @@ class Tensor:
     return x, h
 
   # ---- attention, rows in and out
-  def attend(self, k, v, places, window=0, fidelity=None, parts=None, firsts=None, merged=False):
+  def attend(self, k, v, places, window=0, fidelity=None, parts=None, firsts=None, merged=False, apart=False):
     """softmax(self @ k^T + mask) @ v, with the mask from each query row's place (and window), in one kernel
     (tensor.py:797-841). k and v may be repeat views (grouped-query attention). RoPE scales q beforehand. firsts, an
     int32 column like places, raises each row's first visible key: sequences that share one cache in regions of their
-    own (llama.py:293-318's slots). merged writes the result as merge() of it, (rows, heads * width)."""
+    own (llama.py:293-318's slots); apart says that no two rows share a region and each is keys / rows long, so the call
+    may be planned by region. merged writes the result as merge() of it, (rows, heads * width)."""
     if len(self.shape) > 3: raise ValueError(f"attend takes three dimensions, not {self.shape}")
     if window < 0 or parts is not None and parts <= 0: raise ValueError("attention needs a nonnegative window and positive parts")
     if not (self.dtype == "bf16" and k.dtype == v.dtype and k.dtype in ("bf16", *BFP) and self.batch == k.batch == v.batch):
@@ -875,7 +876,7 @@ class Tensor:
       osh, osr = out.sb, out.sr
     args = _lib.AttentionArgs(q.addr, k.addr, v.addr, out.addr, places.addr, q.sb, q.sr, k.sb, k.sr, v.sb, v.sr,
                               osh, osr, q.rows if places.batch > 1 else 0, q.batch, rep, q.rows, k.rows, q.cols,
-                              window, parts or 0, 0, 0, 0)
+                              window, parts or 0, int(bool(apart)), 0, 0)
     if k.dtype in BFP:  # a block-float cache, read in place (test_kernels.py:2106-2132)
       (args.k_exps, args.k), (args.v_exps, args.v) = k._bfp_planes(), v._bfp_planes()
       args.kv_fmt = _lib.DTYPES[k.dtype]

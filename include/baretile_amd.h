@@ -287,7 +287,9 @@ int bt_matmul_residual_rms(bt_runtime *rt, const bt_operand *a, int b_fmt, uint6
  * is applied: baretile's RoPE pre-scales q (llama.py:210-216).
  *
  * firsts, when given, raises each row's first visible key (a batch of sequences with their own regions of one cache,
- * as the reference's slots use it, llama.py:293-318).
+ * as the reference's slots use it, llama.py:293-318). The library can't see whether rows share a region: apart says that
+ * none do, as where every sequence has one row, and lets a call of 2 to 32 rows plan by region. It changes the plan
+ * and the order of sums, never which keys a row sees.
  *
  * parts splits a decode step's keys (at most 64 query rows per key head: rep * rows <= 64) between that many blocks,
  * as attention_kernel's parts does; 0 picks a count from the shape. With more than one part the blocks write fp32
@@ -301,7 +303,8 @@ int bt_matmul_residual_rms(bt_runtime *rt, const bt_operand *a, int b_fmt, uint6
 typedef struct {
   uint64_t q, k, v, out, places;
   int64_t q_sh, q_sr, k_sh, k_sr, v_sh, v_sr, o_sh, o_sr, places_sh;
-  int32_t heads, rep, rows, keys, head_dim, window, parts, pad_;
+  int32_t heads, rep, rows, keys, head_dim, window, parts;
+  int32_t apart;      /* nonzero: firsts gives every row a region of keys / rows rows of its own (below) */
   uint64_t scratch, scratch_bytes;
   uint64_t firsts;    /* 0, or int32 with the first key each row sees (head stride firsts_sh: 0 or rows) */
   int64_t firsts_sh;

@@ -836,6 +836,32 @@ def test_attention_rows_in_tiles_of_their_own(rt, slots, rep, part, hd):
     assert np.allclose(got[:, r:r + 1], want, rtol=0.011, atol=0.011), r
 
 
+# rows said to be apart (tiles by row) and not (packed tiles): each row's own region, and two rows a region, which the
+# plan by row must get right as well
+@pytest.mark.parametrize("apart", [0, 1])
+@pytest.mark.parametrize("rows,share,rep,region,hd", [(2, 1, 17, 70, 64), (32, 1, 20, 40, 64), (32, 1, 1, 129, 128), (8, 1, 3, 512, 64),
+                                                      (8, 2, 3, 300, 64), (6, 6, 1, 1300, 128), (33, 3, 2, 64, 64)])
+def test_attention_rows_apart_or_sharing_regions(rt, rows, share, rep, region, hd, apart):
+  rng = np.random.default_rng(rows + rep + share)
+  E, kvh, keys = 2 * rep, 2, rows // share * region
+  q = B.bf16(rng.normal(0, 1, (E, rows, hd)) / np.sqrt(hd))
+  k, v = (B.bf16(rng.normal(0, 1, (kvh, keys, hd))) for _ in range(2))
+  firsts = np.broadcast_to(np.arange(rows) // share * region, (E, rows)).astype(np.int32)
+  places = firsts + rng.integers(0, region, rows, dtype=np.int32)
+  o = rt.dram_alloc(E * rows * hd * 2)
+  args = _lib.AttentionArgs(*(up(rt, B.bf16_bits(t)) for t in (q, k, v)), o, up(rt, places), rows * hd, hd, keys * hd, hd, keys * hd,
+                            hd, rows * hd, hd, rows, E, rep, rows, keys, hd, 0, 0, apart, 0, 0, up(rt, firsts.copy()), rows)
+  need = ctypes.c_uint64()
+  _lib.call("attention_scratch", ctypes.byref(args), ctypes.byref(need))
+  if need.value: args.scratch, args.scratch_bytes = rt.dram_alloc(need.value), need.value
+  rt.run("attention", "attention", ctypes.byref(args))
+  got = bits_to_float(down(rt, o, (E, rows, hd), np.uint16))
+  for r in range(rows):
+    own = slice(firsts[0, r], places[0, r] + 1)
+    want = ops.attention(q[:, r:r + 1], k[:, own], v[:, own], np.full((1, 1, 1), keys), 0, rep)
+    assert np.allclose(got[:, r:r + 1], want, rtol=0.011, atol=0.011), r
+
+
 def test_attention_rows_without_keys_are_zero(rt):
   # a place before the first key hides every key: p is zero and so is the output (kernels.py:823-826)
   rng = np.random.default_rng(5)
