@@ -402,6 +402,31 @@ def test_split_gemm_rows(rt, m, k, n):
     assert np.all(np.abs(out - silu) <= 2.0 ** -7 * np.abs(silu) + 1e-30), fmt  # one bf16 rounding, and fp32's in silu
 
 
+def test_scratch_of_rising_prompts(chip):
+  # prompts of rising lengths: the split GEMM's partial sums take 4 to 32 MB here, and the buffers outgrown on the way stay
+  # below the live one (at most twice the largest request): 128 MB in all
+  from baretile_amd.runtime import Runtime
+  rt = Runtime(chip)
+  def free():  # hipMemGetInfo of the HIP runtime that the library is linked to
+    mem = (ctypes.c_size_t * 2)()
+    assert ctypes.CDLL("libamdhip64.so.7").hipMemGetInfo(ctypes.byref(mem, 0), ctypes.byref(mem, 8)) == 0
+    return mem[0]
+  try:
+    k = n = 4096
+    a, out, cols = rt.dram_alloc(1000 * k * 2), rt.dram_alloc(1000 * n * 2), rt.dram_alloc(n // 16 * (k // 64) * 576)
+    for d, size in ((a, 1000 * k * 2), (cols, n // 16 * (k // 64) * 576)): rt.fill32(d, 0, size // 4)
+    def product(m):
+      rt.run("matmul", "matmul", ctypes.byref(_lib.operand(a, "bf16", 0, k, 1)), _lib.BFP4, cols, 1, 1, m, k, n, None,
+             ctypes.byref(_lib.operand(out, "bf16", 0, n, 1)))
+    product(33)  # loads the code
+    rt.wait()
+    before = free()
+    for m in range(34, 1001, 37): product(m)
+    rt.wait()
+    assert before - free() <= 128 << 20
+  finally: rt.close()
+
+
 GEMM_CASES = [(300, 1000, 520, "bf16"), (96, 576, 1536, "fp32"), (2048, 256, 8192, "bf16"), (2048, 192, 4096, "fp32"),
               (160, 320, 8192, "bf16"), (1000, 224, 4096, "bf16"), (520, 640, 1296, "fp32"), (2048, 320, 6144, "bf16"),
               (2048, 192, 6144, "fp32"), (2048, 128, 8192, "fp32")]
