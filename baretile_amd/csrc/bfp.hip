@@ -218,21 +218,22 @@ __device__ __forceinline__ int nibble_q(uint32_t w, int j) {  // the inverse: va
 // 16 rows, left the loads' lines mostly unused. The bound is HBM: 9/16 (bfp4) or 17/16 (bfp8) bytes a value each way.
 // LDS rows are 8 bytes longer than their runs, so that the 4 lane groups' rows, 8 apart, start 16 banks apart. WIDE: the
 // value plane starts on 8 bytes (it is byte addressed otherwise). 4096 x 14336 in bfp4: 53 us a block a tile, 25 us so
-// (2.9 TB/s).
-constexpr int RUNS_B = 16;  // runs a block
-template <int FMT, bool WIDE>
+// (2.9 TB/s). RUNS: the block's runs; 4, a tile a wave, where there would be fewer than 256 blocks of 16, each a chain of
+// 4 tiles a wave (bfp4, 15 x 1817: 3.9 us on 16 runs, 3.3 a block a tile, 2.4 on 4; 1024 x 2048 4.5, 5.1 and 2.8).
+constexpr int RUNS_B = 16;
+template <int FMT, bool WIDE, int RUNS>
 __global__ void __launch_bounds__(256) columns_kernel(const uint8_t *exps, const uint8_t *vals, int64_t rows,
                                                       uint32_t runs, uint32_t chunks, FastDiv groups, FastDiv chunks_d,
                                                       uint8_t *dst) {
-  constexpr int TB = FMT == BT_BFP8 ? 1088 : 576, RB = FMT == BT_BFP8 ? 16 : 8, S = RUNS_B * RB + 8;
+  constexpr int TB = FMT == BT_BFP8 ? 1088 : 576, RB = FMT == BT_BFP8 ? 16 : 8, S = RUNS * RB + 8;
   __shared__ __attribute__((aligned(16))) uint8_t lv[64 * S];
-  __shared__ __attribute__((aligned(16))) uint8_t le[RUNS_B][64];  // a tile's exponent bytes, as it stores them
-  const uint32_t q = fdiv(blockIdx.x, groups), b = fdiv(q, chunks_d), chunk = q - b * chunks, run0 = (blockIdx.x - q * groups.d) * RUNS_B;
+  __shared__ __attribute__((aligned(16))) uint8_t le[RUNS][64];  // a tile's exponent bytes, as it stores them
+  const uint32_t q = fdiv(blockIdx.x, groups), b = fdiv(q, chunks_d), chunk = q - b * chunks, run0 = (blockIdx.x - q * groups.d) * RUNS;
   const int t = threadIdx.x;
   const int64_t k0 = (int64_t)chunk * 64;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int row = t / RUNS_B + 16 * i, run = t % RUNS_B;
+  for (int i = 0; i < RUNS / 4; i++) {
+    const int row = t / RUNS + 256 / RUNS * i, run = t % RUNS;
     const bool in = k0 + row < rows && run0 + run < runs;
     const int64_t at = ((int64_t)b * rows + k0 + row) * runs + run0 + run;  // the run's number in the planes
     uint2 w[RB / 8];
@@ -252,7 +253,7 @@ __global__ void __launch_bounds__(256) columns_kernel(const uint8_t *exps, const
   __syncthreads();
   const int l = t & 63, n = l & 15;
 #pragma unroll
-  for (int i = 0; i < RUNS_B / 4; i++) {
+  for (int i = 0; i < RUNS / 4; i++) {
     const uint32_t run = (t >> 6) + 4 * i;
     if (run0 + run >= runs) break;  // uniform in the wave
     uint8_t *out = dst + ((int64_t)((int64_t)b * runs + run0 + run) * chunks + chunk) * TB;
@@ -294,6 +295,26 @@ __global__ void __launch_bounds__(64) bf16_columns_kernel(const uint16_t *src, i
   uint4 *out = (uint4 *)(dst + tile * 1024 + 16 * l);
   out[0] = make_uint4(w[0], w[1], w[2], w[3]);
   out[1] = make_uint4(w[4], w[5], w[6], w[7]);
+}
+
+// Readback a thread a value: finds it in its tile, decodes it exactly. For small results, where a block's chain of the
+// kernel below is longer than the byte loads it saves.
+template <int FMT>
+__global__ void __launch_bounds__(256) columns_value_kernel(const uint8_t *src, int64_t total, int64_t rows, int64_t cols,
+                                                            int64_t chunks, int64_t runs, uint16_t *dst) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= total) return;
+  const int64_t n = t % cols, k = t / cols % rows, b = t / cols / rows;
+  const int kk = (int)(k % 64), h = kk / 32, g = (kk % 32) / 8, j = kk % 8, l = g * 16 + (int)(n % 16);
+  const int64_t tile = (b * runs + n / 16) * chunks + k / 64;
+  if (FMT == BT_BF16) {
+    dst[t] = ((const uint16_t *)src)[tile * 1024 + 16 * l + 8 * h + j];
+    return;
+  }
+  const uint8_t *tp = src + tile * (FMT == BT_BFP8 ? 1088 : 576);
+  const uint32_t e = (tp[16 * g + 8 * h + j] + exp_bias<FMT>()) & 255u;
+  const int q = FMT == BT_BFP8 ? (int)(int8_t)tp[64 + 16 * l + 8 * h + j] : nibble_q(*(const uint32_t *)(tp + 64 + 8 * l + 4 * h), j) * 16;
+  dst[t] = (uint16_t)unpacked_bits(q, e);
 }
 
 // Readback of 16 neighbouring runs of one chunk a block: each of its 4 waves loads 4 tiles as contiguous stretches, every
@@ -452,16 +473,25 @@ int bt_bfp_columns(bt_runtime *rt, int fmt, uint64_t exps, uint64_t vals, int64_
   if (dst % 16) return fail(BT_EINVAL, "columns tiles must be 16-byte aligned");
   int64_t chunks = (rows + 63) / 64, nruns = (cols + 15) / 16, tiles = batch * nruns * chunks;
   if (tiles >= (1ll << 31)) return fail(BT_EINVAL, "too many tiles");
-  const int64_t groups = (nruns + RUNS_B - 1) / RUNS_B;
+  const bool few = batch * chunks * ((nruns + RUNS_B - 1) / RUNS_B) < 256;
+  const int per = few ? 4 : RUNS_B;
+  const int64_t groups = (nruns + per - 1) / per;
   const FastDiv gd = make_fastdiv((uint32_t)groups), cd = make_fastdiv((uint32_t)chunks);
+  const unsigned blocks = (unsigned)(batch * chunks * groups);
+#define BT_COLUMNS_N(FMT, WIDE, RUNS)                                                                                \
+  columns_kernel<FMT, WIDE, RUNS><<<blocks, 256, 0, r->stream>>>((const uint8_t *)exps, (const uint8_t *)vals, rows,   \
+                                                                 (uint32_t)nruns, (uint32_t)chunks, gd, cd, (uint8_t *)dst)
 #define BT_COLUMNS(FMT, WIDE)                                                                                        \
-  columns_kernel<FMT, WIDE><<<(unsigned)(batch * chunks * groups), 256, 0, r->stream>>>(                             \
-    (const uint8_t *)exps, (const uint8_t *)vals, rows, (uint32_t)nruns, (uint32_t)chunks, gd, cd, (uint8_t *)dst)
+  do {                                                                                                               \
+    if (few) BT_COLUMNS_N(FMT, WIDE, 4);                                                                             \
+    else BT_COLUMNS_N(FMT, WIDE, RUNS_B);                                                                            \
+  } while (0)
   if (fmt == BT_BFP8 && vals % 8 == 0) BT_COLUMNS(BT_BFP8, true);
   else if (fmt == BT_BFP8) BT_COLUMNS(BT_BFP8, false);
   else if (vals % 8 == 0) BT_COLUMNS(BT_BFP4, true);
   else BT_COLUMNS(BT_BFP4, false);
 #undef BT_COLUMNS
+#undef BT_COLUMNS_N
   BT_LAUNCHED("bfp_columns");
   return BT_OK;
 }
@@ -510,6 +540,19 @@ int bt_columns_unpack(bt_runtime *rt, int fmt, uint64_t src, int64_t batch, int6
   if (batch * nruns * chunks >= (1ll << 31)) return fail(BT_EINVAL, "too many tiles");
   const FastDiv gd = make_fastdiv((uint32_t)groups), cd = make_fastdiv((uint32_t)chunks);
   const bool wide = cols % 8 == 0 && dst % 16 == 0;
+  // a thread a value up to where both take the same: 1.5 million values of block floats and of rows stored a column a
+  // thread, half a million of bf16 in whole words (bfp4, a thread a value and in blocks: 60 x 204 2.4 and 9.7 us, 1024 x
+  // 1024 5.1 and 7.6, 1024 x 2048 8.7 and 7.8, 4096 x 4096 52 and 13; bf16, 300 x 2000 3.4 and 3.3, 1024 x 1024 4.6 and
+  // 3.2); also tiles that don't start on the blocks' 16-byte loads
+  const int64_t total = batch * rows * cols;
+  if (total < (fmt == BT_BF16 && wide ? 1 << 19 : 3 << 19) || src % 16) {
+    const unsigned blocks = blocks_for(total, 256);
+    if (fmt == BT_BF16) columns_value_kernel<BT_BF16><<<blocks, 256, 0, r->stream>>>((const uint8_t *)src, total, rows, cols, chunks, nruns, (uint16_t *)dst);
+    else if (fmt == BT_BFP8) columns_value_kernel<BT_BFP8><<<blocks, 256, 0, r->stream>>>((const uint8_t *)src, total, rows, cols, chunks, nruns, (uint16_t *)dst);
+    else columns_value_kernel<BT_BFP4><<<blocks, 256, 0, r->stream>>>((const uint8_t *)src, total, rows, cols, chunks, nruns, (uint16_t *)dst);
+    BT_LAUNCHED("columns_unpack");
+    return BT_OK;
+  }
 #define BT_UNPACK(FMT, WIDE)                                                                                         \
   columns_unpack_kernel<FMT, WIDE><<<(unsigned)(batch * chunks * groups), 256, 0, r->stream>>>(                      \
     (const uint8_t *)src, rows, cols, (uint32_t)nruns, (uint32_t)chunks, gd, cd, (uint16_t *)dst)

@@ -175,6 +175,28 @@ def test_block_floats_at_the_edges_of_blocks(rt, fmt, src, shape, lead, gap):
   assert np.array_equal(down(rt, out, (b, r, c), np.uint16), want)
 
 
+# results large enough for the readback in blocks of 16 runs (1.5 million values, half a million of bf16 in whole words)
+# and for re-laying 16 runs a block (256 blocks of them), whole rows and odd ones, and sizes just below; and tiles that
+# don't start on 16 bytes, which a thread a value reads
+@pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bfp4"])
+@pytest.mark.parametrize("shape", [(1, 1030, 4104), (1, 1025, 4101), (3, 129, 4066), (2, 500, 2000), (1, 512, 1016)])
+def test_large_columns_read_back(rt, fmt, shape):
+  b, r, c = shape
+  x = np.random.default_rng(r).normal(0, 1, shape).astype(np.float32)
+  if fmt == "bf16": cols, size, want = bf16_columns(rt, x), 2048, B.bf16_bits(x)
+  else:
+    cols, size = columns(rt, *pack(rt, x, fmt), fmt, b, r, c), 1088 if fmt == "bfp8" else 576
+    want = B.decode_fields(*B.bfp_fields(np.pad(B.bf16(x), ((0, 0), (0, 0), (0, -c % 16))), fmt), fmt)[..., :c]
+  size *= b * -(-r // 64) * -(-c // 16)
+  out = rt.dram_alloc(b * r * c * 2)
+  shifted = rt.dram_alloc(size + 4) + 4
+  rt.copy(shifted, cols, size)
+  for tiles in (cols, shifted):
+    rt.fill32(out, 0, b * r * c // 2)
+    rt.run("readback", "columns_unpack", _lib.DTYPES[fmt], tiles, b, r, c, out)
+    assert np.array_equal(down(rt, out, shape, np.uint16), want)
+
+
 # ---- matmul -----------------------------------------------------------------------------------------------------
 
 def test_matmul_exact(rt):
