@@ -2911,9 +2911,15 @@ static void launch_gemm_dt(const MatmulArgs &args, hipStream_t s) {
   }
   {
     bt_operand res{};
-    const bool fits = args.m > 128 && (FMT == BT_BF16 ? args.k % 32 == 0
-                                                      : (args.m >= 512 || (int64_t)((args.m + 127) / 128) * ((args.n + 255) / 256) >= 64) &&
-                                                          args.k % 64 == 0 && (int64_t)args.chunks * args.nruns * Tile<FMT>::bytes < (1ll << 32));
+    // block-float B of fewer than 512 rows: bf16 out stays on gemm2 while its 128 x 128 blocks fill at most one round of
+    // the CUs (468 x 192 x 7040 bfp8 8.4 us there, 13.8 here; 336 x 832 x 6208 22.1 and 24.3; 374 x 1344 x 10560 bfp4 28.6 and
+    // 29.9) and comes here when they take two (340 x 704 x 13008 bfp8 44 and 31); fp32 out, whose tiles gemm2 stores
+    // slowly, from 64 blocks of 128 x 256 (411 x 512 x 4288 30 and 21)
+    const bool rows = FMT == BT_BF16 || args.m >= 512 ||
+                      (DT == BT_BF16 ? (int64_t)((args.m + 127) / 128) * ((args.n + 127) / 128) > 256
+                                     : (int64_t)((args.m + 127) / 128) * ((args.n + 255) / 256) >= 64);
+    const bool fits = args.m > 128 && rows && (FMT == BT_BF16 ? args.k % 32 == 0
+                                                              : args.k % 64 == 0 && (int64_t)args.chunks * args.nruns * Tile<FMT>::bytes < (1ll << 32));
     if (fits && (DT == BT_BF16 || residual_program(args, &res))) {
       const Gemm3Shape sh = gemm3_shape(args, FMT == BT_BFP4);
       const int mb = (args.m + sh.bm - 1) / sh.bm, nb = (args.n + sh.bn - 1) / sh.bn;

@@ -424,6 +424,18 @@ def test_split_gemm_rows(rt, m, k, n):
     assert np.all(np.abs(out - silu) <= 2.0 ** -7 * np.abs(silu) + 1e-30), fmt  # one bf16 rounding, and fp32's in silu
 
 
+# either side of the lines between the GEMMs: block floats of fewer than 512 rows at one round of 128 x 128 blocks and over
+# it; all give the 64-row products' bits
+@pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
+@pytest.mark.parametrize("m,k,n,out", [(500, 192, 8192, "bf16"), (500, 192, 8208, "bf16"), (257, 128, 5376, "fp32"), (257, 128, 5380, "fp32")])
+def test_gemm_at_the_lines_between_kernels(rt, fmt, m, k, n, out):
+  rng = np.random.default_rng(m + n)
+  x, w = rng.normal(0, 1, (m, k)), rng.normal(0, 0.05, (k, n)).astype(np.float32)
+  cols = columns(rt, *pack(rt, w, fmt), fmt, 1, k, n)
+  sliced = np.concatenate([matmul(rt, x[i:i + 64], cols, fmt, 1, n, out=out)[0] for i in range(0, m, 64)])
+  assert np.array_equal(matmul(rt, x, cols, fmt, 1, n, out=out)[0], sliced)
+
+
 def test_scratch_of_rising_prompts(chip):
   # prompts of rising lengths: the split GEMM's partial sums take 4 to 32 MB here, and the buffers outgrown on the way stay
   # below the live one (at most twice the largest request): 128 MB in all
