@@ -3025,10 +3025,11 @@ extern "C" int bt_matmul(bt_runtime *rt, const bt_operand *a, int b_fmt, uint64_
   }
   // A prefill-sized product whose block-float B the GEMM doesn't read as stored (K not in whole chunks), or reads more
   // slowly than bf16 (bfp8 over many 128-row blocks, each decoding B again: 2048 x 4096 x 4096 88 us, 85 unpacked first,
-  // while 256-row blocks gain, 481 us against 534 at 28672 columns): B unpacked once into bf16 tiles in the runtime's
-  // scratch (the same values bit for bit), then the bf16 GEMM.
+  // while 256-row blocks gain, 481 us against 534 at 28672 columns; fp32 out, whose stores hide less of the decoding, from
+  // 512 rows: 552 x 320 x 1632 17.0 and 14.8, 960 x 1088 x 2560 30.8 and 28.7): B unpacked once into bf16 tiles in the
+  // runtime's scratch (the same values bit for bit), then the bf16 GEMM.
   const bool bf16_out = out->dtype == BT_BF16 && (!epilogue || epilogue->dtype != BT_FP32);
-  if (b_fmt != BT_BF16 && (k % 64 != 0 || (b_fmt == BT_BFP8 && m >= 1024 && gemm3_shape(args, false).bm == 128)) &&
+  if (b_fmt != BT_BF16 && (k % 64 != 0 || (b_fmt == BT_BFP8 && m >= (bf16_out ? 1024 : 512) && gemm3_shape(args, false).bm == 128)) &&
       (bf16_out || residual_program(args, nullptr)) &&
       m >= 512 && k % 32 == 0 && a->sc == 1 && (int64_t)args.chunks * args.nruns * 2048 < (1ll << 32)) {
     const int64_t tiles = (int64_t)args.chunks * args.nruns * (b_batch > 1 ? b_batch : 1);

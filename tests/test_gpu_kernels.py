@@ -425,9 +425,10 @@ def test_split_gemm_rows(rt, m, k, n):
 
 
 # either side of the lines between the GEMMs: block floats of fewer than 512 rows at one round of 128 x 128 blocks and over
-# it; all give the 64-row products' bits
+# it, and 511 and 512 rows, where fp32 out of bfp8 is unpacked first; all give the 64-row products' bits
 @pytest.mark.parametrize("fmt", ["bfp8", "bfp4"])
-@pytest.mark.parametrize("m,k,n,out", [(500, 192, 8192, "bf16"), (500, 192, 8208, "bf16"), (257, 128, 5376, "fp32"), (257, 128, 5380, "fp32")])
+@pytest.mark.parametrize("m,k,n,out", [(500, 192, 8192, "bf16"), (500, 192, 8208, "bf16"), (257, 128, 5376, "fp32"), (257, 128, 5380, "fp32"),
+                                       (511, 320, 1632, "fp32"), (512, 320, 1632, "fp32"), (512, 320, 1632, "bf16")])
 def test_gemm_at_the_lines_between_kernels(rt, fmt, m, k, n, out):
   rng = np.random.default_rng(m + n)
   x, w = rng.normal(0, 1, (m, k)), rng.normal(0, 0.05, (k, n)).astype(np.float32)
