@@ -437,6 +437,37 @@ def test_gemm_at_the_lines_between_kernels(rt, fmt, m, k, n, out):
   assert np.array_equal(matmul(rt, x, cols, fmt, 1, n, out=out)[0], sliced)
 
 
+# SiLU x up on 128- and 256-row blocks, B as stored or unpacked first, whichever a format's rule takes: the bits of the
+# bf16 product of its values; recorded where the scratch can't grow, B is read as stored
+@pytest.mark.parametrize("m,k,n", [(1540, 128, 21888), (1432, 64, 12896)])
+def test_swiglu_blocks_give_the_same_bits(chip, m, k, n):
+  from baretile_amd.runtime import Runtime
+  rt = Runtime(chip)
+  try:
+    rng = np.random.default_rng(m)
+    x, w = up(rt, B.bf16_bits(rng.normal(0, 1, (m, k)))), rng.normal(0, 0.05, (k, n)).astype(np.float32)
+    exps, vals = pack(rt, w, "bfp8")
+    cols, same = columns(rt, exps, vals, "bfp8", 1, k, n), bf16_columns(rt, bfp_values(w, "bfp8"))
+    outs = [rt.dram_alloc(m * n) for _ in range(3)]
+    def swiglu(fmt, b, out):
+      rt.run("swiglu", "matmul_swiglu", ctypes.byref(_lib.operand(x, "bf16", m * k, k, 1)), _lib.DTYPES[fmt], b, m, k, n,
+             ctypes.byref(_lib.operand(out, "bf16", m * n // 2, n // 2, 1)))
+    g = ctypes.c_void_p()
+    _lib.call("graph_begin", rt.handle)
+    swiglu("bfp8", cols, outs[2])
+    _lib.call("graph_end", rt.handle, ctypes.byref(g))
+    swiglu("bfp8", cols, outs[0])
+    swiglu("bf16", same, outs[1])
+    want = down(rt, outs[1], (m, n // 2), np.uint16)
+    assert np.array_equal(down(rt, outs[0], (m, n // 2), np.uint16), want)
+    for _ in range(2):
+      rt.fill32(outs[2], 0, m * n // 4)
+      _lib.call("graph_launch", rt.handle, g)
+      assert np.array_equal(down(rt, outs[2], (m, n // 2), np.uint16), want)
+    _lib.call("graph_destroy", g)
+  finally: rt.close()
+
+
 def test_scratch_of_rising_prompts(chip):
   # prompts of rising lengths: the split GEMM's partial sums take 4 to 32 MB here, and the buffers outgrown on the way stay
   # below the live one (at most twice the largest request): 128 MB in all
