@@ -3217,12 +3217,19 @@ extern "C" int bt_matmul_swiglu(bt_runtime *rt, const bt_operand *a, int b_fmt, 
     BT_LAUNCHED("matmul_swiglu");
     return BT_OK;
   }
-  // block-float B with K in whole chunks: read as it is stored by the GEMM itself; otherwise unpacked once into bf16
-  // tiles in the runtime's scratch
-  if (b_fmt != BT_BF16 && k % 64 != 0) {
+  // block-float B with K in whole chunks: read as it is stored by the GEMM itself, but for bfp8 against a long K in one
+  // round of 256-row blocks with few columns, where the decoding (3.6 us a thousand rows of K) costs more than the
+  // unpacking (3 us and 0.7 a million values; 2390 x 3776 x 3584 110 us as stored, 106 unpacked first; 1516 x 3712 x 10592
+  // 114 and 128). Otherwise unpacked once into bf16 tiles in the runtime's scratch
+  const bool decode_long = b_fmt == BT_BFP8 && mb * nb > 128 && mb * nb <= 256 && 3600 * k > 3000000 + 680 * k * n / 1000;
+  void *bt16 = nullptr;
+  if (b_fmt != BT_BF16 && (k % 64 != 0 || decode_long)) {
     const int64_t tiles = (int64_t)args.chunks * args.nruns;
-    void *bt16 = runtime_scratch(r, (size_t)tiles * 2048);
-    if (!bt16) return fail(BT_ESTATE, "matmul_swiglu: no scratch for B's bf16 tiles (inside a capture, or out of memory)");
+    bt16 = runtime_scratch(r, (size_t)tiles * 2048);
+    if (!bt16 && k % 64 != 0) return fail(BT_ESTATE, "matmul_swiglu: no scratch for B's bf16 tiles (inside a capture, or out of memory)");
+  }
+  if (bt16) {
+    const int64_t tiles = (int64_t)args.chunks * args.nruns;
     const unsigned blocks = (unsigned)((tiles + 3) / 4);
     if (b_fmt == BT_BFP8) tiles_bf16_kernel<BT_BFP8><<<blocks, 256, 0, r->stream>>>(args.b, (uint8_t *)bt16, tiles);
     else tiles_bf16_kernel<BT_BFP4><<<blocks, 256, 0, r->stream>>>(args.b, (uint8_t *)bt16, tiles);

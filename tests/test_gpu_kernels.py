@@ -439,7 +439,7 @@ def test_gemm_at_the_lines_between_kernels(rt, fmt, m, k, n, out):
 
 # SiLU x up on 128- and 256-row blocks, B as stored or unpacked first, whichever a format's rule takes: the bits of the
 # bf16 product of its values; recorded where the scratch can't grow, B is read as stored
-@pytest.mark.parametrize("m,k,n", [(1540, 128, 21888), (1432, 64, 12896)])
+@pytest.mark.parametrize("m,k,n", [(4100, 3392, 1984), (1540, 128, 21888), (1432, 64, 12896)])
 def test_swiglu_blocks_give_the_same_bits(chip, m, k, n):
   from baretile_amd.runtime import Runtime
   rt = Runtime(chip)
