@@ -227,7 +227,7 @@ struct OneInput {
   int op;      // -1: another kind of program
   bool a, b;   // whether the operand is the product (else the input)
 };
-__device__ __forceinline__ OneInput one_input(const bt_program &p, int n_inst) {
+__host__ __device__ __forceinline__ OneInput one_input(const bt_program &p, int n_inst) {
   const bt_inst ld = p.inst[0], in = p.inst[1];
   const bool ok = n_inst == 2 && p.n_inputs == 1 && ld.op == BT_OP_LOAD && ld.dst != 0 && in.op >= BT_OP_ADD &&
                   in.op <= BT_OP_CMPEQ && p.result == in.dst && (in.a == 0 || in.a == ld.dst) && (in.b == 0 || in.b == ld.dst);
@@ -236,8 +236,9 @@ __device__ __forceinline__ OneInput one_input(const bt_program &p, int n_inst) {
 
 // The epilogue of both kernels: lane holds rows 4g .. 4g+3 of the 16 x 16 tile at (mt, run), column col.
 // ONE: a batch of one, so the output's matrix is matrix 0. PROG: 1 runs the epilogue program, 0 stores plainly, -1
-// reads which from the arguments.
-template <int DT, bool INL = false, bool ONE = false, int PROG = -1>
+// reads which from the arguments. ONE_IN: 1 looks whether the program is one operation on the product and an input, 0
+// leaves such programs to the evaluator, 2 takes the program for one.
+template <int DT, bool INL = false, bool ONE = false, int PROG = -1, int ONE_IN = 1>
 __device__ __forceinline__ void store_tile(const MatmulArgs &args, const Head &h, const f32x4 &acc, int b, int mt,
                                            int run, int g, int col) {
   const int n = run * 16 + col;
@@ -261,7 +262,7 @@ __device__ __forceinline__ void store_tile(const MatmulArgs &args, const Head &h
   // the lane's 4 values, without the evaluator's register file (its other registers read as 0 until written); the
   // same arithmetic, so the same bits
   const bt_inst in0 = args.prog.inst[0];
-  if (h.n_inst == 1 && args.prog.n_inputs == 0 && args.prog.result == in0.dst && in0.op != BT_OP_LOAD &&
+  if (ONE_IN != 2 && h.n_inst == 1 && args.prog.n_inputs == 0 && args.prog.result == in0.dst && in0.op != BT_OP_LOAD &&
       in0.op != BT_OP_CONST && in0.op != BT_OP_MOV && in0.op != BT_OP_WHERE) {
     Vals<4> va, vb;
 #pragma unroll
@@ -280,8 +281,8 @@ __device__ __forceinline__ void store_tile(const MatmulArgs &args, const Head &h
   }
   // one operation on the product and an input: the lane's 4 values of the input loaded together (3 rows of 2048 x 2048
   // bfp8 with a residual 10.8 -> 7.7 us, 40 rows 20.4 -> 13.7)
-  const OneInput one = one_input(args.prog, h.n_inst);
-  if (one.op >= 0) {
+  const OneInput one = ONE_IN ? one_input(args.prog, h.n_inst) : OneInput{-1, false, false};
+  if (ONE_IN == 2 || one.op >= 0) {
     Vals<4> r, va, vb;
 #pragma unroll
     for (int i = 0; i < 4; i++) r.x[i] = load_operand<DT>(args.prog.in[0], ONE ? 0 : b, min(mt * 16 + 4 * g + i, m - 1), n);
@@ -645,13 +646,15 @@ __global__ void __launch_bounds__(256) gemv_x_kernel(const XArgs h) {
 // waited for behind the values. The weights are read with the streaming cache policy (read once): 6.18 and 8.61.
 // A's rows in LDS are G chunks long, so mapping a thread's pieces of A to rows divides by a constant (about 75
 // fewer VALU instructions a wave than a division by the product's K): 5.92 and 8.35.
-// MODE: 0 stores plainly, 1 runs the epilogue program, 2 adds an fp32 residual (res, fp32 out) whose values are loaded
+// MODE: 0 stores plainly, 1 runs the epilogue program, 4 one that is one operation on the product and an input (its own
+// mode: in one kernel with the evaluator the two took 95 registers, four waves a SIMD, not six, and products of more waves
+// than that lost, 154 x 384 x 7520 bfp4 with ReLU 6.2 -> 7.0 us), 2 adds an fp32 residual (res, fp32 out) whose values are loaded
 // with A, ahead of the weights (8 rows of 576 x 576 bfp8 8.5 us through the evaluator, 4.9 so, 4.8 plain), 3 is SiLU x
 // up (B gate then up columns, bf16 out): the block's first two waves take gate runs, the others the up runs of the same
 // columns, which reach the gate waves through LDS (8 rows of 576 x 3072 bfp8 7.5 us on skinny2_kernel, 5.1 so).
 template <int FMT, int DT, int MT, int NRW, int G, int MODE>
 __global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args, const bt_operand res) {
-  static_assert(MODE < 2 || (MT == 1 && NRW == 1), "the residual and SiLU x up modes take a tile a wave");
+  static_assert(MODE < 2 || MODE == 4 || (MT == 1 && NRW == 1), "the residual and SiLU x up modes take a tile a wave");
   constexpr int TB = Tile<FMT>::bytes, R = (G + 3) / 4;  // R: rounds of 4 chunks (bfp4)
   extern __shared__ __attribute__((aligned(16))) uint16_t la[];  // A: 16 MT rows, kp halfwords apart
   // bfp4: each chunk's exponents as gaps placed in the bf16 exponent field (place_gaps), 128 bytes a chunk a run
@@ -792,10 +795,10 @@ __global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args, 
 #pragma unroll
       for (int i = 0; i < 4; i++) acc[0][i] += rv[i];
     }
-    if constexpr (MODE == 1) {
+    if constexpr (MODE == 1 || MODE == 4) {
 #pragma unroll
       for (int t = 0; t < MT; t++)
-        store_tile<DT, false, true, 1>(args, h, acc[t], 0, (int)blockIdx.y * MT + t, run0 + r, g, col);
+        store_tile<DT, false, true, 1, MODE == 4 ? 2 : 0>(args, h, acc[t], 0, (int)blockIdx.y * MT + t, run0 + r, g, col);
     } else {
       // without a program the output is plain (bf16 or fp32, contiguous rows, byte offsets within 32 bits: the host
       // checks): a buffer store a value, as the lean GEMV stores
@@ -2523,6 +2526,7 @@ static void launch_lds_g(const MatmulArgs &args, unsigned blocks, hipStream_t s)
   bt_operand res{};
   if (DT == BT_FP32 && plain_out(args) && residual_program(args, &res) && res.ptr && res.rep == 1 && res.cyc == 0)
     skinny_lds_kernel<FMT, BT_FP32, MT, NRW, G, 2><<<grid, 256, lds, s>>>(args, res);
+  else if (args.n_inst && one_input(args.prog, args.n_inst).op >= 0) skinny_lds_kernel<FMT, DT, MT, NRW, G, 4><<<grid, 256, lds, s>>>(args, res);
   else if (args.n_inst) skinny_lds_kernel<FMT, DT, MT, NRW, G, 1><<<grid, 256, lds, s>>>(args, res);
   else skinny_lds_kernel<FMT, DT, MT, NRW, G, 0><<<grid, 256, lds, s>>>(args, res);
 }
