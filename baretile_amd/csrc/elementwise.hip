@@ -71,7 +71,7 @@ __global__ void __launch_bounds__(256) elementwise_row_kernel(const SegProgram p
     const int64_t c0 = (int64_t)sg * SEG;
     const int n = (int)min((int64_t)SEG, cols - c0);
     SegInputs x;
-    fetch_seg<DT, FULL>(p, bb, r, c0, n, x);
+    fetch_seg<DT, FULL, ROWS>(p, bb, r, c0, n, x);
     const seg_t y = run_seg<DT, FULL>(p, x, rv);
     const uint32_t io[SEG] = {y[0], y[1], y[2], y[3], y[4], y[5], y[6], y[7]};
     store_segment<DT>(out, bb, r, c0, n, io);
@@ -209,7 +209,7 @@ __global__ void __launch_bounds__(WPO > 4 ? 64 * WPO : 256) reduce_seg_kernel(co
     uint32_t io[SEG] = {};
     if constexpr (std::is_same_v<P, SegProgram>) {
       SegInputs x;
-      fetch_seg<DT, FULL>(prog, b, r, c0, n, x);
+      fetch_seg<DT, FULL, true>(prog, b, r, c0, n, x);
       const seg_t y = run_seg<DT, FULL>(prog, x, rv);
 #pragma unroll
       for (int v = 0; v < SEG; v++) io[v] = y[v];
@@ -376,7 +376,7 @@ int bt_elementwise(bt_runtime *rt, const bt_program *prog, int64_t batch, int64_
       const FastDiv fs = make_fastdiv((uint32_t)segs);
       const unsigned blocks = (unsigned)((nseg + 255) / 256);
       SegProgram sp;
-      if (sp.make(*prog, batch, rows, cols)) {
+      if (sp.make(*prog, batch, rows)) {
         if (prog->dtype == BT_BF16) launch_rows<BT_BF16>(sp, batch, rows, cols, *out, r->stream);
         else if (prog->dtype == BT_FP32) launch_rows<BT_FP32>(sp, batch, rows, cols, *out, r->stream);
         else launch_rows<BT_INT32>(sp, batch, rows, cols, *out, r->stream);
@@ -439,7 +439,7 @@ int bt_reduce(bt_runtime *rt, const bt_program *prog, int kind, int axis, int64_
     else reduce_seg_kernel<BT_INT32, WPO, P, FULL><<<blocks, threads, 0, r->stream>>>(p, kind, batch, rows, cols, *out); \
   } while (0)
     SegProgram sp;
-    if (!sp.make(*prog, batch, rows, cols)) {
+    if (!sp.make(*prog, batch, rows)) {
       if (outs < 2048) BT_RSEG(4, bt_program, true, *prog);  // (16 waves would leave each lane too few registers)
       else BT_RSEG(1, bt_program, true, *prog);
     } else {

@@ -38,13 +38,13 @@ struct RowInst {
 struct SegProgram {
   int32_t n_row, n_vec, n_in, n_tmp;
   uint8_t in_at[SEG_IN];  // the operand behind each input slot
-  uint8_t wide[SEG_IN];   // its segments are whole and start on 16 bytes
+  uint8_t wide[SEG_IN];   // its columns are contiguous and 1: every row starts on 16 bytes, 2 (4-byte values): some may
   RowInst row[BT_MAX_INST];
   SegInst vec[BT_MAX_INST + 1];
   bt_operand in[BT_MAX_INPUTS];
 
-  // Translates prog for segments of [batch, rows, cols]; false when it doesn't fit the slots.
-  inline bool make(const bt_program &prog, int64_t batch, int64_t rows, int64_t cols);
+  // Translates prog for segments of rows of [batch, rows, cols]; false when it doesn't fit the slots.
+  inline bool make(const bt_program &prog, int64_t batch, int64_t rows);
 };
 
 static inline int op_arity(int op) {
@@ -67,7 +67,7 @@ static inline int take_slot(uint32_t &used, int n) {
   return -1;
 }
 
-inline bool SegProgram::make(const bt_program &prog, int64_t batch, int64_t rows, int64_t cols) {
+inline bool SegProgram::make(const bt_program &prog, int64_t batch, int64_t rows) {
   // every instruction as a value of its own: its operands are the values last written to the registers it names
   struct Value {
     bool row, in, need;
@@ -188,7 +188,7 @@ inline bool SegProgram::make(const bt_program &prog, int64_t batch, int64_t rows
     uint64_t starts = o.ptr;
     if (rows > 1) starts |= (uint64_t)o.sr * size;
     if (batch > 1) starts |= (uint64_t)o.sb * size;
-    wide[k] = o.sc == 1 && cols % SEG == 0 && starts % 16 == 0;
+    wide[k] = o.sc != 1 ? 0 : starts % 16 == 0 ? 1 : size == 4 ? 2 : 0;
   }
   return true;
 }
@@ -293,20 +293,21 @@ __device__ __forceinline__ seg_t run_row(const SegProgram &p, int64_t b, int64_t
 }
 
 // The segment's 8 values of one input as they are stored: wide bf16 as 4 words of two values, anything else a value
-// each, 0 past the row's end.
+// each, 0 past the row's end (n values to it). Wide segments but a row's last take 16-byte loads.
 __device__ __forceinline__ seg_t seg_load(const bt_operand &o, bool wide, int64_t b, int64_t r, int64_t c0, int n) {
   const int64_t at = operand_matrix(o, b) * o.sb + r * o.sr + c0 * o.sc;
   if (o.dtype == BT_BF16) {
     const uint16_t *s = (const uint16_t *)o.ptr + at;
-    if (wide) {
+    if (wide && n == SEG) {
       const words4 w = gload((const words4 *)s);
       return seg_t{w[0], w[1], w[2], w[3], 0u, 0u, 0u, 0u};
     }
     auto get = [&](int v) -> uint32_t { return v < n ? gload(s + v * o.sc) : 0u; };
-    return seg_t{get(0), get(1), get(2), get(3), get(4), get(5), get(6), get(7)};
+    const seg_t x = seg_t{get(0), get(1), get(2), get(3), get(4), get(5), get(6), get(7)};
+    return wide ? seg_t{x[0] | x[1] << 16, x[2] | x[3] << 16, x[4] | x[5] << 16, x[6] | x[7] << 16, 0u, 0u, 0u, 0u} : x;
   }
   const uint32_t *s = (const uint32_t *)o.ptr + at;
-  if (wide) {
+  if (wide && n == SEG) {
     const words4 w0 = gload((const words4 *)s), w1 = gload((const words4 *)s + 1);
     return seg_t{w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
   }
@@ -323,6 +324,16 @@ __device__ __forceinline__ seg_t seg_convert(const seg_t &x, int dtype, bool wid
   return seg_map(x, [&](uint32_t w) { return convert_raw<DT>(w, dtype); });
 }
 
+// Whether input k of row (b, r) is wide. ROWS: a wave's lanes share the row, so that where only some rows start on 16
+// bytes (of rows of 1643 floats every fourth) this row's start counts, in a uniform branch; otherwise every row's. (With whole
+// segments of aligned rows alone taking wide loads, 423 x 3628 int32 x + y took 12.6 us, 3 x 40 x 7898 fp32 9.5; so 7.3 and
+// 8.9; 11.2 and 9.0 on the general evaluator.)
+template <bool ROWS>
+__device__ __forceinline__ bool seg_wide(const SegProgram &p, int k, int64_t b, int64_t r) {
+  if (p.wide[k] != 2) return p.wide[k];
+  const bt_operand &o = p.in[p.in_at[k]];
+  return ROWS && (o.ptr + 4 * (uint64_t)(operand_matrix(o, b) * o.sb + r * o.sr)) % 16 == 0;
+}
 // The program's inputs over a segment, in its dtype, every load issued before the first is converted. FULL: a program
 // of any number of inputs and stored values; otherwise three inputs at most and no stored value, on fewer registers
 // (106 against 162: four waves a SIMD, not three).
@@ -331,17 +342,19 @@ struct SegInputs {
 };
 static_assert(SEG_IN == 4 && SEG_TMP == 4, "SegInputs and run_seg name four of each");
 inline bool seg_small(const SegProgram &p) { return p.n_in <= 3 && p.n_tmp == 0; }
-template <int DT, bool FULL>
+template <int DT, bool FULL, bool ROWS>
 __device__ __forceinline__ void fetch_seg(const SegProgram &p, int64_t b, int64_t r, int64_t c0, int n, SegInputs &i) {
+  const bool w0 = p.n_in > 0 && seg_wide<ROWS>(p, 0, b, r), w1 = p.n_in > 1 && seg_wide<ROWS>(p, 1, b, r);
+  const bool w2 = p.n_in > 2 && seg_wide<ROWS>(p, 2, b, r), w3 = FULL && p.n_in > 3 && seg_wide<ROWS>(p, 3, b, r);
   i.x0 = i.x1 = i.x2 = i.x3 = (seg_t)(0u);
-  if (p.n_in > 0) i.x0 = seg_load(p.in[p.in_at[0]], p.wide[0], b, r, c0, n);
-  if (p.n_in > 1) i.x1 = seg_load(p.in[p.in_at[1]], p.wide[1], b, r, c0, n);
-  if (p.n_in > 2) i.x2 = seg_load(p.in[p.in_at[2]], p.wide[2], b, r, c0, n);
-  if (FULL && p.n_in > 3) i.x3 = seg_load(p.in[p.in_at[3]], p.wide[3], b, r, c0, n);
-  if (p.n_in > 0) i.x0 = seg_convert<DT>(i.x0, p.in[p.in_at[0]].dtype, p.wide[0]);
-  if (p.n_in > 1) i.x1 = seg_convert<DT>(i.x1, p.in[p.in_at[1]].dtype, p.wide[1]);
-  if (p.n_in > 2) i.x2 = seg_convert<DT>(i.x2, p.in[p.in_at[2]].dtype, p.wide[2]);
-  if (FULL && p.n_in > 3) i.x3 = seg_convert<DT>(i.x3, p.in[p.in_at[3]].dtype, p.wide[3]);
+  if (p.n_in > 0) i.x0 = seg_load(p.in[p.in_at[0]], w0, b, r, c0, n);
+  if (p.n_in > 1) i.x1 = seg_load(p.in[p.in_at[1]], w1, b, r, c0, n);
+  if (p.n_in > 2) i.x2 = seg_load(p.in[p.in_at[2]], w2, b, r, c0, n);
+  if (FULL && p.n_in > 3) i.x3 = seg_load(p.in[p.in_at[3]], w3, b, r, c0, n);
+  if (p.n_in > 0) i.x0 = seg_convert<DT>(i.x0, p.in[p.in_at[0]].dtype, w0);
+  if (p.n_in > 1) i.x1 = seg_convert<DT>(i.x1, p.in[p.in_at[1]].dtype, w1);
+  if (p.n_in > 2) i.x2 = seg_convert<DT>(i.x2, p.in[p.in_at[2]].dtype, w2);
+  if (FULL && p.n_in > 3) i.x3 = seg_convert<DT>(i.x3, p.in[p.in_at[3]].dtype, w3);
 }
 
 // Runs the instructions that vary along the row: the result's bits.

@@ -654,25 +654,26 @@ def test_reductions(rt):
 
 # ---- attention --------------------------------------------------------------------------------------------------
 
-def random_program(rt, rng, dtype, shape, where):
+def random_program(rt, rng, dtype, shape, where, gap=0):
   """A program of random instructions over inputs of random forms (whole, one row or one value a row for all, every
-  second column, each dtype), and a function that gives it for batch entry b alone."""
+  second column, each dtype; rows `gap` values apart), and a function that gives it from row `first` of batch entry b on."""
   b, r, c = shape
+  s = c + gap
   inputs = []
   for _ in range(int(rng.integers(1, 7))):
     kind = rng.choice(["bf16", "fp32", "int32"]) if dtype != "int32" else "int32"
-    sb, sr, sc = [(r * c, c, 1), (0, 0, 1), (r, 1, 0), (0, 0, 0), (2 * r * c, 2 * c, 2)][int(rng.choice(5, p=[.4, .2, .2, .1, .1]))]
-    values = rng.normal(0, 2, 2 * b * r * c) if kind != "int32" else rng.integers(-9, 10, 2 * b * r * c)
+    sb, sr, sc = [(r * s, s, 1), (0, 0, 1), (r, 1, 0), (0, 0, 0), (2 * r * s, 2 * s, 2)][int(rng.choice(5, p=[.4, .2, .2, .1, .1]))]
+    values = rng.normal(0, 2, 2 * b * r * s) if kind != "int32" else rng.integers(-9, 10, 2 * b * r * s)
     dev = up(rt, B.bf16_bits(values) if kind == "bf16" else values.astype(np.float32 if kind == "fp32" else np.int32))
     inputs.append((dev, kind, sb, sr, sc))
   names = (["add", "sub", "mul", "max", "min", "cmplt", "cmpeq", "neg", "relu"] +
            (["div", "exp", "sqrt", "recip", "sigmoid", "silu", "tanh", "gelu", "sin", "ftob", "log2"] if dtype != "int32" else []) +
            (["where"] if where else []))
   picks = [(rng.choice(names), rng.random(3)) for _ in range(int(rng.integers(1, 16)))]
-  def build(entry):
+  def build(entry, first=0):
     p = Program(dtype)
     size = lambda kind: 2 if kind == "bf16" else 4
-    regs = [p.load(p.input(_lib.operand(dev + entry * sb * size(kind), kind, sb, sr, sc))) for dev, kind, sb, sr, sc in inputs]
+    regs = [p.load(p.input(_lib.operand(dev + (entry * sb + first * sr) * size(kind), kind, sb, sr, sc))) for dev, kind, sb, sr, sc in inputs]
     regs.append(p.const(3 if dtype == "int32" else 0.7))
     for name, at in picks:  # mostly the newest values, so that chains and values kept for later both come up
       src = [regs[-1 - int(u * u * len(regs))] for u in at]
@@ -716,6 +717,45 @@ def test_large_programs_equal_small_ones(rt, dtype, shape):
       sums = down(rt, some, (b, r), np.float32)
       ok = np.abs(total).sum(2) < 3e38  # past that fp32 partial sums may overflow
       assert np.all((np.abs(sums - total.sum(2)) <= bound)[ok]), trial
+
+
+# the segment kernels in every form, each program against the same one on rows few enough for the small kernel (bit for
+# bit), and reductions of its values: rows that start on 16 bytes and end in part of a segment, rows of which some start
+# there, more than one turn a wave, one and four waves a row; programs of few and of many inputs come up by chance
+@pytest.mark.parametrize("dtype", ["bf16", "fp32", "int32"])
+@pytest.mark.parametrize("shape,gap", [((2, 33, 1004), 0), ((1, 66, 1001), 7), ((3, 40, 1643), 1), ((5, 2000, 12), 4), ((3, 2800, 520), 0),
+                                       ((2, 300, 200), 0), ((1, 17000, 67), 5), ((1, 2100, 4100), 4)])
+def test_large_programs_in_every_form(rt, dtype, shape, gap):
+  b, r, c = shape
+  rng = np.random.default_rng(r + c)
+  kind = np.uint16 if dtype == "bf16" else np.uint32
+  whole, part = rt.dram_alloc(b * r * c * kind().itemsize), rt.dram_alloc((1 << 16) * kind().itemsize)
+  rows, red = ((1 << 16) - 1) // c, rt.dram_alloc(b * r * 4)
+  step = max(1, r // 3 - rows)  # three stretches of rows: the first, one inside, the last
+  for trial in range(8):
+    build = random_program(rt, rng, dtype, shape, where=trial % 2, gap=gap)
+    prog = build(0)
+    rt.run("elementwise", "elementwise", ctypes.byref(prog), b, r, c, ctypes.byref(_lib.operand(whole, dtype, r * c, c, 1)))
+    got = down(rt, whole, shape, kind)
+    vals = bits_to_float(got) if dtype == "bf16" else got.view(np.float32 if dtype == "fp32" else np.int32)
+    for e in range(b):
+      for first in sorted({0, min(step, max(0, r - rows)), max(0, r - rows)}):
+        n = min(rows, r - first)
+        rt.run("elementwise", "elementwise", ctypes.byref(build(e, first)), 1, n, c, ctypes.byref(_lib.operand(part, dtype, n * c, c, 1)))
+        want = down(rt, part, (n, c), kind)
+        wv = bits_to_float(want) if dtype == "bf16" else want.view(vals.dtype)
+        mine = got[e, first:first + n]
+        assert np.all((mine == want) | (np.isnan(vals[e, first:first + n]) & np.isnan(wv) if dtype != "int32" else False)), (trial, e, first)
+    if c < 64: continue
+    out = ctypes.byref(_lib.operand(red, dtype if dtype == "int32" else "fp32", r, 1, 1))
+    rt.run("reduce", "reduce", ctypes.byref(prog), _lib.REDUCE_MAX, 2, b, r, c, 0, 0, out)
+    assert np.array_equal(down(rt, red, (b, r), vals.dtype), vals.max(2), equal_nan=dtype != "int32"), trial
+    if dtype == "int32" or not np.isfinite(vals).all(): continue
+    rt.run("reduce", "reduce", ctypes.byref(prog), _lib.REDUCE_SUM, 2, b, r, c, 0, 0, out)
+    total, size = vals.astype(np.float64).sum(2), np.abs(vals.astype(np.float64)).sum(2)
+    # c fp32 additions, and bf16's rounding of the sum; past fp32's range partial sums may overflow
+    bound = c * 2.0 ** -24 * size + (2.0 ** -8 * np.abs(total) if dtype == "bf16" else 0)
+    assert np.all((np.abs(down(rt, red, (b, r), np.float32) - total) <= bound)[size < 3e38]), trial
 
 
 def attend(rt, q, k, v, places, window=0, parts=0):
