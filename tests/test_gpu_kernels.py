@@ -380,17 +380,13 @@ def test_split_k_rows(rt, fmt, m, k, n, out):
     assert np.array_equal(matmul(rt, x, cols, fmt, 1, n, out=out, prog=prog)[0], (plain + res).astype(np.float32))
 
 
-# (rows, K, N, output): rows > 64 run the tiled GEMM, except up to 256 rows when its 128 x 128 blocks would be fewer
-# than 128 (then the skinny kernel: 96 x 1536 here). With bf16 B (block floats unpacked to it from 512 rows up) and
-# K in 32s, 2048 x 8192 takes 256 x 256 blocks, 2048 x 4096 (fp32 with the residual) and 1000 x 4096 blocks of 128
-# rows; 1000 and 520 leave partial blocks, chunks of K and runs of N. bfp4 B with K in whole chunks (256, 192, 640)
-# is read by the GEMM as it is stored from 512 rows up. 2048 x 6144 takes blocks of 256 x 192 (256 of them, one round
-# of the CUs, where 256 x 256 would leave a quarter idle).
-# a prompt's chunk against a long K: the tiled GEMM's blocks split K between them. Rows either side of the plan's limits
-# and of a block's 128, columns off its 256, K of as few chunks a split as it takes; the formats still sum K alike, so a
-# block float is bit for bit the bf16 product of its values
+# a prompt's chunk against a long K: the tiled GEMM's blocks split K between them. Rows just over the plan's limits and
+# either side of a block's 128, columns off its 256, K of as few chunks a split as it takes; then rows, K and sizes just
+# below the limits, which don't split. The formats sum K alike, so a block float is bit for bit the bf16 product of its
+# values, and bf16 out is the fp32 sum rounded half up
 @pytest.mark.parametrize("m,k,n", [(33, 4096, 4096), (65, 4096, 1536), (127, 2048, 3000), (129, 1280, 576), (257, 1024, 1001),
-                                   (300, 1088, 500), (520, 4160, 260), (1000, 1024, 130)])
+                                   (300, 1088, 500), (520, 4160, 260), (1000, 1024, 130),
+                                   (32, 4096, 4096), (33, 4096, 4080), (64, 4032, 4208), (128, 1216, 5008), (256, 1216, 640), (257, 960, 1001)])
 def test_split_gemm_rows(rt, m, k, n):
   rng = np.random.default_rng(m)
   x, w = B.bf16(rng.normal(0, 1, (m, k))), rng.normal(0, 0.05, (k, n)).astype(np.float32)
@@ -404,8 +400,7 @@ def test_split_gemm_rows(rt, m, k, n):
     want, size = ops.matmul(x, wq), np.abs(x.astype(np.float64)) @ np.abs(wq.astype(np.float64))
     plain = matmul(rt, x, cols, fmt, 1, n)[0]
     assert np.all(np.abs(plain - want) <= 2.0 ** -8 * size)
-    same = bf16_columns(rt, wq)
-    assert np.array_equal(plain, matmul(rt, x, same, "bf16", 1, n)[0]), fmt
+    if fmt != "bf16": assert np.array_equal(plain, matmul(rt, x, bf16_columns(rt, wq), "bf16", 1, n)[0]), fmt
     p = Program("bf16", epilogue=True)
     relu2 = matmul(rt, x, cols, fmt, 1, n, prog=p.build(p.op("mul", p.op("relu", p.value()), p.const(2.0))))[0]
     assert np.array_equal(relu2, 2 * np.maximum(plain, 0)), fmt
@@ -413,6 +408,7 @@ def test_split_gemm_rows(rt, m, k, n):
     prog = p.build(p.op("add", p.value(), p.load(p.input(_lib.operand(dres, "fp32", m * n, n, 1)))))
     full = matmul(rt, x, cols, fmt, 1, n, out="fp32")[0]
     assert np.all(np.abs(full - want) <= k * 2.0 ** -24 * size)  # k fp32 additions at most
+    assert np.array_equal(plain, packed(full)), fmt
     assert np.array_equal(matmul(rt, x, cols, fmt, 1, n, out="fp32", prog=prog)[0], full + res), fmt
     if n % 32: continue
     got = rt.dram_alloc(m * n)
@@ -422,6 +418,39 @@ def test_split_gemm_rows(rt, m, k, n):
     silu = g / (1 + np.exp(-g)) * u
     out = bits_to_float(down(rt, got, (m, n // 2), np.uint16))
     assert np.all(np.abs(out - silu) <= 2.0 ** -7 * np.abs(silu) + 1e-30), fmt  # one bf16 rounding, and fp32's in silu
+
+
+def test_split_gemm_recorded_first(chip):
+  # recorded on a fresh runtime, whose scratch has no room for the partial sums and can't grow: the kernels that don't
+  # split K, summing in another order; replayed with eager work (which then does split) between
+  from baretile_amd.runtime import Runtime
+  rt = Runtime(chip)
+  try:
+    m, k, n = 300, 2048, 576
+    rng = np.random.default_rng(7)
+    x, w = B.bf16(rng.normal(0, 1, (m, k))), rng.normal(0, 0.05, (k, n)).astype(np.float32)
+    wq = bfp_values(w, "bfp8")
+    cols = columns(rt, *pack(rt, w, "bfp8"), "bfp8", 1, k, n)
+    a = ctypes.byref(_lib.operand(up(rt, B.bf16_bits(x)), "bf16", m * k, k, 1))
+    full, half = rt.dram_alloc(m * n * 4), rt.dram_alloc(m * n)
+    g = ctypes.c_void_p()
+    _lib.call("graph_begin", rt.handle)
+    rt.run("matmul", "matmul", a, _lib.BFP8, cols, 1, 1, m, k, n, None, ctypes.byref(_lib.operand(full, "fp32", m * n, n, 1)))
+    rt.run("swiglu", "matmul_swiglu", a, _lib.BFP8, cols, m, k, n, ctypes.byref(_lib.operand(half, "bf16", m * n // 2, n // 2, 1)))
+    _lib.call("graph_end", rt.handle, ctypes.byref(g))
+    want, size = ops.matmul(x, wq), np.abs(x.astype(np.float64)) @ np.abs(wq.astype(np.float64))
+    gate, other = want[:, :n // 2], want[:, n // 2:]
+    silu = gate / (1 + np.exp(-gate)) * other
+    # gate and up within 2^-8 of the sums of magnitudes (as bt_matmul's bf16), silu's slope below 1.1, one rounding
+    bound = 2.0 ** -8 * (1.1 * size[:, :n // 2] * (np.abs(other) + 2.0 ** -8 * size[:, n // 2:]) + np.abs(gate) * size[:, n // 2:] + np.abs(silu))
+    for _ in range(3):
+      rt.fill32(full, 0, m * n)
+      _lib.call("graph_launch", rt.handle, g)
+      assert np.all(np.abs(down(rt, full, (m, n), np.float32) - want) <= k * 2.0 ** -24 * size)
+      assert np.all(np.abs(bits_to_float(down(rt, half, (m, n // 2), np.uint16)) - silu) <= bound)
+      assert np.all(np.abs(matmul(rt, x, cols, "bfp8", 1, n, out="fp32")[0] - want) <= k * 2.0 ** -24 * size)
+    _lib.call("graph_destroy", g)
+  finally: rt.close()
 
 
 # either side of the lines between the GEMMs: block floats of fewer than 512 rows at one round of 128 x 128 blocks and over
@@ -493,6 +522,12 @@ def test_scratch_of_rising_prompts(chip):
   finally: rt.close()
 
 
+# (rows, K, N, output): rows > 64 run the tiled GEMM, except up to 256 rows when its 128 x 128 blocks would be fewer
+# than 128 (then the skinny kernel: 96 x 1536 here). K stays below 1024, where it is not split. With bf16 B and K in 32s,
+# 2048 x 8192 takes 256 x 256 blocks, 2048 x 4096 (fp32 with the residual) and 1000 x 4096 blocks of 128 rows; 1000 and
+# 520 leave partial blocks, chunks of K and runs of N. Block floats with K in whole chunks (256, 192, 640) are read as
+# they are stored, bfp8 on many 128-row blocks and any with K in part of a chunk unpacked first from 512 rows up. 2048 x
+# 6144 takes blocks of 256 x 192 (256 of them, one round of the CUs, where 256 x 256 would leave a quarter idle).
 GEMM_CASES = [(300, 1000, 520, "bf16"), (96, 576, 1536, "fp32"), (2048, 256, 8192, "bf16"), (2048, 192, 4096, "fp32"),
               (160, 320, 8192, "bf16"), (1000, 224, 4096, "bf16"), (520, 640, 1296, "fp32"), (2048, 320, 6144, "bf16"),
               (2048, 192, 6144, "fp32"), (2048, 128, 8192, "fp32")]
@@ -501,8 +536,8 @@ GEMM_CASES = [(300, 1000, 520, "bf16"), (96, 576, 1536, "fp32"), (2048, 256, 819
 @pytest.mark.parametrize("fmt", ["bf16", "bfp8", "bfp4"])
 @pytest.mark.parametrize("case", GEMM_CASES, ids=lambda c: "m{}k{}n{}{}".format(*c))
 def test_gemm_equals_row_slices(rt, fmt, case):
-  # The GEMM sums each output in the same order as the decode kernels (64-row chunks of K, lower half then upper), so
-  # it equals, bit for bit, the same product computed 64 rows at a time; with a fused epilogue (relu for bf16, a
+  # Where it doesn't split K the GEMM sums each output in the same order as the decode kernels (64-row chunks of K, lower
+  # half then upper), so it equals, bit for bit, the same product computed 64 rows at a time; with a fused epilogue (relu for bf16, a
   # residual add for fp32) as well. And it is within the reference's bound of the oracle.
   m, k, n, out = case
   rng = np.random.default_rng(m + k + n)

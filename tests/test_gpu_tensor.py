@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from baretile_amd.tensor import Recording, Tensor, jit
+from helpers import bits_to_float
 from oracle import bfp as B, ops
 
 pytestmark = pytest.mark.gpu
@@ -19,6 +20,33 @@ def packed(v):  # half-up bf16 rounding of a computed result (test/conftest.py:1
 
 
 def value(t): return np.array(t.tolist()).reshape(t.shape)
+
+
+# Large normalizations through the lazy graph, whole rows and odd ones, against float64. bf16 rounds every step to 8 bits,
+# at most 2^-8 of it. The mean: its sum, 1 / c and their product, three roundings. The value: the difference (1); the root
+# of the variance, half of two for the difference squared, one each for the square, the sum, 1 / c, their product and the
+# eps (3.5), then the root, the reciprocal and the product (3): 7.5, and their squares. fp32's unit is that of adding c
+# values in a row
+@pytest.mark.parametrize("dtype", ["bf16", "fp32"])
+@pytest.mark.parametrize("rows,cols", [(2048, 4096), (600, 1001), (17000, 72)])
+def test_large_normalizations(rt, dtype, rows, cols):
+  rng = np.random.default_rng(cols)
+  a = rng.normal(0.5, 1.5, (rows, cols)).astype(np.float32)
+  if dtype == "bf16": a = B.bf16(a)
+  x = Tensor.frombytes(rt, rows, cols, (B.bf16_bits(a) if dtype == "bf16" else a).tobytes(), dtype=dtype)
+  read = lambda t: (bits_to_float(np.frombuffer(t.realize().tobytes(), np.uint16)) if dtype == "bf16" else
+                    np.frombuffer(t.realize().tobytes(), np.float32)).reshape(rows, cols).astype(np.float64)
+  d = a.astype(np.float64)
+  mean = d.mean(1, keepdims=True)
+  scale = 1 / np.sqrt(((d - mean) ** 2).mean(1, keepdims=True) + 1e-5)
+  want, unit = (d - mean) * scale, 2.0 ** -8 if dtype == "bf16" else cols * 2.0 ** -24
+  assert np.all(np.abs(read(x.layernorm()) - want) <= unit * (8 * np.abs(want) + 3.1 * np.abs(d).mean(1, keepdims=True) * scale))
+  low = d - d.max(1, keepdims=True)
+  want = np.exp(low) / np.exp(low).sum(1, keepdims=True)
+  # the argument's rounding is a relative error of exp as large as the argument, in the value and, weighted, in the sum;
+  # exp's own in both, the sum's, the reciprocal's and the product's: 5, and their squares
+  weighted = (want * np.abs(low)).sum(1, keepdims=True)
+  assert np.all(np.abs(read(x.softmax()) - want) <= want * unit * (1.05 * (np.abs(low) + weighted) + 5.1))
 
 
 def test_readme_and_ramp_known_answers(rt):
