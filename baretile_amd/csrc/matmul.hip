@@ -395,10 +395,12 @@ __device__ __forceinline__ void sum_slices(f32x4 (&acc)[MT], const SlicePos &p, 
 // tile buffer and reads zeros without touching memory, so the compiler can count the loads and let each chunk start
 // as soon as its own have landed. Weight bytes are read once, so they are loaded non-temporal (sc1 nt), which keeps
 // them from displacing cached lines on their way. ONE: a single matrix (batch of one), without broadcast arithmetic.
-// PROG: whether the epilogue runs a program; the plain kernels carry no interpreter, so their code stays small.
+// PROG: 1 where the epilogue runs a program, 2 where that is one operation on the product and an input; the plain kernels
+// carry no interpreter and the interpreter's not that operation, so their code stays small (with both in one kernel, products
+// with ReLU or SiLU took 2-4% longer: 17 x 2528 x 1888 bfp8 25.2 us, 24.3 so, 103 x 5248 x 768 16.7 and 16.2).
 constexpr int STREAM = 18;  // cache-policy bits of a buffer load: sc1 | nt
 
-template <int FMT, int DT, int ROWS, int G, bool ONE, bool PROG, bool SL>
+template <int FMT, int DT, int ROWS, int G, bool ONE, int PROG, bool SL>
 __global__ void __launch_bounds__(SL ? 512 : 256) gemv_kernel(const MatmulArgs args, int slices_arg) {
   constexpr int SLOT = ROWS * 64, TB = Tile<FMT>::bytes;  // SLOT: halfwords of one chunk's scaled x
   // LDS, sized at launch: each wave's slots, then (with slices) each wave's partial tile
@@ -500,7 +502,7 @@ __global__ void __launch_bounds__(SL ? 512 : 256) gemv_kernel(const MatmulArgs a
                                                  orr, at * 4, 0, 0);
     }
   } else {
-    store_tile<DT, false, ONE, PROG ? 1 : 0>(args, h, acc[0], b, 0, run, g, col);
+    store_tile<DT, false, ONE, PROG ? 1 : 0, PROG == 2 ? 2 : 0>(args, h, acc[0], b, 0, run, g, col);
   }
 }
 
@@ -825,7 +827,7 @@ __global__ void __launch_bounds__(256) skinny_lds_kernel(const MatmulArgs args, 
 // SWI: B holds gate columns then up columns (n = 2f); a wave's two runs are gate run u and up run u + n / 32, and it
 // writes silu(g) * u for its 16 columns of the bf16 out (f wide), g and u rounded to bf16 first, as the tiled GEMM's
 // SiLU-mul epilogue does.
-template <int FMT, int DT, int G, bool PROG, bool SL, bool RES = false, bool SWI = false>
+template <int FMT, int DT, int G, int PROG, bool SL, bool RES = false, bool SWI = false>
 __global__ void __launch_bounds__(SL ? 512 : 256) skinny2_kernel(const MatmulArgs args, int slices_arg,
                                                                  const bt_operand res) {
   constexpr int TB = Tile<FMT>::bytes, MT = 2, NR = 2;
@@ -964,11 +966,11 @@ __global__ void __launch_bounds__(SL ? 512 : 256) skinny2_kernel(const MatmulArg
     if (run0 + r >= h.nruns) continue;
 #pragma unroll
     for (int t = 0; t < MT; t++)
-      store_tile<DT, false, false, PROG ? 1 : 0>(args, h, acc[r * MT + t], b, mg * MT + t, run0 + r, g, col);
+      store_tile<DT, false, false, PROG ? 1 : 0, PROG == 2 ? 2 : 0>(args, h, acc[r * MT + t], b, mg * MT + t, run0 + r, g, col);
   }
 }
 
-template <int FMT, int DT, int G, bool ONE, bool PROG, int MT, bool SL>
+template <int FMT, int DT, int G, bool ONE, int PROG, int MT, bool SL>
 __global__ void __launch_bounds__(SL ? 512 : 256) skinny_vec_kernel(const MatmulArgs args, int slices_arg) {
   constexpr int TB = Tile<FMT>::bytes;
   extern __shared__ __attribute__((aligned(16))) uint8_t dyn[];  // with slices: each wave's partial tiles
@@ -1074,7 +1076,7 @@ __global__ void __launch_bounds__(SL ? 512 : 256) skinny_vec_kernel(const Matmul
   if (p.s == 0 && p.valid)
 #pragma unroll
     for (int t = 0; t < MT; t++)
-      store_tile<DT, false, ONE, PROG ? 1 : 0>(args, h, acc[t], b, mg * MT + t, run, g, col);
+      store_tile<DT, false, ONE, PROG ? 1 : 0, PROG == 2 ? 2 : 0>(args, h, acc[t], b, mg * MT + t, run, g, col);
 }
 
 // B-side scaling, for A of any strides: each lane turns its 16 B values into bf16 q * 2^d with v_ldexp_f32 and
@@ -2575,6 +2577,20 @@ static void launch_x(const MatmulArgs &args, hipStream_t s) {
   }
 }
 
+// A launch with P as the kernels' PROG.
+#define BT_BY_PROG(...)                                                      \
+  do {                                                                       \
+    if (!args.n_inst) {                                                      \
+      constexpr int P = 0;                                                   \
+      __VA_ARGS__;                                                           \
+    } else if (one_input(args.prog, args.n_inst).op >= 0) {                  \
+      constexpr int P = 2;                                                   \
+      __VA_ARGS__;                                                           \
+    } else {                                                                 \
+      constexpr int P = 1;                                                   \
+      __VA_ARGS__;                                                           \
+    }                                                                        \
+  } while (0)
 template <int FMT, int DT>
 static void launch_dt(const MatmulArgs &args, unsigned blocks, hipStream_t s, bool vec) {
   const bool rows_contiguous = args.a.sc == 1 && (int64_t)args.k * 2 < (1ll << 31);
@@ -2595,22 +2611,18 @@ static void launch_dt(const MatmulArgs &args, unsigned blocks, hipStream_t s, bo
     if (args.m == 1) {
       constexpr int SB = 64 * 2;  // slot bytes a chunk
       if (!lean && sl > 1) {
-        if (args.n_inst) launch_sliced(gemv_kernel<FMT, DT, 1, 8, false, true, true>, args, units, sl, 8 * SB, 1024, s);
-        else launch_sliced(gemv_kernel<FMT, DT, 1, 8, false, false, true>, args, units, sl, 8 * SB, 1024, s);
+        BT_BY_PROG(launch_sliced(gemv_kernel<FMT, DT, 1, 8, false, P, true>, args, units, sl, 8 * SB, 1024, s));
       } else if (!lean) {
-        if (args.n_inst) launch_sliced(gemv_kernel<FMT, DT, 1, 12, false, true, false>, args, units, 1, 12 * SB, 0, s);
-        else launch_sliced(gemv_kernel<FMT, DT, 1, 12, false, false, false>, args, units, 1, 12 * SB, 0, s);
+        BT_BY_PROG(launch_sliced(gemv_kernel<FMT, DT, 1, 12, false, P, false>, args, units, 1, 12 * SB, 0, s));
       } else if (group == 9) launch_sliced(gemv_kernel<FMT, DT, 1, 9, true, false, false>, args, units, 1, 9 * SB, 0, s);
       else if (group == 8) launch_sliced(gemv_kernel<FMT, DT, 1, 8, true, false, false>, args, units, 1, 8 * SB, 0, s);
       else launch_sliced(gemv_kernel<FMT, DT, 1, 12, true, false, false>, args, units, 1, 12 * SB, 0, s);
     } else {
       constexpr int SB = 4 * 64 * 2;
       if (!lean && sl > 1) {
-        if (args.n_inst) launch_sliced(gemv_kernel<FMT, DT, 4, 8, false, true, true>, args, units, sl, 8 * SB, 1024, s);
-        else launch_sliced(gemv_kernel<FMT, DT, 4, 8, false, false, true>, args, units, sl, 8 * SB, 1024, s);
+        BT_BY_PROG(launch_sliced(gemv_kernel<FMT, DT, 4, 8, false, P, true>, args, units, sl, 8 * SB, 1024, s));
       } else if (!lean) {
-        if (args.n_inst) launch_sliced(gemv_kernel<FMT, DT, 4, 12, false, true, false>, args, units, 1, 12 * SB, 0, s);
-        else launch_sliced(gemv_kernel<FMT, DT, 4, 12, false, false, false>, args, units, 1, 12 * SB, 0, s);
+        BT_BY_PROG(launch_sliced(gemv_kernel<FMT, DT, 4, 12, false, P, false>, args, units, 1, 12 * SB, 0, s));
       } else if (group == 9) launch_sliced(gemv_kernel<FMT, DT, 4, 9, true, false, false>, args, units, 1, 9 * SB, 0, s);
       else if (group == 8) launch_sliced(gemv_kernel<FMT, DT, 4, 8, true, false, false>, args, units, 1, 8 * SB, 0, s);
       else launch_sliced(gemv_kernel<FMT, DT, 4, 12, true, false, false>, args, units, 1, 12 * SB, 0, s);
@@ -2633,14 +2645,11 @@ static void launch_dt(const MatmulArgs &args, unsigned blocks, hipStream_t s, bo
     const int sl = one_trip ? 1 : choose_slices(units, args.chunks);
     const bool lean = args.batch == 1 && !args.n_inst && sl == 1 && !two && !one_trip;
     if (one_trip && args.chunks % 9 == 0) {
-      if (args.n_inst) launch_sliced(skinny_vec_kernel<FMT, DT, 9, false, true, 1, false>, args, units, 1, 0, 0, s);
-      else launch_sliced(skinny_vec_kernel<FMT, DT, 9, false, false, 1, false>, args, units, 1, 0, 0, s);
+      BT_BY_PROG(launch_sliced(skinny_vec_kernel<FMT, DT, 9, false, P, 1, false>, args, units, 1, 0, 0, s));
     } else if (one_trip) {
-      if (args.n_inst) launch_sliced(skinny_vec_kernel<FMT, DT, 12, false, true, 1, false>, args, units, 1, 0, 0, s);
-      else launch_sliced(skinny_vec_kernel<FMT, DT, 12, false, false, 1, false>, args, units, 1, 0, 0, s);
+      BT_BY_PROG(launch_sliced(skinny_vec_kernel<FMT, DT, 12, false, P, 1, false>, args, units, 1, 0, 0, s));
     } else if (two && args.chunks <= 2) {  // short K (a head's width): groups of 2
-      if (args.n_inst) launch_sliced(skinny_vec_kernel<FMT, DT, 2, false, true, 2, true>, args, units, sl, 0, 2048, s);
-      else launch_sliced(skinny_vec_kernel<FMT, DT, 2, false, false, 2, true>, args, units, sl, 0, 2048, s);
+      BT_BY_PROG(launch_sliced(skinny_vec_kernel<FMT, DT, 2, false, P, 2, true>, args, units, sl, 0, 2048, s));
     } else if (two && pairs_fill(args)) {  // two runs a wave: half the units, each slice's partial 4 tiles
       const int64_t units2 = (int64_t)args.batch * ((args.nruns + 1) / 2) * ((args.mtiles + 1) / 2);
       const int sl2 = pair_slices(args);
@@ -2650,14 +2659,11 @@ static void launch_dt(const MatmulArgs &args, unsigned blocks, hipStream_t s, bo
       bt_operand res{};
       if (DT == BT_FP32 && residual_program(args, &res))
         skinny2_kernel<FMT, DT, 4, false, true, true><<<blocks, wpb * 64, lds, s>>>(args, sl2, res);
-      else if (args.n_inst) skinny2_kernel<FMT, DT, 4, true, true><<<blocks, wpb * 64, lds, s>>>(args, sl2, res);
-      else skinny2_kernel<FMT, DT, 4, false, true><<<blocks, wpb * 64, lds, s>>>(args, sl2, res);
+      else BT_BY_PROG(skinny2_kernel<FMT, DT, 4, P, true><<<blocks, wpb * 64, lds, s>>>(args, sl2, res));
     } else if (two) {
-      if (args.n_inst) launch_sliced(skinny_vec_kernel<FMT, DT, 8, false, true, 2, true>, args, units, sl, 0, 2048, s);
-      else launch_sliced(skinny_vec_kernel<FMT, DT, 8, false, false, 2, true>, args, units, sl, 0, 2048, s);
+      BT_BY_PROG(launch_sliced(skinny_vec_kernel<FMT, DT, 8, false, P, 2, true>, args, units, sl, 0, 2048, s));
     } else if (!lean) {
-      if (args.n_inst) launch_sliced(skinny_vec_kernel<FMT, DT, 8, false, true, 1, true>, args, units, sl, 0, 1024, s);
-      else launch_sliced(skinny_vec_kernel<FMT, DT, 8, false, false, 1, true>, args, units, sl, 0, 1024, s);
+      BT_BY_PROG(launch_sliced(skinny_vec_kernel<FMT, DT, 8, false, P, 1, true>, args, units, sl, 0, 1024, s));
     } else if (group == 9) {
       launch_sliced(skinny_vec_kernel<FMT, DT, 9, true, false, 1, false>, args, units, 1, 0, 0, s);
     } else {
@@ -2666,6 +2672,7 @@ static void launch_dt(const MatmulArgs &args, unsigned blocks, hipStream_t s, bo
   } else if (vec) skinny_kernel<FMT, DT, true><<<blocks, 256, 0, s>>>(args);
   else skinny_kernel<FMT, DT, false><<<blocks, 256, 0, s>>>(args);
 }
+#undef BT_BY_PROG
 
 // The split-K kernels for 5 to 32 rows of one A against a long K (more than 12 chunks, a multiple of 64): false
 // when the product doesn't fit them or the runtime has no scratch for the partials (then the one-launch kernels run
