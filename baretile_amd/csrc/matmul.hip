@@ -2543,7 +2543,10 @@ static void launch_lds(const MatmulArgs &args, unsigned blocks, hipStream_t s) {
   launch_lds_n<FMT, DT, 1, 1>(args, blocks, s);
 }
 
-// SiLU x up on skinny_lds_kernel: up to 256 rows of block-float B with a short K; false when the product doesn't fit.
+// SiLU x up on skinny_lds_kernel, for up to 256 rows of block-float B with a short K. Each block of 16 rows reads B again
+// (from L2, past the first), where skinny2_kernel reads it once for 32, and is the faster at every row count: bfp8, us there
+// and here, K 576 and 3072 columns at 8 rows 6.9 and 4.6, at 64 9.1 and 4.7, at 256 9.5 and 7.3; K 768 and 8192 columns at 8
+// 8.2 and 5.5, at 128 11.0 and 10.3.
 template <int FMT, int G>
 static void launch_lds_swiglu_g(const MatmulArgs &args, hipStream_t s) {
   const dim3 grid((unsigned)((args.nruns / 2 + 1) / 2), (unsigned)((args.m + 15) / 16));

@@ -89,12 +89,12 @@ def test_a_program_built_again_keeps_its_own_inputs_and_limits():
 
 @pytest.mark.parametrize("hd", [64, 128])
 def test_attention_scratch_of_rows_with_regions(hd):
-  # rows with first keys of their own: parts chosen by the caller keep the packed tiles' partial sums (a tile 16 pairs,
+  # rows with regions of their own, said to be apart: parts chosen by the caller keep the packed tiles' partial sums (a tile 16 pairs,
   # 32 + 16 hd floats a part), the library's own plan fits the 8 MiB of bt_attention_noalloc at every size
   from baretile_amd import _lib
   def scratch(kvh, rep, rows, keys, parts, fmt):
     args = _lib.AttentionArgs(4096, 4096, 4096, 4096, 4096, rows * hd, hd, keys * hd, hd, keys * hd, hd, rows * hd, hd, rows,
-                              kvh * rep, rep, rows, keys, hd, 0, parts, 0, 0, 0, 4096, rows, fmt, 0, 4096, 4096)
+                              kvh * rep, rep, rows, keys, hd, 0, parts, 1, 0, 0, 4096, rows, fmt, 0, 4096, 4096)
     need = ctypes.c_uint64()
     _lib.call("attention_scratch", ctypes.byref(args), ctypes.byref(need))
     return need.value

@@ -990,7 +990,7 @@ def test_attention_rows_in_tiles_of_their_own(rt, slots, rep, part, hd):
   places = firsts + rng.integers(0, part, slots, dtype=np.int32)
   o = rt.dram_alloc(E * slots * hd * 2)
   args = _lib.AttentionArgs(*(up(rt, B.bf16_bits(t)) for t in (q, k, v)), o, up(rt, places), slots * hd, hd, keys * hd, hd, keys * hd,
-                            hd, slots * hd, hd, slots, E, rep, slots, keys, hd, 0, 0, 0, 0, 0, up(rt, firsts.copy()), slots)
+                            hd, slots * hd, hd, slots, E, rep, slots, keys, hd, 0, 0, 1, 0, 0, up(rt, firsts.copy()), slots)
   need = ctypes.c_uint64()
   _lib.call("attention_scratch", ctypes.byref(args), ctypes.byref(need))
   if need.value: args.scratch, args.scratch_bytes = rt.dram_alloc(need.value), need.value
