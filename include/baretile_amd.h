@@ -221,7 +221,8 @@ int bt_matmul_row(bt_runtime *rt, const bt_row_args *args);
  * rounded to bf16 as stored, silu(g) = g / (1 + exp(-g)), in fp32. A is bf16 with contiguous rows, k a multiple of
  * 32; out is bf16 with contiguous, 16-byte aligned rows. Where the tiled GEMM runs it (more than 64 rows, unless its
  * grid would be small), a block-float B whose k is no multiple of 64 is unpacked to bf16 in the runtime's scratch first
- * (BT_ESTATE inside a capture when that scratch would have to grow); otherwise B is read as stored, through split-K
+ * (BT_ESTATE inside a capture when that scratch would have to grow), and so, where the scratch allows, is a bfp8 B with
+ * a long k and few columns, with the same results; otherwise B is read as stored, through split-K
  * partial sums in that scratch where bt_matmul would split K (inside a capture that would have to grow it, a one-launch
  * kernel instead). */
 int bt_matmul_swiglu(bt_runtime *rt, const bt_operand *a, int b_fmt, uint64_t b, int64_t m, int64_t k, int64_t n,
