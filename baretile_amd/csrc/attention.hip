@@ -1113,12 +1113,16 @@ static int plan_attention(const bt_attention_args *a, AttnPlan *p) {
   const int kvh = a->heads / a->rep, np = a->rep * a->rows;
   // rows with regions of their own: tiles by row while they are few (a decode step's slots, one token each), where the
   // parts are the library's to choose: its plans take 5.7 MB of scratch at most, while parts that a caller chose for
-  // packed tiles would outgrow bt_attention_noalloc's 8 MiB over 16 times the tiles. Only where the caller says that the
-  // regions are apart: rows that share one would each read it again, which packed tiles read once for 16 pairs, on parts
-  // planned for a region's share of the keys (24 rows of one head of 64 over 23136 shared keys 174.9 us by row, 18.5
-  // packed).
-  const bool by_row = a->apart && a->firsts && a->rows > 1 && a->rows <= 32 && a->parts == 0;
+  // packed tiles would outgrow bt_attention_noalloc's 8 MiB over 16 times the tiles. Where packed tiles would split the
+  // keys too (4 of them at most), only if the caller says that the regions are apart: rows that share one would each read it
+  // again, which packed tiles read once for 16 pairs, on parts planned for a region's share of the keys (24 rows of one head
+  // of 64 over 23136 shared keys 174.9 us by row, 18.5 packed). More packed tiles would take the prefill kernel, whose few
+  // blocks walk all the keys: up to 384 tiles by row are faster there whatever the regions (24 rows of 7 heads over 10992 keys
+  // in two regions 153 us there, 37 by row; 57 calls with shared regions 0.14 to 1.0 of the prefill's time, at 512 tiles 0.7
+  // and 1.3).
   const int per_row = (a->rep + 15) / 16;
+  const bool by_row = a->firsts && a->rows > 1 && a->rows <= 32 && a->parts == 0 &&
+                      (a->apart || (np > 64 && (int64_t)kvh * a->rows * per_row <= 384));
   p->tiles = Tiles{by_row ? a->rows * per_row : (np + 15) / 16, by_row ? per_row : 0, make_fastdiv((uint32_t)a->rep),
                    make_fastdiv((uint32_t)per_row)};
   p->decode = by_row || p->tiles.n <= 4;  // few query rows for each key head: split the keys instead

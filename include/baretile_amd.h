@@ -289,8 +289,9 @@ int bt_matmul_residual_rms(bt_runtime *rt, const bt_operand *a, int b_fmt, uint6
  *
  * firsts, when given, raises each row's first visible key (a batch of sequences with their own regions of one cache,
  * as the reference's slots use it, llama.py:293-318). The library can't see whether rows share a region: apart says that
- * none do, as where every sequence has one row, and lets a call of 2 to 32 rows plan by region. It changes the plan
- * and the order of sums, never which keys a row sees.
+ * none do, as where every sequence has one row, and lets any call of 2 to 32 rows plan by region (without it only calls
+ * of more than 64 query rows a key head do, where few key heads and rows make that the faster plan either way). It
+ * changes the plan and the order of sums, never which keys a row sees.
  *
  * parts splits a decode step's keys (at most 64 query rows per key head: rep * rows <= 64) between that many blocks,
  * as attention_kernel's parts does; 0 picks a count from the shape. With more than one part the blocks write fp32

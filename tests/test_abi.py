@@ -107,9 +107,10 @@ def test_attention_scratch_of_rows_with_regions(hd):
 
 
 @pytest.mark.parametrize("hd", [64, 128])
-def test_attention_plans_by_region_only_where_rows_are_apart(hd):
-  # rows whose regions may be shared take the plan of a call without regions; rows said to be apart the plan by row,
-  # within bt_attention_noalloc's 8 MiB at every size
+def test_attention_plans_by_region_where_rows_are_apart(hd):
+  # rows whose regions may be shared take the plan of a call without regions where that splits the keys (64 pairs a key
+  # head) or the tiles by row would be more than 384; the others, and rows said to be apart, the plan by row, within
+  # bt_attention_noalloc's 8 MiB at every size
   from baretile_amd import _lib
   def scratch(kvh, rep, rows, keys, fmt, firsts, apart):
     args = _lib.AttentionArgs(4096, 4096, 4096, 4096, 4096, rows * hd, hd, keys * hd, hd, keys * hd, hd, rows * hd, hd, rows,
@@ -122,8 +123,9 @@ def test_attention_plans_by_region_only_where_rows_are_apart(hd):
       for rows in (1, 2, 8, 31, 32, 33):
         for keys in (100, 512, 1000, 4096):
           for fmt in (_lib.BF16, _lib.BFP8):
-            plain = scratch(kvh, rep, rows, keys * rows, fmt, 0, 0)
-            assert scratch(kvh, rep, rows, keys * rows, fmt, 4096, 0) == plain == scratch(kvh, rep, rows, keys * rows, fmt, 0, 1)
-            assert scratch(kvh, rep, rows, keys * rows, fmt, 4096, 1) <= 8 << 20
+            plain, apart = scratch(kvh, rep, rows, keys * rows, fmt, 0, 0), scratch(kvh, rep, rows, keys * rows, fmt, 4096, 1)
+            by_row = rep * rows > 64 and rows <= 32 and kvh * rows * -(-rep // 16) <= 384
+            assert scratch(kvh, rep, rows, keys * rows, fmt, 4096, 0) == (apart if by_row else plain)
+            assert plain == scratch(kvh, rep, rows, keys * rows, fmt, 0, 1) and apart <= 8 << 20
   # 8 slots of 512 rows, 3 heads a key head: 9 parts of one block of keys for each of 24 tiles
   assert scratch(3, 3, 8, 8 * 512, _lib.BF16, 4096, 1) == 24 * 9 * (32 + 16 * hd) * 4
