@@ -3262,11 +3262,13 @@ extern "C" int bt_matmul_swiglu(bt_runtime *rt, const bt_operand *a, int b_fmt, 
       if ((mb * (nb - t)) % 256 == 0) { tail = t; break; }
   }
   // 128-row blocks throughout where their rounds take less than the 256-row ones'. A round of theirs takes, of half a
-  // 256-row round: bf16 1.08-1.15 up to K 1024, 1.19-1.22 at 1600 and 1.37 at 7936 (B is read twice as often; 2538 x 512 x
-  // 21152 in 7 rounds 93 us, in 4 of 256 rows 98; 3339 x 1728 x 15616 231 and 217), bfp4 1.18-1.23, bfp8 1.28-1.30
-  // (and decoded twice as often: 2911 x 6272 x 25280 in 9 rounds 1022 us, in 5 of 256 rows 885; 1432 x 1344 x 12896 in 3
-  // rounds 88, in 2 93)
-  const double round128 = b_fmt == BT_BFP8 ? 1.3 : b_fmt == BT_BFP4 ? 1.23 : k <= 1024 ? 1.12 : k <= 4096 ? 1.22 : 1.4;
+  // 256-row round: bf16 1.08-1.15 up to K 1024, 1.19-1.24 above (B is read twice as often; 2538 x 512 x 21152 in 7 rounds
+  // 93 us, in 4 of 256 rows 98; 3339 x 1728 x 15616 231 and 217; 2944 x 7296 x 7616 in 3 rounds 341, in 2 367) and 1.37 with
+  // few rows against a long K (793 x 7936 x 24672), bfp4 1.18-1.23, bfp8 1.18-1.20 up to K 512, 1.23-1.25 to 1024, then
+  // 1.25-1.30 (decoded twice as often: 2911 x 6272 x 25280 in 9 rounds 1022 us, in 5 of 256 rows 885; 2361 x 448 x 27168 in 8
+  // rounds 114, in 5 120)
+  const double round128 = b_fmt == BT_BFP8 ? (k <= 512 ? 1.19 : k <= 1024 ? 1.24 : 1.3) : b_fmt == BT_BFP4 ? 1.23 :
+                          k <= 1024 ? 1.12 : k <= 4096 || m > 1024 ? 1.24 : 1.4;
   if (!tail && (mb128 * nb + 255) / 256 * round128 < 2 * ((mb * nb + 255) / 256)) tail = nb;
   auto launch = [&](auto fmt) {
     constexpr int FMT = decltype(fmt)::value;
